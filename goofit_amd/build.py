@@ -28,7 +28,7 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("GOOFIT_AMD_ARCH", "gfx950")
 HIP_FLAGS = [f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-ffp-contract=off", "-fPIC",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wall", "-Wno-unused-parameter"]
-HIP_SOURCES = ["gf_kernels.hip", "gf_mlp.hip", "gf_capi.hip"]
+HIP_SOURCES = ["gf_coherent.hip", "gf_kernels.hip", "gf_lines.hip", "gf_mlp.hip", "gf_capi.hip"]
 
 CXX = os.environ.get("CXX", "g++")
 CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall", "-Wextra", "-Wno-unused-parameter"]

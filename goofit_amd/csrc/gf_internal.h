@@ -9,6 +9,7 @@
 // accumulators (acc[level]); a leaf leaves its value in T.
 #pragma once
 
+#include <hip/hip_runtime_api.h>
 #include <stdint.h>
 
 #define GF_MAX_OBS 8      // observable columns per event
@@ -173,11 +174,13 @@ struct GfNormOp {
     double c0, c1;
 };
 
-// Host-side launchers (gf_kernels.hip).
+// Host-side launchers (gf_kernels.hip, gf_coherent.hip, gf_lines.hip).
 namespace gfk {
 struct Partial {
     double s, c;
 };
+// k_finish for the sweep launched before it on stream s (gf_kernels.hip).
+int launch_finish(const GfProgArgs &a, Partial *partials, int nblocks, GfResult *result, hipStream_t s);
 // inl: parameter/normalisation values in the kernel arguments (null: device arrays).
 // Reductions: one partial per workgroup, then one workgroup adds them into *result.
 int launch_reduce_metric(const GfProgArgs &a, const GfInline *inl, int metric, Partial *partials, GfResult *result,
