@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -10,6 +11,7 @@
 #include <chrono>
 #include <complex>
 #include <map>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -113,7 +115,7 @@ struct gf_ctx {
     GfIns *d_ins = nullptr;
     size_t cap_params = 0, cap_consts = 0, cap_norms = 0, cap_obsid = 0, cap_ins = 0;
     GfDalitzSlot *d_dz = nullptr;
-    GfResDesc *d_res = nullptr;  // GF_MAX_DALITZ * GF_MAX_RES
+    GfLinePlan *d_plan = nullptr;  // one per Dalitz node, then one for a stack of lineshapes (gf_tddp_gram)
     GfDecay decay{};
 
     std::map<int, WaveCache> caches;
@@ -677,11 +679,62 @@ gf_status scan_dalitz(gf_ctx *ctx) {
     return GF_OK;
 }
 
+// The structure of a lineshape plan for the n resonances in res: their terms sorted into
+// classes (GfLinePlan; the numbers are filled in on the device).  both: every resonance
+// at (m12, m13) and again at (m13, m12), as the cache of a time-dependent node holds them.
+void line_plan(const gf_ctx *ctx, const GfResDesc *res, int n, bool both, GfLinePlan &plan) {
+    struct Entry {
+        std::array<int, 4> key;  // swap, pair, spin, norm
+        GfLineTerm term;
+    };
+    std::vector<Entry> all;
+    for(int sw = 0; sw < (both ? 2 : 1); sw++)
+        for(int i = 0; i < n; i++) {
+            const GfResDesc &r = res[i];
+            Entry e{};
+            e.key       = {both ? sw : (r.swap != 0), -1, 0, 1};
+            e.term.res  = i;
+            e.term.p    = r.p;
+            e.term.kind = r.kind == GR_RBW_SYM ? GR_RBW : r.kind;
+            if(r.kind != GR_NONRES) {
+                const unsigned spin = (unsigned)ctx->consts[r.c], cyc = (unsigned)ctx->consts[r.c + 1];
+                // without spin there are no barrier factors: the flag makes no difference
+                e.key = {e.key[0], (int)std::min(cyc, 3u), (int)spin, (spin == 0 || ctx->consts[r.c + 2] != 0.0) ? 1 : 0};
+                if(r.kind == GR_RBW_SYM) {  // the second half, one channel on (RBW.cu:80-81)
+                    Entry h  = e;
+                    h.key[1] = (int)((cyc + 1) % 3);
+                    all.push_back(h);
+                }
+            }
+            all.push_back(e);
+        }
+    std::stable_sort(all.begin(), all.end(), [](const Entry &a, const Entry &b) { return a.key < b.key; });
+    memset(&plan, 0, sizeof(plan));
+    std::set<std::pair<int, int>> seen;  // rows with a term already
+    for(size_t k = 0; k < all.size(); k++) {
+        const auto &key = all[k].key;
+        if(k == 0 || key != all[k - 1].key) {
+            GfLineClass &c = plan.cls[plan.nclass++];
+            c.first        = (int)k;
+            c.swap         = key[0];
+            c.pair         = key[1];
+            c.spin         = key[2];
+            c.norm         = key[3];
+        }
+        GfLineClass &c = plan.cls[plan.nclass - 1];
+        c.count++;
+        c.res |= 1u << all[k].term.res;
+        plan.term[k]     = all[k].term;
+        plan.term[k].cls = plan.nclass - 1;
+        plan.term[k].add = seen.insert({key[0], all[k].term.res}).second ? 0 : 1;
+    }
+    plan.nterm = (int)all.size();
+}
+
 gf_status upload_dalitz_table(gf_ctx *ctx) {
     GfDalitzSlot slots[GF_MAX_DALITZ];
-    GfResDesc res[GF_MAX_DALITZ * GF_MAX_RES];
+    std::vector<GfLinePlan> plans(GF_MAX_DALITZ);
     memset(slots, 0, sizeof(slots));
-    memset(res, 0, sizeof(res));
     for(size_t s = 0; s < ctx->dalitz.size(); s++) {
         const DalitzNode &d = ctx->dalitz[s];
         auto it             = ctx->caches.find(d.cache_key);
@@ -698,11 +751,11 @@ gf_status upload_dalitz_table(gf_ctx *ctx) {
         slots[s].col_tag    = d.col_tag;
         slots[s].res_kind   = d.res_kind;
         slots[s].res_p      = d.res_p;
-        for(int i = 0; i < d.nres; i++)
-            res[s * GF_MAX_RES + i] = d.res[i];
+        line_plan(ctx, d.res.data(), d.nres, d.td, plans[s]);
     }
     GF_HIP(hipMemcpyAsync(ctx->d_dz, slots, sizeof(slots), hipMemcpyHostToDevice, ctx->stream));
-    GF_HIP(hipMemcpyAsync(ctx->d_res, res, sizeof(res), hipMemcpyHostToDevice, ctx->stream));
+    GF_HIP(hipMemcpyAsync(ctx->d_plan, plans.data(), GF_MAX_DALITZ * sizeof(GfLinePlan), hipMemcpyHostToDevice,
+                          ctx->stream));
     GF_HIP(hipStreamSynchronize(ctx->stream));
     return GF_OK;
 }
@@ -1119,12 +1172,12 @@ void tiles_to_matrix(gf_ctx *ctx, const double *tiles, int nres, double *out) {
 }
 
 // Gram of the node's lineshapes over grid cells (mode 0), points (1) or its data
-// cache (2) into out (nres x nres complex).  stack/nstack (device array of at most
-// GF_MAX_RES descriptors) replaces the node's resonance list when given;
+// cache (2) into out (nres x nres complex).  stack/nstack (device plan of at most
+// GF_MAX_RES rows) replaces the node's lineshapes when given;
 // td_grid selects the time-dependent grid's m13 bin count.
 gf_status run_gram(gf_ctx *ctx, const DalitzNode &d, int slot, int mode, const double *grid6, const double *m12,
                    const double *m13, const double *w, int64_t np, int eff_func, double *out,
-                   const GfResDesc *stack = nullptr, int nstack = 0, int td_grid = 0) {
+                   GfLinePlan *stack = nullptr, int nstack = 0, int td_grid = 0) {
     gf_status st = ensure_layout(ctx);
     if(st)
         return st;
@@ -1138,8 +1191,8 @@ gf_status run_gram(gf_ctx *ctx, const DalitzNode &d, int slot, int mode, const d
     st = flush_uploads(ctx);
     if(st)
         return st;
-    int64_t nb = (np + 127) / 128;
-    int64_t cap = (int64_t)ctx->cu_count * 4;
+    int64_t nb = (np + GG_BLOCK - 1) / GG_BLOCK;
+    int64_t cap = (int64_t)ctx->cu_count * GG_PER_CU;
     if(nb > cap)
         nb = cap;
     if(nb < 1)
@@ -1148,10 +1201,10 @@ gf_status run_gram(gf_ctx *ctx, const DalitzNode &d, int slot, int mode, const d
     if(st)
         return st;
     GfProgArgs a         = prog_args(ctx);
-    const GfResDesc *res = stack ? stack : ctx->d_res + slot * GF_MAX_RES;
+    GfLinePlan *plan     = stack ? stack : ctx->d_plan + slot;
     const int nres       = stack ? nstack : d.nres;
     int rc = gfk::launch_gram(a, mode, grid6, m12, m13, w, np, slot, d.col_m12, d.col_m13, eff_pc, eff_cval, td_grid,
-                              res, nres, ctx->d_gram_partials, ctx->d_gram_tiles, (int)nb, ctx->stream);
+                              plan, nres, ctx->d_gram_partials, ctx->d_gram_tiles, (int)nb, ctx->stream);
     if(rc)
         return fail(GF_ERR_HIP, "Gram launch failed (%d)", rc);
     GF_HIP(hipMemcpyAsync(ctx->h_gram_tiles, ctx->d_gram_tiles, 768 * sizeof(double), hipMemcpyDeviceToHost,
@@ -1258,7 +1311,7 @@ gf_status gf_ctx_create(gf_ctx **out, int device) {
     TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     TRY(hipMalloc((void **)&c->d_cols, GF_MAX_OBS * sizeof(double *)));
     TRY(hipMalloc((void **)&c->d_dz, GF_MAX_DALITZ * sizeof(GfDalitzSlot)));
-    TRY(hipMalloc((void **)&c->d_res, GF_MAX_DALITZ * GF_MAX_RES * sizeof(GfResDesc)));
+    TRY(hipMalloc((void **)&c->d_plan, (GF_MAX_DALITZ + 1) * sizeof(GfLinePlan)));
     TRY(hipMalloc((void **)&c->d_partials, GF_MAX_PARTIALS * sizeof(gfk::Partial)));
     TRY(hipMalloc((void **)&c->d_counter, 64));
     TRY(hipMalloc((void **)&c->d_result, 64));
@@ -1323,7 +1376,7 @@ void gf_ctx_destroy(gf_ctx *c) {
     if(c->h_multi_out)
         (void)hipHostFree(c->h_multi_out);
     void *dev[] = {c->col_base,  c->d_cols,   c->d_params,   c->d_consts,        c->d_norms,
-                   c->d_obsid,   c->d_ins,    c->d_dz,       c->d_res,           c->d_partials,
+                   c->d_obsid,   c->d_ins,    c->d_dz,       c->d_plan,          c->d_partials,
                    c->d_counter, c->d_result, c->d_err, c->d_gram_partials, c->d_gram_tiles,
                    c->d_fuse_slots};
     for(void *p : dev)
@@ -2048,7 +2101,7 @@ gf_status gf_dalitz_cache(gf_ctx *ctx, int dalitz_func, uint64_t res_mask) {
     if(nb > (int64_t)ctx->cu_count * 8)
         nb = (int64_t)ctx->cu_count * 8;
     GfProgArgs a = prog_args(ctx);
-    int rc = gfk::launch_dalitz_cache(a, slot, wc.offset, wc.n, mask, ctx->d_res + slot * GF_MAX_RES, d->nres,
+    int rc = gfk::launch_dalitz_cache(a, slot, wc.offset, wc.n, mask, ctx->d_plan + slot,
                                       (int)(nb < 1 ? 1 : nb), ctx->stream);
     if(rc)
         return fail(GF_ERR_HIP, "cache launch failed (%d)", rc);
@@ -2199,9 +2252,7 @@ gf_status gf_tddp_gram(gf_ctx *ctx, int tddp_func, const double grid6[6], double
     const int ng = (int)groups.size();
     std::vector<std::complex<double>> G((size_t)m * m);
     std::vector<char> have((size_t)m * m, 0);
-    GfResDesc *dstack = nullptr;
-    if(hipMalloc((void **)&dstack, GF_MAX_RES * sizeof(GfResDesc)) != hipSuccess)
-        return fail(GF_ERR_NOMEM, "cannot allocate the Gram stack");
+    GfLinePlan *dstack = ctx->d_plan + GF_MAX_DALITZ, stack_plan;
     gf_status st = GF_OK;
     for(int u = 0; u < ng && !st; u++) {
         for(int v = (ng == 1 ? 0 : u + 1); v < ng && !st; v++) {
@@ -2216,8 +2267,8 @@ gf_status gf_tddp_gram(gf_ctx *ctx, int tddp_func, const double grid6[6], double
             std::vector<GfResDesc> st_res(idx.size());
             for(size_t k = 0; k < idx.size(); k++)
                 st_res[k] = all[idx[k]];
-            if(hipMemcpyAsync(dstack, st_res.data(), st_res.size() * sizeof(GfResDesc), hipMemcpyHostToDevice,
-                              ctx->stream) != hipSuccess
+            line_plan(ctx, st_res.data(), (int)st_res.size(), false, stack_plan);
+            if(hipMemcpyAsync(dstack, &stack_plan, sizeof(stack_plan), hipMemcpyHostToDevice, ctx->stream) != hipSuccess
                || hipStreamSynchronize(ctx->stream) != hipSuccess) {
                 st = fail(GF_ERR_HIP, "copy of the Gram stack failed");
                 break;
@@ -2236,7 +2287,6 @@ gf_status gf_tddp_gram(gf_ctx *ctx, int tddp_func, const double grid6[6], double
                 }
         }
     }
-    (void)hipFree(dstack);
     if(st)
         return st;
     for(int i = 0; i < n; i++)
@@ -2368,7 +2418,7 @@ gf_status gf_time_dalitz_cache(gf_ctx *ctx, int dalitz_func, int reps, double *m
     uint32_t mask = d->nres >= 32 ? 0xffffffffu : ((1u << d->nres) - 1u);
     GF_HIP(hipEventRecord(ctx->ev0, ctx->stream));
     for(int r = 0; r < reps; r++) {
-        int rc = gfk::launch_dalitz_cache(a, slot, wc.offset, wc.n, mask, ctx->d_res + slot * GF_MAX_RES, d->nres,
+        int rc = gfk::launch_dalitz_cache(a, slot, wc.offset, wc.n, mask, ctx->d_plan + slot,
                                           (int)(nb < 1 ? 1 : nb), ctx->stream);
         if(rc)
             return fail(GF_ERR_HIP, "cache launch failed (%d)", rc);
@@ -2996,7 +3046,7 @@ gf_status gf_dalitz_generate(gf_ctx *ctx, int dalitz_func, int64_t n, uint64_t s
     const uint64_t key = gfd::mix64(seed ^ 0x6A09E667F3BCC909ull);
     int64_t have = 0, base = 0;
     auto pass = [&](double env) -> gf_status {
-        if(gfk::launch_dalitz_candidates(a, ctx->d_res + slot * GF_MAX_RES, d->nres, d->p_coup, eff_pc, eff_cval,
+        if(gfk::launch_dalitz_candidates(a, ctx->d_plan + slot, d->p_coup, eff_pc, eff_cval,
                                          d->col_m12,
                                          d->col_m13, box, key, base, B, env, c, c + B, flag, bcount, bmax,
                                          ctx->stream))

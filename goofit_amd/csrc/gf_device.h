@@ -253,89 +253,6 @@ __device__ __forceinline__ double damping_factor_square_norm(double cmmom, int s
     return (spin == 2) ? dfsqres : dfsq;
 }
 
-// spinFactor, Resonance.cu:99-155 (PAIR_12 = 0, PAIR_13 = 1, PAIR_23 = 2)
-__device__ __forceinline__ double spin_factor(unsigned spin, const GfDecay &d, double m12, double m13, double m23,
-                                              unsigned cyc) {
-    if(0 == spin)
-        return 1;
-    double _mA  = (0 == cyc ? d.daug1Mass : (1 == cyc ? d.daug3Mass : d.daug2Mass));
-    double _mB  = (0 == cyc ? d.daug2Mass : (1 == cyc ? d.daug1Mass : d.daug3Mass));
-    double _mC  = (0 == cyc ? d.daug3Mass : (1 == cyc ? d.daug2Mass : d.daug1Mass));
-    double _mAC = (0 == cyc ? m13 : (1 == cyc ? m23 : m12));
-    double _mBC = (0 == cyc ? m23 : (1 == cyc ? m12 : m13));
-    double _mAB = (0 == cyc ? m12 : (1 == cyc ? m13 : m23));
-    double massFactor = 1.0 / (_mAB);
-    double sFactor    = -1;
-    sFactor *= ((_mBC - _mAC) + (massFactor * (d.motherMass * d.motherMass - _mC * _mC) * (_mA * _mA - _mB * _mB)));
-    if(2 == spin) {
-        sFactor *= sFactor;
-        double t1        = d.motherMass * d.motherMass - _mC * _mC;
-        double extraterm = ((_mAB - (2 * d.motherMass * d.motherMass) - (2 * _mC * _mC)) + massFactor * (t1 * t1));
-        double t2        = _mA * _mA - _mB * _mB;
-        extraterm *= ((_mAB - (2 * _mA * _mA) - (2 * _mB * _mB)) + massFactor * (t2 * t2));
-        extraterm /= 3;
-        sFactor -= extraterm;
-    }
-    return sFactor;
-}
-
-// plainBW<I>, src/PDFs/physics/resonances/RBW.cu:9-86
-template <int I>
-__device__ __forceinline__ double2 rbw(const GfDecay &d, double resmass, double reswidth, unsigned spin,
-                                       unsigned cyclic_index, bool norm, double m12, double m13, double m23) {
-    double2 result  = make_double2(0.0, 0.0);
-    double resmass2 = resmass * resmass;
-#pragma unroll
-    for(int i = 0; i < I; i++) {
-        double rMassSq      = (0 == cyclic_index ? m12 : (1 == cyclic_index ? m13 : m23));
-        double mass_daug1   = 2 == cyclic_index ? d.daug2Mass : d.daug1Mass;
-        double mass_daug2   = 0 == cyclic_index ? d.daug2Mass : d.daug3Mass;
-        double bachelorMass = (0 == cyclic_index ? d.daug3Mass : (1 == cyclic_index ? d.daug2Mass : d.daug1Mass));
-        double frFactor       = 1;
-        double frFactorMother = 1;
-        double measureDaughterMoms = two_body_cm_mom(rMassSq, mass_daug1, mass_daug2);
-        double nominalDaughterMoms = two_body_cm_mom(resmass2, mass_daug1, mass_daug2);
-        double measureDaughterMomsMother;
-        double nominalDaughterMomsMother = 0;
-        if(norm) {
-            measureDaughterMomsMother = two_body_cm_mother_mom(rMassSq, d.motherMass, bachelorMass);
-            nominalDaughterMomsMother = two_body_cm_mother_mom(resmass2, d.motherMass, bachelorMass);
-        } else {
-            measureDaughterMomsMother = two_body_cm_mom(d.motherMass * d.motherMass, sqrt(rMassSq), bachelorMass);
-        }
-        if(0 != spin) {
-            if(norm) {
-                frFactor = damping_factor_square_norm(nominalDaughterMoms, spin, d.meson_radius)
-                           / damping_factor_square_norm(measureDaughterMoms, spin, d.meson_radius);
-                frFactorMother = damping_factor_square_norm(nominalDaughterMomsMother, spin, d.mother_meson_radius)
-                                 / damping_factor_square_norm(measureDaughterMomsMother, spin, d.mother_meson_radius);
-            } else {
-                frFactor       = damping_factor_square(measureDaughterMoms, spin, d.meson_radius);
-                frFactorMother = damping_factor_square(measureDaughterMomsMother, spin, d.mother_meson_radius);
-            }
-        }
-        double A  = (resmass2 - rMassSq);
-        double B  = resmass2 * reswidth * odd_power(measureDaughterMoms / nominalDaughterMoms, spin) * frFactor
-                   / sqrt(rMassSq);
-        double C  = 1.0 / (A * A + B * B);
-        double re = A * C, im = B * C;
-        double s1 = sqrt(frFactor);
-        re *= s1;
-        im *= s1;
-        double s2 = sqrt(frFactorMother);
-        re *= s2;
-        im *= s2;
-        double sf = spin_factor(spin, d, m12, m13, m23, cyclic_index);
-        re *= sf;
-        im *= sf;
-        result.x += re;
-        result.y += im;
-        if(I > 1)
-            cyclic_index = (cyclic_index + 1) % 3;
-    }
-    return result;
-}
-
 // hFun, dh_dsFun, fsFun, dFun: Resonance.cu:5-46 (pi truncated to 3.14159265359 as there)
 __device__ __forceinline__ double h_fun(double s, double daug2Mass, double daug3Mass) {
     const double _pi = 3.14159265359;
@@ -349,14 +266,6 @@ __device__ __forceinline__ double dh_ds_fun(double s, double daug2Mass, double d
     double k_s       = two_body_cm_mom(s, daug2Mass, daug3Mass);
     return h_fun(s, daug2Mass, daug3Mass) * (1.0 / (8.0 * (k_s * k_s)) - 1.0 / (2.0 * s)) + 1.0 / (2.0 * _pi * s);
 }
-__device__ __forceinline__ double fs_fun(double s, double m2, double gam, double daug2Mass, double daug3Mass) {
-    double k_s   = two_body_cm_mom(s, daug2Mass, daug3Mass);
-    double k_Am2 = two_body_cm_mom(m2, daug2Mass, daug3Mass);
-    double f     = gam * m2 / (k_Am2 * k_Am2 * k_Am2);
-    f *= ((k_s * k_s) * (h_fun(s, daug2Mass, daug3Mass) - h_fun(m2, daug2Mass, daug3Mass))
-          + (m2 - s) * (k_Am2 * k_Am2) * dh_ds_fun(m2, daug2Mass, daug3Mass));
-    return f;
-}
 __device__ __forceinline__ double d_fun(double s, double daug2Mass, double daug3Mass) {
     const double _pi = 3.14159265359;
     double sm        = daug2Mass + daug3Mass;
@@ -367,71 +276,137 @@ __device__ __forceinline__ double d_fun(double s, double daug2Mass, double daug3
            - sm24 * m / (_pi * (k_m2 * k_m2 * k_m2));
 }
 
-// gouSak, src/PDFs/physics/resonances/GS.cu:9-75 (dFun/fsFun take daug2/daug3 masses in every channel, as there)
-__device__ __forceinline__ double2 gounaris_sakurai(const GfDecay &d, double resmass, double reswidth, unsigned spin,
-                                                   unsigned cyclic_index, bool norm, double m12, double m13,
-                                                   double m23) {
-    double rMassSq      = (0 == cyclic_index ? m12 : (1 == cyclic_index ? m13 : m23));
-    double bachelorMass = (0 == cyclic_index ? d.daug3Mass : (1 == cyclic_index ? d.daug2Mass : d.daug1Mass));
-    double frFactor     = 1;
-    double frFactorD    = 1;
-    resmass *= resmass;
-    double md1 = (2 == cyclic_index ? d.daug2Mass : d.daug1Mass);
-    double md2 = (0 == cyclic_index ? d.daug2Mass : d.daug3Mass);
-    double measureDaughterMoms = two_body_cm_mom(rMassSq, md1, md2);
-    double nominalDaughterMoms = two_body_cm_mom(resmass, md1, md2);
-    double measureDaughterMomsMother;
-    double nominalDaughterMomsMother = 0;
-    if(norm) {
-        measureDaughterMomsMother = two_body_cm_mother_mom(rMassSq, d.motherMass, bachelorMass);
-        nominalDaughterMomsMother = two_body_cm_mother_mom(resmass, d.motherMass, bachelorMass);
-    } else {
-        measureDaughterMomsMother = two_body_cm_mom(d.motherMass * d.motherMass, sqrt(rMassSq), bachelorMass);
+// ------------------------------------------------------------- lineshapes
+//
+// plainBW (src/PDFs/physics/resonances/RBW.cu:9-86) and gouSak (GS.cu:9-75), each
+// (A + iB) / (A^2 + B^2) sqrt(F F_mother) S(spin), factorised.  With q, p the momenta of
+// the daughters and of the bachelor at the point and q0, p0 at the nominal mass,
+//   plain:  A = m^2 - s,         B = m^2 G (q / q0)^(2 spin + 1) F / sqrt(s)
+//   GS:     A = m^2 - s + f(s),  B = m G (q / q0)^(2 spin + 1) F,  times 1 + d G / m
+// and F = D(q0) / D(q) (or D'(q) without normalisation), F_mother likewise.  So B =
+// kb bf and the amplitude's factor is ks sf, where bf = q^(2 spin + 1) / (D(q) sqrt(s)) and
+// sf = S / sqrt(D(q) D(p)) depend on the point only and kb, ks on the mass and width only:
+// line_class forms the former once for all resonances of a class, k_line_plan the latter
+// once per launch, and a resonance costs one division per point.  (Evaluating each
+// shape apart took 422 FP64 operations and a dozen square roots and divisions.)
+// The momenta keep the thresholds' rules: a factor 1 - (ma + mb)^2 / s below zero is 1.
+
+// At one point: s the pair's mass squared, r = 1 / s, u = q / sqrt(s), q2 = q^2; bf and sf
+// as above.
+
+// The pair's part: s, 1 / s and the momentum (two_body_cm_mom).
+__device__ __forceinline__ void line_pair(const GF_CONST GfLineClass &c, double m12, double m13, double m23,
+                                          double &s, double &r, double &u, double &q2) {
+    s         = 0 == c.pair ? m12 : (1 == c.pair ? m13 : m23);
+    double k1 = 1 - c.sum2 / s;
+    k1        = k1 >= 0 ? k1 : 1;
+    if(c.dif2 != 0) {  // uniform: equal daughter masses give exactly 1
+        const double k2 = 1 - c.dif2 / s;
+        k1 *= k2 >= 0 ? k2 : 1;
     }
-    if(0 != spin) {
-        if(norm) {
-            frFactor = damping_factor_square_norm(nominalDaughterMoms, spin, d.meson_radius);
-            frFactor /= damping_factor_square_norm(measureDaughterMoms, spin, d.meson_radius);
-            frFactorD = damping_factor_square_norm(nominalDaughterMomsMother, spin, d.mother_meson_radius);
-            frFactorD /= damping_factor_square_norm(measureDaughterMomsMother, spin, d.mother_meson_radius);
-        } else {
-            frFactor  = damping_factor_square(measureDaughterMoms, spin, d.meson_radius);
-            frFactorD = damping_factor_square(measureDaughterMomsMother, spin, d.mother_meson_radius);
-        }
-    }
-    double D = (1.0 + d_fun(resmass, d.daug2Mass, d.daug3Mass) * reswidth / sqrt(resmass));
-    double E = resmass - rMassSq + fs_fun(rMassSq, resmass, reswidth, d.daug2Mass, d.daug3Mass);
-    double F = sqrt(resmass) * reswidth * odd_power(measureDaughterMoms / nominalDaughterMoms, spin) * frFactor;
-    D /= (E * E + F * F);
-    double re = D * E, im = D * F;
-    double s1 = sqrt(frFactor);
-    re *= s1;
-    im *= s1;
-    double s2 = sqrt(frFactorD);
-    re *= s2;
-    im *= s2;
-    double sf = spin_factor(spin, d, m12, m13, m23, cyclic_index);
-    re *= sf;
-    im *= sf;
-    return make_double2(re, im);
+    r  = 1.0 / s;
+    u  = 0.5 * sqrt(k1);
+    q2 = 0.25 * s * k1;
 }
 
-// One resonance of a Dalitz node: getResonanceAmplitude (Amp3Body_TD.cu:36-39)
-// dispatched on the wave-uniform kind instead of a function pointer.
-__device__ __forceinline__ double2 lineshape(const GfResDesc &r, const double *__restrict__ P,
-                                             const double *__restrict__ Cn, const GfDecay &d, double m12,
-                                             double m13, double m23) {
-    if(r.kind == GR_NONRES)
-        return make_double2(1.0, 0.0);  // nonres, NonRes.cu:8-11
-    double mass   = P[r.p];
-    double width  = P[r.p + 1];
-    unsigned spin = (unsigned)Cn[r.c];
-    unsigned cyc  = (unsigned)Cn[r.c + 1];
-    bool norm     = Cn[r.c + 2] != 0.0;
-    switch(r.kind) {
-    case GR_RBW: return rbw<1>(d, mass, width, spin, cyc, norm, m12, m13, m23);
-    case GR_RBW_SYM: return rbw<2>(d, mass, width, spin, cyc, norm, m12, m13, m23);
-    default: return gounaris_sakurai(d, mass, width, spin, cyc, norm, m12, m13, m23);
+// The class's part: barrier and spin factors (dampingFactorSquareNorm, dampingFactorSquare
+// and spinFactor, Resonance.cu:77-155).
+__device__ __forceinline__ void line_class(const GF_CONST GfLinePlan *__restrict__ plan,
+                                           const GF_CONST GfLineClass &c, double m12, double m13, double m23, double s,
+                                           double r, double u, double q2, double &bf, double &sf) {
+    bf = u;
+    sf = 1.0;
+    if(0 == c.spin)
+        return;
+    for(int k = 0; k < c.spin; ++k)
+        bf *= q2;
+    const double z = c.r2 * q2;
+    double g;  // sqrt(g) multiplies the amplitude
+    if(c.norm) {
+        // the bachelor's momentum in the form of two_body_cm_mother_mom, 0.5 s / M times two
+        // square roots that are 1 below s = (M - mc)^2, the end of the plot
+        double k = 1.0;
+        if(s >= c.mdif2 * (1 - 1e-15)) {
+            const double k1 = 1 - c.msum2 / s, k2 = 1 - c.mdif2 / s;
+            k = (k1 >= 0 ? k1 : 1) * (k2 >= 0 ? k2 : 1);
+        }
+        const double zm = c.rm2 * s * s * k;
+        const double dq = 2 == c.spin ? fma(z, z + 3, 9) : 1 + z;
+        const double dm = 2 == c.spin ? fma(zm, zm + 3, 9) : 1 + zm;
+        g               = 1.0 / (dq * dm);
+        bf *= g * dm;
+    } else {
+        const double pm = two_body_cm_mom(plan->m2, sqrt(s), c.mc);
+        const double f  = 2 == c.spin ? 13 * z / ((z - 3) * (z - 3)) + 9 * z * z : 2 * z;
+        g               = f * damping_factor_square(pm, c.spin, plan->rm);
+        bf *= f;
+    }
+    const double sAC = 0 == c.pair ? m13 : (1 == c.pair ? m23 : m12);
+    const double sBC = 0 == c.pair ? m23 : (1 == c.pair ? m12 : m13);
+    double f         = -fma(r, c.s0, sBC - sAC);
+    if(2 == c.spin)
+        f = fma(f, f, -(fma(r, c.s2, s - c.s1) * fma(r, c.s4, s - c.s3)) * (1.0 / 3.0));
+    sf = sqrt(g) * f;
+}
+
+// One resonance's term at the point.
+__device__ __forceinline__ double2 line_term(const GF_CONST GfLinePlan *__restrict__ plan, const GF_CONST GfLineTerm &t,
+                                             double s, double bf, double sf) {
+    double A = t.m2 - s, B = t.kb * bf;
+    if(t.kind == GR_GS) {
+        // hFun takes the masses of daughters 2 and 3 in every channel, as there
+        const double _pi = 3.14159265359;
+        double k1        = 1 - plan->gsum2 / s;
+        k1               = k1 >= 0 ? k1 : 1;
+        const double k2  = 1 - plan->gdif2 / s;
+        k1 *= k2 >= 0 ? k2 : 1;
+        const double rs = sqrt(s), u = 0.5 * sqrt(k1);
+        const double h  = (2 / _pi) * u * gfmath::log_d(rs * fma(2, u, 1) * plan->ginv);
+        A               = fma(t.f0, fma(0.25 * s * k1, h - t.h0, A * t.d0), A);
+        B *= rs;
+    }
+    const double C = t.ks * sf / fma(A, A, B * B);
+    return make_double2(A * C, B * C);
+}
+
+// Every wave of the plan whose resonance is in mask, at one point: emit(row, swap, add,
+// value).  m23 is the same for the swapped point (m13, m12).  All control flow is
+// uniform over the wave.
+template <class Emit>
+__device__ __forceinline__ void line_waves(const GfLinePlan *__restrict__ plan_, double m12, double m13,
+                                           double m23, uint32_t mask, const Emit &emit) {
+    const GF_CONST GfLinePlan *__restrict__ plan = as_const(plan_);
+    double s = 0, r = 0, u = 0, q2 = 0, bf, sf;
+    int chan = -1;
+    for(int ci = 0; ci < plan->nclass; ++ci) {
+        const GF_CONST GfLineClass &c = plan->cls[ci];
+        if(!(c.res & mask))
+            continue;
+        const int k1 = c.first + c.count;
+        if(c.pair < 0) {  // nonres, NonRes.cu:8-11
+            for(int k = c.first; k < k1; ++k)
+                if((mask >> plan->term[k].res) & 1u)
+                    emit(plan->term[k].res, c.swap, 0, make_double2(1.0, 0.0));
+            continue;
+        }
+        const double x = c.swap ? m13 : m12, y = c.swap ? m12 : m13;
+        if(chan != 4 * c.swap + c.pair) {
+            chan = 4 * c.swap + c.pair;
+            line_pair(c, x, y, m23, s, r, u, q2);
+        }
+        line_class(plan, c, x, y, m23, s, r, u, q2, bf, sf);
+        // two terms at a time: their divisions are independent chains
+        int k = c.first;
+        for(; k + 1 < k1; k += 2) {
+            const GF_CONST GfLineTerm &t0 = plan->term[k], &t1 = plan->term[k + 1];
+            const double2 v0 = line_term(plan, t0, s, bf, sf), v1 = line_term(plan, t1, s, bf, sf);
+            if((mask >> t0.res) & 1u)
+                emit(t0.res, c.swap, t0.add, v0);
+            if((mask >> t1.res) & 1u)
+                emit(t1.res, c.swap, t1.add, v1);
+        }
+        if(k < k1 && ((mask >> plan->term[k].res) & 1u))
+            emit(plan->term[k].res, c.swap, plan->term[k].add, line_term(plan, plan->term[k], s, bf, sf));
     }
 }
 

@@ -79,6 +79,43 @@ struct GfResDesc {
     int32_t swap;  // 1: evaluated at (m13, m12) -- the B wave of a time-dependent node
 };
 
+// The lineshapes of a Dalitz node as the kernels evaluate them.  Resonances with the
+// same pair, spin, normalisation flag and orientation (swap) form a class: everything
+// that depends on the point and not on the mass and width (momenta, barrier factors,
+// the spin factor) is formed once per class, and a resonance adds one term (a plain or
+// Gounaris-Sakurai denominator).  The structure comes from the host with the program;
+// k_line_plan fills in the numbers from the current masses, widths and decay constants
+// before each use.
+#define GF_MAX_TERMS (4 * GF_MAX_RES)  // both halves of symmetrised shapes, A and B waves
+struct GfLineClass {
+    int32_t first, count;  // its terms
+    int32_t pair, spin, norm, swap;  // pair -1: the non-resonant wave, 1 inside the plot
+    uint32_t res;          // bit i: a term of resonance i
+    int32_t pad;
+    double sum2, dif2;     // (ma + mb)^2, (ma - mb)^2 of the pair
+    double mc;             // the bachelor's mass
+    double msum2, mdif2;   // (M + mc)^2, (M - mc)^2
+    double r2, rm2;        // meson radius squared, mother radius squared / (4 M^2)
+    double s0, s1, s2, s3, s4;  // spin factor constants
+};
+struct GfLineTerm {
+    int32_t kind;  // GfRes: GR_RBW, GR_GS or GR_NONRES
+    int32_t res;   // destination row
+    int32_t p;     // index in params[] of mass (width at p+1)
+    int32_t cls;   // its class
+    int32_t add;   // 1: adds to the row (the second half of a symmetrised shape)
+    double m2;     // mass^2
+    double kb, ks; // factors of the denominator's imaginary part and of the amplitude
+    double f0, h0, d0;  // Gounaris-Sakurai: f(s) = f0 (k^2 (h(s) - h0) + (m^2 - s) d0)
+};
+struct GfLinePlan {
+    int32_t nclass, nterm;
+    double m2, rm;              // mother mass squared, mother radius
+    double gsum2, gdif2, ginv;  // Gounaris-Sakurai: (m2 + m3)^2, (m2 - m3)^2, 1 / (m2 + m3)
+    GfLineClass cls[GF_MAX_TERMS];
+    GfLineTerm term[GF_MAX_TERMS];
+};
+
 // Time-resolution models of a time-dependent Dalitz node.
 enum GfTimeRes : int32_t { GT_TRUTH = 0, GT_THREEGAUSS = 1 };
 
@@ -240,22 +277,25 @@ int launch_batch_points(const GfProgArgs &a, int nres, const GfBatchWork *work, 
 // Accept-reject generation: candidates (uniform in box) with accept flags, and
 // the ordered compaction of the accepted ones.
 // eff_pc >= 0: efficiency subprogram; -1: efficiency 1; -2: the constant eff_const.
-int launch_dalitz_candidates(const GfProgArgs &a, const GfResDesc *res, int nres, int p_coup, int eff_pc,
+int launch_dalitz_candidates(const GfProgArgs &a, GfLinePlan *plan, int p_coup, int eff_pc,
                              double eff_const, int id12, int id13, const double box[4], uint64_t key, int64_t base,
                              int64_t nc, double fmax, double *c12, double *c13, uint8_t *flag, int *bcount,
                              double *bmax, void *stream);
 int launch_compact(const double *c12, const double *c13, const uint8_t *flag, int64_t nc, const int64_t *boff,
                    int64_t limit, double *o12, double *o13, void *stream);
-int launch_dalitz_cache(const GfProgArgs &a, int slot, int64_t offset, int64_t n, uint32_t mask,
-                        const GfResDesc *res, int nres, int nblocks, void *stream);
+// plan (here and below): the lineshapes' structure; its numbers are filled in first.
+int launch_dalitz_cache(const GfProgArgs &a, int slot, int64_t offset, int64_t n, uint32_t mask, GfLinePlan *plan,
+                        int nblocks, void *stream);
 // mode 0: grid cells (grid6 host array); 1: points (m12, m13, w device arrays); 2: data cache of `slot`.
 // Writes 768 doubles (tiles RR, II, RI in MFMA register layout) to tiles_dev.
-// td_grid: the grid of a time-dependent node (m13 bin count grid6[5]); res[i].swap
-// evaluates entry i at (m13, m12).
+// td_grid: the grid of a time-dependent node (m13 bin count grid6[5]).
 int launch_gram(const GfProgArgs &a, int mode, const double *grid6, const double *m12, const double *m13,
                 const double *w, int64_t npoints, int slot, int id_m12, int id_m13, int eff_pc, double eff_const,
-                int td_grid, const GfResDesc *res, int nres, double *partials, double *tiles_dev, int nblocks,
+                int td_grid, GfLinePlan *plan, int nres, double *partials, double *tiles_dev, int nblocks,
                 void *stream);
+// Points per workgroup pass of the Gram kernel and its workgroups per CU (LDS).
+#define GG_BLOCK 256
+#define GG_PER_CU 2
 int launch_identity_check(const double *col, int64_t n, int32_t *flag, void *stream);
 int mfma_probe(const double *dev_a, const double *dev_b, double *dev_out, void *stream);
 }  // namespace gfk

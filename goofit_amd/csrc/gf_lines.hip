@@ -15,9 +15,76 @@ namespace {
 
 // ------------------------------------------------------------- Dalitz cache
 
-__global__ __launch_bounds__(256) void k_dalitz_cache(GfProgArgs A, int slot, int64_t offset, int64_t n,
-                                                      uint32_t mask, const GfResDesc *__restrict__ res, int nres) {
-    const GfDalitzSlot dz = A.dz[slot];
+// The numbers of a lineshape plan from the current masses, widths and decay constants,
+// one lane per term (GfLinePlan; the nominal-mass parts of plainBW and gouSak).
+__global__ __launch_bounds__(GF_MAX_TERMS) void k_line_plan(GfLinePlan *plan, const double *__restrict__ P, GfDecay d) {
+    const int t = threadIdx.x;
+    if(t == 0) {
+        const double a = d.daug2Mass + d.daug3Mass, b = d.daug2Mass - d.daug3Mass;
+        plan->m2    = d.motherMass * d.motherMass;
+        plan->rm    = d.mother_meson_radius;
+        plan->gsum2 = a * a;
+        plan->gdif2 = b * b;
+        plan->ginv  = 1.0 / a;
+    }
+    if(t >= plan->nterm)
+        return;
+    GfLineTerm &r   = plan->term[t];
+    GfLineClass &c  = plan->cls[r.cls];
+    const int pair  = c.pair, spin = c.spin;
+    if(pair < 0)
+        return;
+    const double M = d.motherMass;
+    // daughters and bachelor of the pair (RBW.cu:13-16), and the spin factor's A, B, C
+    const double da = 2 == pair ? d.daug2Mass : d.daug1Mass;
+    const double db = 0 == pair ? d.daug2Mass : d.daug3Mass;
+    const double mA = 0 == pair ? d.daug1Mass : (1 == pair ? d.daug3Mass : d.daug2Mass);
+    const double mB = 0 == pair ? d.daug2Mass : (1 == pair ? d.daug1Mass : d.daug3Mass);
+    const double mC = 0 == pair ? d.daug3Mass : (1 == pair ? d.daug2Mass : d.daug1Mass);
+    if(t == c.first) {
+        const double t1 = M * M - mC * mC, t2 = mA * mA - mB * mB;
+        c.sum2  = (da + db) * (da + db);
+        c.dif2  = (da - db) * (da - db);
+        c.mc    = mC;
+        c.msum2 = (M + mC) * (M + mC);
+        c.mdif2 = (M - mC) * (M - mC);
+        c.r2    = d.meson_radius * d.meson_radius;
+        c.rm2   = d.mother_meson_radius * d.mother_meson_radius * 0.25 / (M * M);
+        c.s0    = t1 * t2;
+        c.s1    = 2 * M * M + 2 * mC * mC;
+        c.s2    = t1 * t1;
+        c.s3    = 2 * mA * mA + 2 * mB * mB;
+        c.s4    = t2 * t2;
+    }
+    const double m  = P[r.p], w = P[r.p + 1], m2 = m * m;
+    const double q0 = gfd::two_body_cm_mom(m2, da, db);
+    double kb       = (r.kind == GR_GS ? sqrt(m2) : m2) * w / gfd::odd_power(q0, spin);
+    double ks       = 1.0;
+    if(spin != 0 && c.norm) {
+        const double p0 = gfd::two_body_cm_mother_mom(m2, M, mC);
+        const double f  = gfd::damping_factor_square_norm(q0, spin, d.meson_radius);
+        kb *= f;
+        ks = sqrt(f) * sqrt(gfd::damping_factor_square_norm(p0, spin, d.mother_meson_radius));
+    }
+    if(r.kind == GR_GS) {
+        // dFun and fsFun at the nominal mass (GS.cu:53-57)
+        const double k0 = gfd::two_body_cm_mom(m2, d.daug2Mass, d.daug3Mass);
+        ks *= 1.0 + gfd::d_fun(m2, d.daug2Mass, d.daug3Mass) * w / sqrt(m2);
+        r.f0 = w * m2 / (k0 * k0 * k0);
+        r.h0 = gfd::h_fun(m2, d.daug2Mass, d.daug3Mass);
+        r.d0 = k0 * k0 * gfd::dh_ds_fun(m2, d.daug2Mass, d.daug3Mass);
+    }
+    r.m2 = m2;
+    r.kb = kb;
+    r.ks = ks;
+}
+
+// The wave cache.  16 shapes over 1e6 events: 65 us, 1214 vector instructions per wave of 64
+// events (34 us of issue) beside 256 MB of stores (40 us at the fill rate); 290 us with each
+// shape evaluated by itself.
+__global__ __launch_bounds__(256) void k_dalitz_cache(GfProgArgs A, int slot, int64_t offset, int64_t n, uint32_t mask,
+                                                      const GfLinePlan *__restrict__ plan) {
+    const GfDalitzSlot dz = gfd::as_const(A.dz)[slot];
     const GfDecay D       = A.decay;
     double2 *wave         = const_cast<double2 *>(dz.wave);
     double2 *wave_b       = const_cast<double2 *>(dz.wave_b);  // time-dependent nodes only
@@ -27,24 +94,18 @@ __global__ __launch_bounds__(256) void k_dalitz_cache(GfProgArgs A, int slot, in
         const double m12  = c12[offset + e];
         const double m13  = c13[offset + e];
         const bool inside = gfd::in_dalitz(m12, m13, D.motherMass, D.daug1Mass, D.daug2Mass, D.daug3Mass);
-        // SpecialResonanceCalculator.cu:36-37
+        // SpecialResonanceCalculator.cu:36-37; the B wave is at the reversed point with the
+        // same m23 (SpecialWaveCalculator.cu:55-58)
         const double m23 = D.motherMass * D.motherMass + D.daug1Mass * D.daug1Mass + D.daug2Mass * D.daug2Mass
                            + D.daug3Mass * D.daug3Mass - m12 - m13;
-        for(int i = 0; i < nres; ++i) {
-            if(!((mask >> i) & 1u))
-                continue;
-            double2 w = make_double2(0.0, 0.0);
-            if(inside)
-                w = gfd::lineshape(res[i], A.params, A.consts, D, m12, m13, m23);
-            wave[(int64_t)i * dz.ncache + e] = w;
-            if(wave_b) {
-                // SpecialWaveCalculator.cu:55-58: the B wave at the reversed point, same m23
-                double2 v = make_double2(0.0, 0.0);
-                if(inside)
-                    v = gfd::lineshape(res[i], A.params, A.consts, D, m13, m12, m23);
-                wave_b[(int64_t)i * dz.ncache + e] = v;
+        gfd::line_waves(plan, m12, m13, m23, mask, [&](int i, int swap, int add, double2 v) {
+            double2 *w = (swap ? wave_b : wave) + (int64_t)i * dz.ncache + e;
+            if(add) {
+                v.x += w->x;
+                v.y += w->y;
             }
-        }
+            *w = make_double2(inside ? v.x : 0.0, inside ? v.y : 0.0);
+        });
     }
 }
 
@@ -57,7 +118,7 @@ __global__ __launch_bounds__(256) void k_dalitz_cache(GfProgArgs A, int slot, in
 // accepted when u_i * fmax < value.  Per block: accepted count and the largest
 // value (to check the envelope).
 template <bool GEN_EFF>
-__global__ __launch_bounds__(256) void k_dalitz_candidates(GfProgArgs A, const GfResDesc *__restrict__ res, int nres,
+__global__ __launch_bounds__(256) void k_dalitz_candidates(GfProgArgs A, const GfLinePlan *__restrict__ plan,
                                                            int p_coup, int eff_pc, double eff_const, int id12,
                                                            int id13, double l12,
                                                            double u12, double l13, double u13, uint64_t key,
@@ -78,13 +139,12 @@ __global__ __launch_bounds__(256) void k_dalitz_candidates(GfProgArgs A, const G
         const double m23 = D.motherMass * D.motherMass + D.daug1Mass * D.daug1Mass + D.daug2Mass * D.daug2Mass
                            + D.daug3Mass * D.daug3Mass - m12 - m13;
         double re = 0.0, im = 0.0;
-#pragma unroll 1
-        for(int r = 0; r < nres; ++r) {
-            const double2 b = gfd::lineshape(res[r], A.params, A.consts, D, m12, m13, m23);
-            const double ar = A.params[p_coup + 2 * r], ai = A.params[p_coup + 2 * r + 1];
-            re += ar * b.x - ai * b.y;
-            im += ar * b.y + ai * b.x;
-        }
+        const GF_CONST double *__restrict__ P = gfd::as_const(A.params) + p_coup;
+        gfd::line_waves(plan, m12, m13, m23, ~0u, [&](int r, int, int, double2 b) {
+            const double ar = P[2 * r], ai = P[2 * r + 1];
+            re = fma(ar, b.x, fma(-ai, b.y, re));
+            im = fma(ar, b.y, fma(ai, b.x, im));
+        });
         double eff = eff_pc == -2 ? eff_const : 1.0;
         if constexpr(GEN_EFF) {
             RegSrc<1> ev;
@@ -158,8 +218,7 @@ __global__ __launch_bounds__(256) void k_compact(const double *__restrict__ c12,
 // ------------------------------------------------------------- FP64-MFMA Gram
 
 
-#define GG_BLOCK 128  // two waves
-#define GG_LD 65      // padded LDS row (doubles): 16 lanes reading one column hit distinct banks
+#define GG_LD 65  // padded LDS row (doubles): 16 lanes reading one column hit distinct banks
 
 struct GramSrc {
     int mode;  // 0 grid, 1 points, 2 data cache
@@ -194,57 +253,64 @@ __global__ __launch_bounds__(256) void k_dalitz_cells(GramSrc S, double *m12, do
         dalitz_cell(S, p, m12[p], m13[p]);
 }
 
-// One block: 128 points per pass; each lane computes the 16 complex amplitudes of
-// its point (wave-uniform control flow), stages them in LDS component-major,
-// and each wave multiplies its 64 points as 16 MFMA k-steps for each of three
-// 16x16 output tiles: RR = R^T E R, II = I^T E I, RI = R^T E I, with
-// E = diag(eff * weight).  Partials: 3 tiles x 64 lanes x 4 values per block.
+// Each wave takes 64 points at a time, on its own: a lane computes the 16 complex
+// amplitudes of its point (wave-uniform control flow) and stages them in the wave's LDS
+// rows component-major, then the wave multiplies its 64 points as 16 MFMA k-steps for
+// each of three 16x16 output tiles: RR = R^T E R, II = I^T E I, RI = R^T E I, with
+// E = diag(eff * weight).  No barrier until the four waves' tiles are added at the end.
+// A point outside the Dalitz plot adds nothing, so a wave with none inside moves on (two
+// fifths of the waves over a box around the plot).  16 shapes on 1414 x 1414 cells: 129 us
+// (46 us of vector and 24 us of matrix-core issue; the 16.5 KB of LDS per wave leave two
+// waves per SIMD, so latency shows), 450-520 us with each shape evaluated by itself over
+// every cell.  Partials: 3 tiles x 64 lanes x 4 values per block.
 template <bool GEN_EFF>
-__global__ __launch_bounds__(GG_BLOCK) void k_gram(GfProgArgs A, GramSrc S, const GfResDesc *__restrict__ res,
-                                                   int nres, double *partials) {
-    __shared__ double Xr[2][16][GG_LD];
-    __shared__ double Xi[2][16][GG_LD];
-    __shared__ double Ew[2][64];
+__global__ __launch_bounds__(GG_BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void k_gram(
+    GfProgArgs A, GramSrc S, const GfLinePlan *__restrict__ plan, int nres, double *partials) {
+    __shared__ double Xr[GG_BLOCK / 64][16][GG_LD];
+    __shared__ double Xi[GG_BLOCK / 64][16][GG_LD];
+    __shared__ double Ew[GG_BLOCK / 64][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const GfDecay D = A.decay;
     gf_double4 RR = {0, 0, 0, 0}, II = {0, 0, 0, 0}, RI = {0, 0, 0, 0};
     const int64_t npts = S.npoints;
-    for(int64_t base = (int64_t)blockIdx.x * GG_BLOCK; base < npts; base += (int64_t)gridDim.x * GG_BLOCK) {
-        const int64_t p  = base + tid;
+    for(int i = 0; i < 16; ++i)  // rows past nres stay 0
+        Xr[wave][i][lane] = Xi[wave][i][lane] = 0.0;
+    for(int64_t base = (int64_t)blockIdx.x * GG_BLOCK + 64 * wave; base < npts;
+        base += (int64_t)gridDim.x * GG_BLOCK) {
+        const int64_t p  = base + lane;
         const bool valid = p < npts;
-        double m12 = 0.0, m13 = 0.0, wt = 1.0;
-        if(S.mode == 0) {
-            dalitz_cell(S, valid ? p : 0, m12, m13);
-        } else if(S.mode == 1) {
-            m12 = valid ? S.m12[p] : 0.0;
-            m13 = valid ? S.m13[p] : 0.0;
-            wt  = (valid && S.w) ? S.w[p] : 1.0;
-        }
         double ew = 0.0;
         if(S.mode == 2) {
             const GfDalitzSlot dz = A.dz[S.slot];
             const int64_t q       = valid ? p : 0;
-            for(int i = 0; i < GF_MAX_RES; ++i) {
-                double2 b = (i < nres) ? dz.wave[(int64_t)i * dz.ncache + q] : make_double2(0.0, 0.0);
+            for(int i = 0; i < nres; ++i) {
+                const double2 b   = dz.wave[(int64_t)i * dz.ncache + q];
                 Xr[wave][i][lane] = b.x;
                 Xi[wave][i][lane] = b.y;
             }
             ew = valid ? 1.0 : 0.0;
         } else {
+            double m12 = 0.0, m13 = 0.0, wt = 1.0;
+            if(S.mode == 0) {
+                dalitz_cell(S, valid ? p : 0, m12, m13);
+            } else {
+                m12 = valid ? S.m12[p] : 0.0;
+                m13 = valid ? S.m13[p] : 0.0;
+                wt  = (valid && S.w) ? S.w[p] : 1.0;
+            }
             const bool inside = valid && gfd::in_dalitz(m12, m13, D.motherMass, D.daug1Mass, D.daug2Mass, D.daug3Mass);
+            if(!__any(inside))
+                continue;
             const double m23  = D.motherMass * D.motherMass + D.daug1Mass * D.daug1Mass + D.daug2Mass * D.daug2Mass
                                + D.daug3Mass * D.daug3Mass - m12 - m13;
-            // one lineshape body in the loop (not 16 inlined copies): registers for occupancy
-#pragma unroll 1
-            for(int i = 0; i < GF_MAX_RES; ++i) {
-                double2 b = make_double2(0.0, 0.0);
-                if(i < nres && inside) {
-                    const bool sw = res[i].swap != 0;  // B wave of a time-dependent node
-                    b = gfd::lineshape(res[i], A.params, A.consts, D, sw ? m13 : m12, sw ? m12 : m13, m23);
+            gfd::line_waves(plan, m12, m13, m23, ~0u, [&](int i, int, int add, double2 b) {
+                if(add) {
+                    b.x += Xr[wave][i][lane];
+                    b.y += Xi[wave][i][lane];
                 }
-                Xr[wave][i][lane] = b.x;
-                Xi[wave][i][lane] = b.y;
-            }
+                Xr[wave][i][lane] = inside ? b.x : 0.0;
+                Xi[wave][i][lane] = inside ? b.y : 0.0;
+            });
             double eff = S.eff_pc == -2 ? S.eff_const : 1.0;
             if constexpr(GEN_EFF) {
                 // The fake event of SpecialResonanceIntegrator.cu:97-101: slot 0 = 2,
@@ -262,10 +328,13 @@ __global__ __launch_bounds__(GG_BLOCK) void k_gram(GfProgArgs A, GramSrc S, cons
                 run<1>(A, A.params, A.norms, S.eff_pc, ev, r0, v0, T);
                 eff = T[0];
             }
-            ew = valid ? eff * wt : 0.0;
+            ew = inside ? eff * wt : 0.0;
         }
         Ew[wave][lane] = ew;
-        __syncthreads();
+        // the wave's own LDS rows: its LDS operations complete in order, the fences keep the
+        // compiler from moving them across
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         // A operand lane l: A[i = l%16][k = l/16]; B operand lane l: B[k = l/16][j = l%16].
         const int comp = lane & 15, sub = lane >> 4;
 #pragma unroll
@@ -279,16 +348,19 @@ __global__ __launch_bounds__(GG_BLOCK) void k_gram(GfProgArgs A, GramSrc S, cons
             II = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, bi, II, 0, 0, 0);
             RI = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, RI, 0, 0, 0);
         }
-        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
-    // add wave 1 into wave 0 through LDS, then write this block's partial
-    double *stage = &Xr[0][0][0];  // 2*16*65 doubles >= 64*12
-    if(wave == 1) {
+    // add the waves' tiles in order through LDS, then write this block's partial
+    __syncthreads();
+    double *stage = &Xr[0][0][0];  // 4 * 16 * 65 doubles >= 3 * 768
+    if(wave > 0) {
+        double *mine = stage + (wave - 1) * 768;
 #pragma unroll
         for(int r = 0; r < 4; ++r) {
-            stage[(0 * 4 + r) * 64 + lane] = RR[r];
-            stage[(1 * 4 + r) * 64 + lane] = II[r];
-            stage[(2 * 4 + r) * 64 + lane] = RI[r];
+            mine[(0 * 4 + r) * 64 + lane] = RR[r];
+            mine[(1 * 4 + r) * 64 + lane] = II[r];
+            mine[(2 * 4 + r) * 64 + lane] = RI[r];
         }
     }
     __syncthreads();
@@ -296,40 +368,61 @@ __global__ __launch_bounds__(GG_BLOCK) void k_gram(GfProgArgs A, GramSrc S, cons
         double *out = partials + (int64_t)blockIdx.x * 768;
 #pragma unroll
         for(int r = 0; r < 4; ++r) {
-            out[(0 * 4 + r) * 64 + lane] = RR[r] + stage[(0 * 4 + r) * 64 + lane];
-            out[(1 * 4 + r) * 64 + lane] = II[r] + stage[(1 * 4 + r) * 64 + lane];
-            out[(2 * 4 + r) * 64 + lane] = RI[r] + stage[(2 * 4 + r) * 64 + lane];
+            double t[3] = {RR[r], II[r], RI[r]};
+#pragma unroll
+            for(int q = 0; q < 3; ++q) {
+                for(int w = 0; w < GG_BLOCK / 64 - 1; ++w)
+                    t[q] += stage[w * 768 + (q * 4 + r) * 64 + lane];
+                out[(q * 4 + r) * 64 + lane] = t[q];
+            }
         }
     }
 }
 
-// Sum the per-block Gram partials: one block per output element, each thread a
-// fixed stride of blocks, then a fixed-order tree (deterministic for a given grid).
+// Sum the per-block Gram partials: a workgroup takes 8 output elements (64 bytes of each
+// block's row), 32 lanes each with a fixed stride of blocks, then the lanes' sums in order
+// (deterministic for a given grid).
 __global__ __launch_bounds__(256) void k_gram_final(const double *__restrict__ partials, int nblocks, double *out) {
-    const int e = blockIdx.x;  // 0..767
+    __shared__ double ls[32][8], lc[32][8];
+    const int e = threadIdx.x & 7, row = threadIdx.x >> 3;
     double s = 0.0, c = 0.0;
-    for(int b = threadIdx.x; b < nblocks; b += blockDim.x)
-        gfd::kb_add(s, c, partials[(int64_t)b * 768 + e]);
-    block_reduce(s, c);
-    if(threadIdx.x == 0)
-        out[e] = gfd::kb_total(s, c);
+#pragma unroll 4
+    for(int b = row; b < nblocks; b += 32)
+        gfd::kb_add(s, c, partials[(int64_t)b * 768 + 8 * blockIdx.x + e]);
+    ls[row][e] = s;
+    lc[row][e] = c;
+    __syncthreads();
+    if(row == 0) {
+        for(int k = 1; k < 32; ++k)
+            gfd::kb_merge(s, c, ls[k][e], lc[k][e]);
+        out[8 * blockIdx.x + e] = gfd::kb_total(s, c);
+    }
 }
 
 }  // namespace
 
 namespace gfk {
 
-int launch_dalitz_candidates(const GfProgArgs &a, const GfResDesc *res, int nres, int p_coup, int eff_pc,
+static int fill_plan(const GfProgArgs &a, GfLinePlan *plan, hipStream_t s) {
+    hipLaunchKernelGGL(k_line_plan, dim3(1), dim3(GF_MAX_TERMS), 0, s, plan, a.params, a.decay);
+    return check(hipGetLastError());
+}
+
+
+int launch_dalitz_candidates(const GfProgArgs &a, GfLinePlan *plan, int p_coup, int eff_pc,
                              double eff_const, int id12, int id13, const double box[4], uint64_t key, int64_t base,
                              int64_t nc, double fmax, double *c12, double *c13, uint8_t *flag, int *bcount,
                              double *bmax, void *stream) {
     const int nb = (int)((nc + 255) / 256);
+    int rc       = fill_plan(a, plan, (hipStream_t)stream);
+    if(rc)
+        return rc;
     if(eff_pc >= 0)
-        hipLaunchKernelGGL(k_dalitz_candidates<true>, dim3(nb), dim3(256), 0, (hipStream_t)stream, a, res, nres,
+        hipLaunchKernelGGL(k_dalitz_candidates<true>, dim3(nb), dim3(256), 0, (hipStream_t)stream, a, plan,
                            p_coup, eff_pc, eff_const, id12, id13, box[0], box[1], box[2], box[3], key, base, nc, fmax,
                            c12, c13, flag, bcount, bmax);
     else
-        hipLaunchKernelGGL(k_dalitz_candidates<false>, dim3(nb), dim3(256), 0, (hipStream_t)stream, a, res, nres,
+        hipLaunchKernelGGL(k_dalitz_candidates<false>, dim3(nb), dim3(256), 0, (hipStream_t)stream, a, plan,
                            p_coup, eff_pc, eff_const, id12, id13, box[0], box[1], box[2], box[3], key, base, nc, fmax,
                            c12, c13, flag, bcount, bmax);
     return check(hipGetLastError());
@@ -343,16 +436,19 @@ int launch_compact(const double *c12, const double *c13, const uint8_t *flag, in
     return check(hipGetLastError());
 }
 
-int launch_dalitz_cache(const GfProgArgs &a, int slot, int64_t offset, int64_t n, uint32_t mask, const GfResDesc *res,
-                        int nres, int nblocks, void *stream) {
-    hipLaunchKernelGGL(k_dalitz_cache, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, a, slot, offset, n, mask, res,
-                       nres);
+int launch_dalitz_cache(const GfProgArgs &a, int slot, int64_t offset, int64_t n, uint32_t mask, GfLinePlan *plan,
+                        int nblocks, void *stream) {
+    int rc = fill_plan(a, plan, (hipStream_t)stream);
+    if(rc)
+        return rc;
+    hipLaunchKernelGGL(k_dalitz_cache, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, a, slot, offset, n, mask,
+                       plan);
     return check(hipGetLastError());
 }
 
 int launch_gram(const GfProgArgs &a, int mode, const double *grid6, const double *m12, const double *m13,
                 const double *w, int64_t npoints, int slot, int id_m12, int id_m13, int eff_pc, double eff_const,
-                int td_grid, const GfResDesc *res, int nres, double *partials, double *tiles_dev, int nblocks,
+                int td_grid, GfLinePlan *plan, int nres, double *partials, double *tiles_dev, int nblocks,
                 void *stream) {
     GramSrc S;
     S.mode = mode;
@@ -377,14 +473,16 @@ int launch_gram(const GfProgArgs &a, int mode, const double *grid6, const double
     S.eff_pc    = eff_pc;
     S.eff_const = eff_const;
     hipStream_t s = (hipStream_t)stream;
-    if(eff_pc >= 0)
-        hipLaunchKernelGGL(k_gram<true>, dim3(nblocks), dim3(GG_BLOCK), 0, s, a, S, res, nres, partials);
-    else
-        hipLaunchKernelGGL(k_gram<false>, dim3(nblocks), dim3(GG_BLOCK), 0, s, a, S, res, nres, partials);
-    int rc = check(hipGetLastError());
+    int rc = mode == 2 ? 0 : fill_plan(a, plan, s);
     if(rc)
         return rc;
-    hipLaunchKernelGGL(k_gram_final, dim3(768), dim3(256), 0, s, partials, nblocks, tiles_dev);
+    if(eff_pc >= 0)
+        hipLaunchKernelGGL(k_gram<true>, dim3(nblocks), dim3(GG_BLOCK), 0, s, a, S, plan, nres, partials);
+    else
+        hipLaunchKernelGGL(k_gram<false>, dim3(nblocks), dim3(GG_BLOCK), 0, s, a, S, plan, nres, partials);
+    if((rc = check(hipGetLastError())))
+        return rc;
+    hipLaunchKernelGGL(k_gram_final, dim3(768 / 8), dim3(256), 0, s, partials, nblocks, tiles_dev);
     return check(hipGetLastError());
 }
 

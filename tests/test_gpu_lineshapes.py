@@ -1,0 +1,129 @@
+"""Lineshapes of every kind, spin, channel, orientation and normalisation flag against the
+oracle: the wave cache (all of it and single resonances), the grid integrals and the
+time-dependent waves.
+
+Tolerance: a wave is a product of a dozen correctly rounded factors, so engine and oracle
+agree to some 1e-15 relative except where the pair's threshold factor 1 - (ma + mb)^2 / s
+cancels, which multiplies the rounding by s / (s - (ma + mb)^2): below 1e3 on these samples."""
+import numpy as np
+import pytest
+
+import oracle as O
+from goofit_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+EQUAL = W.DALITZ_DECAY
+UNEQUAL = (1.96834, 0.13957, 0.49368, 0.13498, 1.5, 5.0)  # three different daughters
+
+SHAPES = {
+    # kind, mass, width, spin, pair, norm
+    "spins": [("RBW", 0.98, 0.06, s, p, True) for s in (0, 1, 2, 3) for p in (0, 1, 2)],
+    "unnormalised": [("RBW", 0.9, 0.1, s, p, False) for s in (0, 1, 2) for p in (0, 1, 2)]
+    + [("GS", 0.7758, 0.15, 1, 2, False)],
+    "gs": [("GS", 0.7758, 0.15, s, p, True) for s in (0, 1, 2) for p in (0, 1, 2)] + [("NONRES", 0, 0, 0, 0, True)],
+    "symmetrised": [("SYM", 0.9, 0.1, s, p, n) for s in (0, 1, 2) for p in (0, 2) for n in (True, False)],
+    "one": [("NONRES", 0, 0, 0, 0, True)],
+}
+
+
+def _model(shapes, decay, td=False):
+    m12, m13 = O.Obs("m12", 0.0, 3.5, 60), O.Obs("m13", 0.0, 3.5, 60)
+    num = O.Obs("evt", 0.0, 1e9, 1, event_number=True)
+    res = []
+    for k, (kind, mass, width, spin, pair, norm) in enumerate(shapes):
+        a = (O.Var(f"re{k}", 0.3 + 0.1 * k), O.Var(f"im{k}", 0.7 - 0.2 * k))
+        mw = (O.Var(f"m{k}", mass), O.Var(f"w{k}", width))
+        if kind == "NONRES":
+            res.append(O.NonRes(f"r{k}", *a))
+        elif kind == "GS":
+            res.append(O.GS(f"r{k}", *a, *mw, spin, pair, norm))
+        else:
+            res.append(O.RBW(f"r{k}", *a, *mw, spin, pair, norm, sym=kind == "SYM"))
+    eff = O.MultiPolynomial("eff", [m12, m13], [O.Var("one", 1.0)], [O.Var("z0", 0.0), O.Var("z1", 0.0)], 0)
+    if td:
+        t, s = O.Obs("t", -2.0, 20.0), O.Obs("s", 0.0, 0.8)
+        mix = [O.Var(n, v) for n, v in zip(("tau", "x", "y", "dx", "dy"), W.TD_MIX)]
+        return O.Tddp("td", t, s, m12, m13, num, decay, mix, res, O.TruthResolution(), eff), res
+    return O.Dalitz("dalitz", m12, m13, num, decay, res, eff), res
+
+
+def _events(n, decay, seed):
+    m12, m13 = W.dalitz_uniform(n, seed, decay)
+    rng = np.random.default_rng(seed)
+    out = rng.choice(n, n // 10, replace=False)  # a tenth outside the plot
+    m12[out], m13[out] = rng.uniform(0.0, 3.5, (2, out.size))
+    return m12, m13
+
+
+def _close(got, ref):
+    np.testing.assert_allclose(got, ref, rtol=1e-12, atol=1e-13 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("decay", [EQUAL, UNEQUAL], ids=["equal", "unequal"])
+@pytest.mark.parametrize("shapes", sorted(SHAPES))
+def test_waves_and_integrals(ctx, shapes, decay):
+    top, res = _model(SHAPES[shapes], decay)
+    for n in (1, 63, 257, 3001):  # ragged waves and workgroups
+        m12, m13 = _events(n, decay, 17 + n)
+        if n == 1:
+            m12, m13 = np.array([1.0]), np.array([1.0])
+        aos = np.stack([m12, m13, np.arange(n, dtype=np.float64)], 1)
+        M = O.Model(top, aos, decay=decay)
+        M.op.sync_params()
+        ctx.set_program(*M.op.prog.arrays())
+        ctx.set_decay(decay)
+        ctx.upload_columns([m12, m13, aos[:, 2]])
+        ctx.set_identity_column(2)
+        ctx.dalitz_set_data_size(0, n)
+        ctx.dalitz_cache(0)
+        funcs, eff = M.op.dalitz_layout(0)
+        inside = W.in_dalitz_np(m12, m13, decay)
+        for i, f in enumerate(funcs):
+            got = ctx.dalitz_get_cache(0, i, n)
+            assert np.all(got[~inside] == 0)
+            if inside.any():
+                _close(got, M.op.dalitz_wave(0, f, aos))
+    # one resonance at a time: the others keep their values
+    before = [ctx.dalitz_get_cache(0, i, n) for i in range(len(funcs))]
+    for i in {0, len(funcs) - 1}:
+        if SHAPES[shapes][i][0] == "NONRES":
+            continue
+        p = M.op.p.copy()
+        at = top.components[i].parameters_idx + 1
+        p[at] *= 1.01
+        ctx.update_params(p)
+        ctx.dalitz_cache(0, 1 << i)
+        for k in range(len(funcs)):
+            same = np.array_equal(ctx.dalitz_get_cache(0, k, n), before[k])
+            assert same == (k != i)
+        ctx.update_params(M.op.p)
+        ctx.dalitz_cache(0, 1 << i)
+        assert np.array_equal(ctx.dalitz_get_cache(0, i, n), before[i])
+    for nb in (1, 8, 61):  # fewer cells than a wave; none inside; ragged
+        grid6 = [0.0, 3.5, nb, 0.0, 3.5, nb]
+        ref = M.op.dalitz_integrals(0, grid6, eff)
+        got = ctx.dalitz_gram(0, grid6, eff, len(funcs))
+        np.testing.assert_allclose(got, ref, rtol=1e-11, atol=1e-12 * max(np.abs(ref).max(), 1e-300))
+
+
+@pytest.mark.parametrize("shapes", ["spins", "gs", "symmetrised"])
+def test_time_dependent_waves(ctx, shapes):
+    """The B waves: every lineshape at the reversed point (a pair below its threshold there)."""
+    n, decay = 1000, UNEQUAL
+    top, res = _model(SHAPES[shapes], decay, td=True)
+    m12, m13 = _events(n, decay, 5)
+    aos = np.stack([np.full(n, 0.5), np.full(n, 0.05), m12, m13, np.arange(n, dtype=np.float64)], 1)
+    M = O.Model(top, aos, decay=decay)
+    M.op.sync_params()
+    ctx.set_program(*M.op.prog.arrays())
+    ctx.set_decay(decay)
+    ctx.upload_columns(list(aos.T.copy()))
+    ctx.set_identity_column(4)
+    ctx.dalitz_set_data_size(0, n)
+    ctx.dalitz_cache(0)
+    funcs = M.op.tddp_layout(0)[0]
+    for i, f in enumerate(funcs):
+        a, b = M.op.tddp_wave(0, f, aos)
+        _close(ctx.dalitz_get_cache(0, i, n), a)
+        _close(ctx.dalitz_get_cache(0, len(funcs) + i, n), b)
