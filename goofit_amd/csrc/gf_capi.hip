@@ -128,6 +128,19 @@ struct gf_ctx {
     };
     std::map<int, NormPoints> norm_points;
 
+    // workspace of gf_dalitz_generate, set up by its first call (out: rows of the last calls
+    // with host output, at most 2^22 kept)
+    struct Generator {
+        uint32_t *bits = nullptr;  // the base of the allocation that holds the next four too
+        int *count     = nullptr;
+        double *bmax   = nullptr;
+        int64_t *boff  = nullptr;
+        GfGenState *state = nullptr;
+        GfGenPass *pass = nullptr, *d_pass = nullptr;  // host-mapped
+        double *out  = nullptr;
+        int64_t rows = 0;
+    } gen;
+
     // reduction scratch
     gfk::Partial *d_partials = nullptr;
     unsigned *d_counter      = nullptr;
@@ -1367,6 +1380,12 @@ void gf_ctx_destroy(gf_ctx *c) {
     for(auto &kv : c->norm_points)
         if(kv.second.buf)
             (void)hipFree(kv.second.buf);
+    if(c->gen.bits)
+        (void)hipFree(c->gen.bits);
+    if(c->gen.out)
+        (void)hipFree(c->gen.out);
+    if(c->gen.pass)
+        (void)hipHostFree(c->gen.pass);
     if(c->d_multi)
         (void)hipFree(c->d_multi);
     if(c->d_multi_partials)
@@ -3018,95 +3037,119 @@ gf_status gf_dalitz_generate(gf_ctx *ctx, int dalitz_func, int64_t n, uint64_t s
     if((st = flush_uploads(ctx)))
         return st;
     const int64_t B  = 1 << 22;  // candidates per pass
-    const int64_t nb = B / 256;
-    double *c = nullptr, *o = nullptr, *bmax = nullptr;
-    uint8_t *flag = nullptr;
-    int *bcount = nullptr;
-    int64_t *boff = nullptr;
+    const int nb     = (int)(B / GF_GEN_BLOCK);
+    // workspace of a call: the passes' bits, counts, largest values and offsets, the state,
+    // and what each pass of a round found (host-mapped)
+    constexpr int round = 32;  // passes queued between two looks at the results
+    gf_ctx::Generator &W = ctx->gen;
+    if(!W.bits) {
+        const size_t at[] = {(size_t)B / 8, (size_t)nb * 4, (size_t)nb * 8, (size_t)nb * 8, sizeof(GfGenState)};
+        uint8_t *q = nullptr;
+        if(hipMalloc((void **)&q, at[0] + at[1] + at[2] + at[3] + at[4]) != hipSuccess)
+            return fail(GF_ERR_NOMEM, "cannot allocate the generator buffers");
+        if(hipHostMalloc((void **)&W.pass, round * sizeof(GfGenPass), hipHostMallocMapped | hipHostMallocCoherent)
+               != hipSuccess
+           || hipHostGetDevicePointer((void **)&W.d_pass, W.pass, 0) != hipSuccess) {
+            if(W.pass)
+                (void)hipHostFree(W.pass);
+            W.pass = nullptr;
+            (void)hipFree(q);
+            return fail(GF_ERR_NOMEM, "cannot allocate the generator buffers");
+        }
+        W.bits  = (uint32_t *)q;
+        W.boff  = (int64_t *)(q + at[0]);
+        W.bmax  = (double *)(q + at[0] + at[2]);
+        W.state = (GfGenState *)(q + at[0] + at[2] + at[3]);
+        W.count = (int *)(q + at[0] + at[2] + at[3] + at[4]);
+    }
+    if(host_out && W.rows < n) {
+        GF_HIP(hipStreamSynchronize(ctx->stream));
+        if(W.out)
+            (void)hipFree(W.out);
+        W.out  = nullptr;
+        W.rows = 0;
+        if(hipMalloc((void **)&W.out, (size_t)n * 2 * 8) != hipSuccess) {
+            W.out = nullptr;
+            return fail(GF_ERR_NOMEM, "cannot allocate the generator buffers");
+        }
+        W.rows = n;
+    }
+    // the output rows are kept for the next call up to this size
     auto release = [&]() {
         (void)hipStreamSynchronize(ctx->stream);
-        void *p[] = {c, o, bmax, flag, bcount, boff};
-        for(void *q : p)
-            if(q)
-                (void)hipFree(q);
+        if(W.rows > ((int64_t)1 << 22)) {
+            (void)hipFree(W.out);
+            W.out  = nullptr;
+            W.rows = 0;
+        }
     };
-    if(hipMalloc((void **)&c, (size_t)B * 2 * 8) != hipSuccess || hipMalloc((void **)&flag, (size_t)B) != hipSuccess
-       || hipMalloc((void **)&bcount, (size_t)nb * 4) != hipSuccess
-       || hipMalloc((void **)&bmax, (size_t)nb * 8) != hipSuccess
-       || hipMalloc((void **)&boff, (size_t)nb * 8) != hipSuccess
-       || (host_out && hipMalloc((void **)&o, (size_t)n * 2 * 8) != hipSuccess)) {
-        release();
-        return fail(GF_ERR_NOMEM, "cannot allocate the generator buffers");
-    }
-    double *o12 = host_out ? o : m12, *o13 = host_out ? o + n : m13;
+    double *o12 = host_out ? W.out : m12, *o13 = host_out ? W.out + n : m13;
     GfProgArgs a = prog_args(ctx);
-    std::vector<int> hc(nb);
-    std::vector<double> hm(nb);
-    std::vector<int64_t> off(nb);
+    const GfGenBox gbox{box[0], box[1], box[2], box[3]};
     const uint64_t key = gfd::mix64(seed ^ 0x6A09E667F3BCC909ull);
     int64_t have = 0, base = 0;
-    auto pass = [&](double env) -> gf_status {
-        if(gfk::launch_dalitz_candidates(a, ctx->d_plan + slot, d->p_coup, eff_pc, eff_cval,
-                                         d->col_m12,
-                                         d->col_m13, box, key, base, B, env, c, c + B, flag, bcount, bmax,
-                                         ctx->stream))
-            return fail(GF_ERR_HIP, "candidate launch failed");
-        GF_HIP(hipMemcpyAsync(hc.data(), bcount, (size_t)nb * 4, hipMemcpyDeviceToHost, ctx->stream));
-        GF_HIP(hipMemcpyAsync(hm.data(), bmax, (size_t)nb * 8, hipMemcpyDeviceToHost, ctx->stream));
-        GF_HIP(hipStreamSynchronize(ctx->stream));
-        return GF_OK;
+    hipStream_t s = ctx->stream;
+    auto pass = [&](bool envelope, int64_t at, int64_t limit, int k) {
+        return gfk::launch_dalitz_candidates(a, ctx->d_plan + slot, d->p_coup, eff_pc, eff_cval, d->col_m12, d->col_m13,
+                                             gbox, key, at, nb, W.state, limit, W.bits, W.count, W.bmax, s)
+                   || gfk::launch_gen_scan(envelope, 0.0, W.count, W.bmax, nb, limit, W.boff, W.state, W.d_pass + k, s)
+                   || (!envelope
+                       && gfk::launch_compact(W.bits, gbox, key, at, nb, W.boff, limit, o12, o13, s));
     };
-    if(!(fmax > 0.0)) {
-        // envelope: 1.25 x the largest value over one pass of candidates
-        st = pass(INFINITY);
-        if(st) {
-            release();
-            return st;
-        }
-        double mx = 0.0;
-        for(double v : hm)
-            mx = std::max(mx, v);
-        if(!(mx > 0.0)) {
-            release();
-            return fail(GF_ERR_INVALID, "|A|^2 * eff is zero on %lld candidates", (long long)B);
-        }
-        fmax = 1.25 * mx;
-        base += B;
+    const bool find = !(fmax > 0.0);
+    if(gfk::launch_line_plan(a, ctx->d_plan + slot, s)
+       || gfk::launch_gen_scan(false, find ? INFINITY : fmax, nullptr, nullptr, 0, 0, nullptr, W.state, nullptr, s)
+       || (find && pass(true, 0, 1, round - 1))) {
+        release();
+        return fail(GF_ERR_HIP, "candidate launch failed");
     }
-    while(have < n) {
-        if((st = pass(fmax))) {
-            release();
-            return st;
-        }
-        double mx    = 0.0;
-        int64_t acc  = 0;
-        for(int64_t b = 0; b < nb; b++) {
-            off[b] = have + acc;
-            acc += hc[b];
-            mx = std::max(mx, hm[b]);
-        }
-        if(mx > fmax) {
-            release();
-            return fail(GF_ERR_INVALID, "envelope %g below the value %g found: raise fmax", fmax, mx);
-        }
-        if(acc > 0) {
-            if(hipMemcpyAsync(boff, off.data(), (size_t)nb * 8, hipMemcpyHostToDevice, ctx->stream) != hipSuccess
-               || gfk::launch_compact(c, c + B, flag, B, boff, n, o12, o13, ctx->stream)) {
-                release();
-                return fail(GF_ERR_HIP, "compaction failed");
-            }
-        }
-        have += acc;
+    if(find)  // envelope: 1.25 x the largest value over one pass of candidates
         base += B;
-        if(base > (int64_t)1 << 40) {
+    // Rounds of passes: one at first, then as many as the acceptance so far asks for (a pass
+    // queued beyond the last one needed finds the rows complete and does nothing).
+    int64_t done = 0;
+    int k        = 1;
+    bool first   = true;
+    while(have < n) {
+        for(int j = 0; j < k; j++)
+            if(pass(false, base + j * B, n, j)) {
+                release();
+                return fail(GF_ERR_HIP, "candidate launch failed");
+            }
+        if(hipStreamSynchronize(s) != hipSuccess) {
+            release();
+            return fail(GF_ERR_HIP, "generation failed");
+        }
+        ctx->stage_in_flight = false;
+        if(first && find) {
+            const double mx = W.pass[round - 1].mx;
+            if(!(mx > 0.0)) {
+                release();
+                return fail(GF_ERR_INVALID, "|A|^2 * eff is zero on %lld candidates", (long long)B);
+            }
+            fmax = 1.25 * mx;
+        }
+        first = false;
+        for(int j = 0; j < k && have < n; j++) {
+            if(W.pass[j].mx > fmax) {
+                release();
+                return fail(GF_ERR_INVALID, "envelope %g below the value %g found: raise fmax", fmax, W.pass[j].mx);
+            }
+            have += W.pass[j].count;
+            base += B;
+            done++;
+        }
+        if(have < n && base > (int64_t)1 << 40) {
             release();
             return fail(GF_ERR_INVALID, "acceptance too low: %lld of %lld events after %lld candidates",
                         (long long)have, (long long)n, (long long)base);
         }
+        const double more = have > 0 ? (double)(n - have) / (double)have * (double)done : (double)(2 * k);
+        k                 = (int)std::min<double>(round - 1, std::max(1.0, std::ceil(more)));
     }
     if(host_out) {
-        if(hipMemcpyAsync(m12, o12, (size_t)n * 8, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess
-           || hipMemcpyAsync(m13, o13, (size_t)n * 8, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess) {
+        if(hipMemcpyAsync(m12, o12, (size_t)n * 8, hipMemcpyDeviceToHost, s) != hipSuccess
+           || hipMemcpyAsync(m13, o13, (size_t)n * 8, hipMemcpyDeviceToHost, s) != hipSuccess) {
             release();
             return fail(GF_ERR_HIP, "copy of the events failed");
         }

@@ -211,6 +211,21 @@ struct GfNormOp {
     double c0, c1;
 };
 
+// Accept-reject generation from an Amp3Body: candidates per workgroup, the box, the state a
+// call keeps on the device (envelope, rows written) and what a pass found.
+#define GF_GEN_BLOCK 2048
+struct GfGenBox {
+    double l12, u12, l13, u13;
+};
+struct GfGenState {
+    double fmax;
+    int64_t have;
+};
+struct GfGenPass {
+    int64_t count;
+    double mx;
+};
+
 // Host-side launchers (gf_kernels.hip, gf_coherent.hip, gf_lines.hip).
 namespace gfk {
 struct Partial {
@@ -274,16 +289,20 @@ int launch_batch_points(const GfProgArgs &a, int nres, const GfBatchWork *work, 
                         const double *stage, int np, int nn, const int *tbl, bool fast, bool const_eff,
                         bool zero_outside, int metric, int mx_min, Partial *partials, const int *first, int ntoys,
                         double *result, uint32_t *counter, uint32_t *stamp, void *stream);
-// Accept-reject generation: candidates (uniform in box) with accept flags, and
-// the ordered compaction of the accepted ones.
+// Accept-reject generation in passes of nblocks x GF_GEN_BLOCK candidates of a counter-based
+// stream: candidates (accepted ones as bits, per-block counts and largest values), the scan
+// of the counts, the ordered write of the accepted.  plan: filled in by launch_line_plan.
 // eff_pc >= 0: efficiency subprogram; -1: efficiency 1; -2: the constant eff_const.
-int launch_dalitz_candidates(const GfProgArgs &a, GfLinePlan *plan, int p_coup, int eff_pc,
-                             double eff_const, int id12, int id13, const double box[4], uint64_t key, int64_t base,
-                             int64_t nc, double fmax, double *c12, double *c13, uint8_t *flag, int *bcount,
-                             double *bmax, void *stream);
-int launch_compact(const double *c12, const double *c13, const uint8_t *flag, int64_t nc, const int64_t *boff,
-                   int64_t limit, double *o12, double *o13, void *stream);
-// plan (here and below): the lineshapes' structure; its numbers are filled in first.
+int launch_line_plan(const GfProgArgs &a, GfLinePlan *plan, void *stream);
+int launch_dalitz_candidates(const GfProgArgs &a, const GfLinePlan *plan, int p_coup, int eff_pc, double eff_const,
+                             int id12, int id13, const GfGenBox &box, uint64_t key, int64_t base, int nblocks,
+                             const GfGenState *st, int64_t limit, uint32_t *bits, int *bcount, double *bmax,
+                             void *stream);
+int launch_gen_scan(bool envelope, double value, const int *bcount, const double *bmax, int nblocks, int64_t limit,
+                    int64_t *boff, GfGenState *st, GfGenPass *out, void *stream);
+int launch_compact(const uint32_t *bits, const GfGenBox &box, uint64_t key, int64_t base, int nblocks,
+                   const int64_t *boff, int64_t limit, double *o12, double *o13, void *stream);
+// plan (here and in launch_gram): the lineshapes' structure; its numbers are filled in first.
 int launch_dalitz_cache(const GfProgArgs &a, int slot, int64_t offset, int64_t n, uint32_t mask, GfLinePlan *plan,
                         int nblocks, void *stream);
 // mode 0: grid cells (grid6 host array); 1: points (m12, m13, w device arrays); 2: data cache of `slot`.

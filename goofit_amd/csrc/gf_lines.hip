@@ -111,35 +111,71 @@ __global__ __launch_bounds__(256) void k_dalitz_cache(GfProgArgs A, int slot, in
 
 // ------------------------------------------------------------- event generation
 
-// Candidates for accept-reject generation from an Amp3Body: point i of the
-// counter-based stream is uniform in the box; its value is
-// |sum_r c_r B_r(m12, m13)|^2 * eff (0 outside the Dalitz plot, as
-// device_DalitzPlot, Amp3Body.cu:60-122, with lineshapes computed directly);
-// accepted when u_i * fmax < value.  Per block: accepted count and the largest
-// value (to check the envelope).
+// Accept-reject generation from an Amp3Body: candidate i of the counter-based stream is
+// uniform in the box; its value is |sum_r c_r B_r(m12, m13)|^2 * eff (0 outside the Dalitz
+// plot, as device_DalitzPlot, Amp3Body.cu:60-122, with lineshapes computed directly);
+// accepted when u_i * fmax < value.
+
+__device__ __forceinline__ void gen_point(const GfGenBox &B, uint64_t key, uint64_t i, double &m12, double &m13) {
+    m12 = B.l12 + gfd::unif01(key, 2 * i) * (B.u12 - B.l12);
+    m13 = B.l13 + gfd::unif01(key, 2 * i + 1) * (B.u13 - B.l13);
+}
+
+// One workgroup takes GF_GEN_BLOCK candidates: all its lanes draw and test them against
+// the plot, the points inside (about a third of a box around it) are gathered in LDS, and
+// only those are evaluated, on full waves -- the lineshapes are nine tenths of the work.
+// Out: the accepted candidates as bits, their number and the largest value (to check the
+// envelope).  Nothing is done once st->have has reached limit.  A pass of 2^22 candidates,
+// 16 shapes: 208 us with every candidate evaluated in its own lane.
 template <bool GEN_EFF>
 __global__ __launch_bounds__(256) void k_dalitz_candidates(GfProgArgs A, const GfLinePlan *__restrict__ plan,
                                                            int p_coup, int eff_pc, double eff_const, int id12,
-                                                           int id13, double l12,
-                                                           double u12, double l13, double u13, uint64_t key,
-                                                           int64_t base, int64_t nc, double fmax,
-                                                           double *__restrict__ c12, double *__restrict__ c13,
-                                                           uint8_t *__restrict__ flag, int *__restrict__ bcount,
+                                                           int id13, GfGenBox B, uint64_t key, int64_t base,
+                                                           const GfGenState *__restrict__ st, int64_t limit,
+                                                           uint32_t *__restrict__ bits, int *__restrict__ bcount,
                                                            double *__restrict__ bmax) {
-    __shared__ int scount[4];
+    __shared__ double x12[GF_GEN_BLOCK], x13[GF_GEN_BLOCK];
+    __shared__ uint16_t at[GF_GEN_BLOCK];
+    __shared__ uint32_t word[GF_GEN_BLOCK / 32];
+    __shared__ int inside_n, scount[4];
     __shared__ double smax[4];
-    const int64_t i   = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid  = i < nc;
-    const GfDecay D   = A.decay;
-    const uint64_t ct = (uint64_t)(base + (valid ? i : 0));
-    const double m12  = l12 + gfd::unif01(key, 2 * ct) * (u12 - l12);
-    const double m13  = l13 + gfd::unif01(key, 2 * ct + 1) * (u13 - l13);
-    double value      = 0.0;
-    if(valid && gfd::in_dalitz(m12, m13, D.motherMass, D.daug1Mass, D.daug2Mass, D.daug3Mass)) {
+    if(st->have >= limit)
+        return;  // uniform over the launch
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const GfDecay D    = A.decay;
+    const double fmax  = st->fmax;
+    const int64_t base0 = base + (int64_t)blockIdx.x * GF_GEN_BLOCK;
+    if(t == 0)
+        inside_n = 0;
+    if(t < GF_GEN_BLOCK / 32)
+        word[t] = 0;
+    __syncthreads();
+    for(int j = t; j < GF_GEN_BLOCK; j += 256) {
+        double m12, m13;
+        gen_point(B, key, (uint64_t)(base0 + j), m12, m13);
+        const bool in = gfd::in_dalitz(m12, m13, D.motherMass, D.daug1Mass, D.daug2Mass, D.daug3Mass);
+        const unsigned long long ball = __ballot(in);
+        int first = 0;
+        if(lane == 0)
+            first = atomicAdd(&inside_n, __popcll(ball));
+        first = __shfl(first, 0, 64);
+        if(in) {  // in any order: what follows does not depend on it
+            const int k = first + __popcll(ball & ((1ull << lane) - 1ull));
+            x12[k] = m12;
+            x13[k] = m13;
+            at[k]  = (uint16_t)j;
+        }
+    }
+    __syncthreads();
+    const int n = inside_n;
+    const GF_CONST double *__restrict__ P = gfd::as_const(A.params) + p_coup;
+    double vm   = 0.0;
+    int count   = 0;
+    for(int k = t; k < n; k += 256) {
+        const double m12 = x12[k], m13 = x13[k];
         const double m23 = D.motherMass * D.motherMass + D.daug1Mass * D.daug1Mass + D.daug2Mass * D.daug2Mass
                            + D.daug3Mass * D.daug3Mass - m12 - m13;
         double re = 0.0, im = 0.0;
-        const GF_CONST double *__restrict__ P = gfd::as_const(A.params) + p_coup;
         gfd::line_waves(plan, m12, m13, m23, ~0u, [&](int r, int, int, double2 b) {
             const double ar = P[2 * r], ai = P[2 * r + 1];
             re = fma(ar, b.x, fma(-ai, b.y, re));
@@ -159,59 +195,131 @@ __global__ __launch_bounds__(256) void k_dalitz_candidates(GfProgArgs A, const G
             run<1>(A, A.params, A.norms, eff_pc, ev, r0, v0, T);
             eff = T[0];
         }
-        value = (re * re + im * im) * eff;
+        const double value = (re * re + im * im) * eff;
+        vm                 = ::fmax(vm, value);
+        const int j        = at[k];
+        if(gfd::unif01(key ^ 0xD1B54A32D192ED03ull, (uint64_t)(base0 + j)) * fmax < value) {
+            atomicOr(&word[j >> 5], 1u << (j & 31));
+            ++count;
+        }
     }
-    const bool acc = valid && gfd::unif01(key ^ 0xD1B54A32D192ED03ull, ct) * fmax < value;
-    if(valid) {
-        c12[i]  = m12;
-        c13[i]  = m13;
-        flag[i] = acc ? 1 : 0;
-    }
-    // block totals: count of accepted, largest value
-    const unsigned long long ball = __ballot(acc);
-    double vm = value;
-    for(int off = 32; off > 0; off >>= 1)
+    for(int off = 32; off > 0; off >>= 1) {
         vm = ::fmax(vm, __shfl_xor(vm, off, 64));
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        count += __shfl_xor(count, off, 64);
+    }
     if(lane == 0) {
-        scount[wave] = __popcll(ball);
+        scount[wave] = count;
         smax[wave]   = vm;
     }
     __syncthreads();
-    if(threadIdx.x == 0) {
-        int c    = 0;
-        double m = 0.0;
-        for(int w = 0; w < 4; ++w) {
-            c += scount[w];
-            m = ::fmax(m, smax[w]);
+    if(t < GF_GEN_BLOCK / 32)
+        bits[(int64_t)blockIdx.x * (GF_GEN_BLOCK / 32) + t] = word[t];
+    if(t == 0) {
+        for(int w = 1; w < 4; ++w) {
+            count += scount[w];
+            vm = ::fmax(vm, smax[w]);
         }
-        bcount[blockIdx.x] = c;
-        bmax[blockIdx.x]   = m;
+        bcount[blockIdx.x] = count;
+        bmax[blockIdx.x]   = vm;
     }
 }
 
-// Write the accepted candidates in order: block b's go to boff[b] + their rank
-// in the block (waves in order, lanes in order); rows >= limit are dropped.
-__global__ __launch_bounds__(256) void k_compact(const double *__restrict__ c12, const double *__restrict__ c13,
-                                                 const uint8_t *__restrict__ flag, int64_t nc,
-                                                 const int64_t *__restrict__ boff, int64_t limit,
-                                                 double *__restrict__ o12, double *__restrict__ o13) {
-    __shared__ int wcount[4];
-    const int64_t i  = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool acc   = i < nc && flag[i];
-    const unsigned long long ball = __ballot(acc);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// One workgroup after a pass: its largest value and accepted count into *out (host-mapped),
+// and the state of the next one.  GF_GEN_ENVELOPE: the pass sets the envelope, 1.25 x its
+// largest value; otherwise boff[b] = the row of block b's first accepted candidate.
+// nblk 0: no pass, the envelope is `value`.
+__global__ __launch_bounds__(1024) void k_gen_scan(int envelope, double value, const int *__restrict__ bcount,
+                                                   const double *__restrict__ bmax, int nblk, int64_t limit,
+                                                   int64_t *__restrict__ boff, GfGenState *st, GfGenPass *out) {
+    __shared__ int64_t wsum[16];
+    __shared__ double wmax[16];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    if(nblk == 0) {
+        if(t == 0) {
+            st->fmax = value;
+            st->have = 0;
+        }
+        return;
+    }
+    const int64_t have = st->have;
+    const int per = (nblk + 1023) / 1024, b0 = t * per, b1 = min(nblk, b0 + per);
+    if(have >= limit) {  // the pass did nothing and has no rows to write
+        for(int b = b0; b < b1 && !envelope; ++b)
+            boff[b] = limit;
+        if(t == 0)
+            out->count = 0, out->mx = 0.0;
+        return;
+    }
+    int64_t sum = 0;
+    double m    = 0.0;
+    for(int b = b0; b < b1; ++b) {
+        sum += bcount[b];
+        m = ::fmax(m, bmax[b]);
+    }
+    int64_t incl = sum;  // inclusive scan over the wave
+    for(int off = 1; off < 64; off <<= 1) {
+        const int64_t v = __shfl_up(incl, off, 64);
+        if(lane >= off)
+            incl += v;
+    }
+    for(int off = 32; off > 0; off >>= 1)
+        m = ::fmax(m, __shfl_xor(m, off, 64));
+    if(lane == 63)
+        wsum[wave] = incl;
     if(lane == 0)
-        wcount[wave] = __popcll(ball);
+        wmax[wave] = m;
     __syncthreads();
-    int before = 0;
+    int64_t before = have, total = 0;
+    for(int w = 0; w < 16; ++w) {
+        if(w < wave)
+            before += wsum[w];
+        total += wsum[w];
+        m = ::fmax(m, wmax[w]);
+    }
+    int64_t row = before + incl - sum;
+    for(int b = b0; b < b1; ++b) {
+        boff[b] = row;
+        row += bcount[b];
+    }
+    if(t == 0) {
+        out->count = total;
+        out->mx    = m;
+        if(envelope)
+            st->fmax = 1.25 * m;
+        else
+            st->have = have + total;
+    }
+}
+
+// Write a pass's accepted candidates in the stream's order: block b's to boff[b] + their
+// rank in the block; rows >= limit are dropped.  The points are drawn again from their
+// counters (a few in a hundred candidates) instead of kept for every candidate.
+__global__ __launch_bounds__(256) void k_compact(const uint32_t *__restrict__ bits, GfGenBox B, uint64_t key,
+                                                 int64_t base, const int64_t *__restrict__ boff, int64_t limit,
+                                                 double *__restrict__ o12, double *__restrict__ o13) {
+    static_assert(GF_GEN_BLOCK == 256 * 8, "a byte of the mask per lane");
+    __shared__ int wcount[4];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    uint32_t m   = (bits[(int64_t)blockIdx.x * (GF_GEN_BLOCK / 32) + (t >> 2)] >> (8 * (t & 3))) & 0xFFu;
+    const int c  = __popc(m);
+    int incl     = c;
+    for(int off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(incl, off, 64);
+        if(lane >= off)
+            incl += v;
+    }
+    if(lane == 63)
+        wcount[wave] = incl;
+    __syncthreads();
+    int64_t dst = boff[blockIdx.x] + incl - c;
     for(int w = 0; w < wave; ++w)
-        before += wcount[w];
-    const unsigned long long lower = lane ? (ball & ((1ull << lane) - 1ull)) : 0ull;
-    const int64_t dst = boff[blockIdx.x] + before + __popcll(lower);
-    if(acc && dst < limit) {
-        o12[dst] = c12[i];
-        o13[dst] = c13[i];
+        dst += wcount[w];
+    const int64_t i0 = base + (int64_t)blockIdx.x * GF_GEN_BLOCK + 8 * t;
+    for(; m && dst < limit; m &= m - 1, ++dst) {
+        double m12, m13;
+        gen_point(B, key, (uint64_t)(i0 + __ffs(m) - 1), m12, m13);
+        o12[dst] = m12;
+        o13[dst] = m13;
     }
 }
 
@@ -409,30 +517,34 @@ static int fill_plan(const GfProgArgs &a, GfLinePlan *plan, hipStream_t s) {
 }
 
 
-int launch_dalitz_candidates(const GfProgArgs &a, GfLinePlan *plan, int p_coup, int eff_pc,
-                             double eff_const, int id12, int id13, const double box[4], uint64_t key, int64_t base,
-                             int64_t nc, double fmax, double *c12, double *c13, uint8_t *flag, int *bcount,
-                             double *bmax, void *stream) {
-    const int nb = (int)((nc + 255) / 256);
-    int rc       = fill_plan(a, plan, (hipStream_t)stream);
-    if(rc)
-        return rc;
+int launch_line_plan(const GfProgArgs &a, GfLinePlan *plan, void *stream) {
+    return fill_plan(a, plan, (hipStream_t)stream);
+}
+
+int launch_dalitz_candidates(const GfProgArgs &a, const GfLinePlan *plan, int p_coup, int eff_pc, double eff_const,
+                             int id12, int id13, const GfGenBox &box, uint64_t key, int64_t base, int nblocks,
+                             const GfGenState *st, int64_t limit, uint32_t *bits, int *bcount, double *bmax,
+                             void *stream) {
     if(eff_pc >= 0)
-        hipLaunchKernelGGL(k_dalitz_candidates<true>, dim3(nb), dim3(256), 0, (hipStream_t)stream, a, plan,
-                           p_coup, eff_pc, eff_const, id12, id13, box[0], box[1], box[2], box[3], key, base, nc, fmax,
-                           c12, c13, flag, bcount, bmax);
+        hipLaunchKernelGGL(k_dalitz_candidates<true>, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, a, plan,
+                           p_coup, eff_pc, eff_const, id12, id13, box, key, base, st, limit, bits, bcount, bmax);
     else
-        hipLaunchKernelGGL(k_dalitz_candidates<false>, dim3(nb), dim3(256), 0, (hipStream_t)stream, a, plan,
-                           p_coup, eff_pc, eff_const, id12, id13, box[0], box[1], box[2], box[3], key, base, nc, fmax,
-                           c12, c13, flag, bcount, bmax);
+        hipLaunchKernelGGL(k_dalitz_candidates<false>, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, a, plan,
+                           p_coup, eff_pc, eff_const, id12, id13, box, key, base, st, limit, bits, bcount, bmax);
     return check(hipGetLastError());
 }
 
-int launch_compact(const double *c12, const double *c13, const uint8_t *flag, int64_t nc, const int64_t *boff,
-                   int64_t limit, double *o12, double *o13, void *stream) {
-    const int nb = (int)((nc + 255) / 256);
-    hipLaunchKernelGGL(k_compact, dim3(nb), dim3(256), 0, (hipStream_t)stream, c12, c13, flag, nc, boff, limit, o12,
-                       o13);
+int launch_gen_scan(bool envelope, double value, const int *bcount, const double *bmax, int nblocks, int64_t limit,
+                    int64_t *boff, GfGenState *st, GfGenPass *out, void *stream) {
+    hipLaunchKernelGGL(k_gen_scan, dim3(1), dim3(1024), 0, (hipStream_t)stream, envelope ? 1 : 0, value, bcount, bmax,
+                       nblocks, limit, boff, st, out);
+    return check(hipGetLastError());
+}
+
+int launch_compact(const uint32_t *bits, const GfGenBox &box, uint64_t key, int64_t base, int nblocks,
+                   const int64_t *boff, int64_t limit, double *o12, double *o13, void *stream) {
+    hipLaunchKernelGGL(k_compact, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, bits, box, key, base, boff, limit,
+                       o12, o13);
     return check(hipGetLastError());
 }
 

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from goofit_amd import capi
 from goofit_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -127,3 +128,65 @@ def test_time_dependent_waves(ctx, shapes):
         a, b = M.op.tddp_wave(0, f, aos)
         _close(ctx.dalitz_get_cache(0, i, n), a)
         _close(ctx.dalitz_get_cache(0, len(funcs) + i, n), b)
+
+
+def _mix64(z):
+    """The finaliser of the counter-based stream (splitmix64)."""
+    z = z + np.uint64(0x9E3779B97F4A7C15)
+    z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+    z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+    return z ^ (z >> np.uint64(31))
+
+
+def _unif(key, counter):
+    return (_mix64(key ^ _mix64(counter)) >> np.uint64(11)) * 2.0 ** -53
+
+
+def test_generated_events_are_the_stream(ctx):
+    """The accepted candidates of the documented stream, in its order, over one pass of 2^22
+    and into the second; a few events, a whole pass, one more than a pass; a box that cuts
+    the plot and one that misses it."""
+    decay, passes, fmax, seed = EQUAL, 2, 4000.0, 23
+    shapes = [("RBW", 0.7758, 0.15, 1, 0, True), ("NONRES", 0, 0, 0, 0, True), ("GS", 0.7758, 0.15, 1, 2, True),
+              ("SYM", 0.98, 0.06, 0, 1, True)]
+    top, res = _model(shapes, decay)
+    box = [0.2, 2.6, 0.1, 3.0]
+    with np.errstate(over="ignore"):
+        key = _mix64(np.array([seed], np.uint64) ^ np.uint64(0x6A09E667F3BCC909))[0]
+        i = np.arange(passes << 22, dtype=np.uint64)
+        m12 = box[0] + _unif(key, np.uint64(2) * i) * (box[1] - box[0])
+        m13 = box[2] + _unif(key, np.uint64(2) * i + np.uint64(1)) * (box[3] - box[2])
+        u = _unif(key ^ np.uint64(0xD1B54A32D192ED03), i)
+    inside = np.nonzero(W.in_dalitz_np(m12, m13, decay))[0]
+    M = O.Model(top, np.zeros((1, 3)), decay=decay)
+    M.op.sync_params()
+    ctx.set_program(*M.op.prog.arrays())
+    ctx.set_decay(decay)
+    ctx.upload_columns([m12[inside], m13[inside], np.arange(inside.size, dtype=np.float64)])
+    ctx.set_identity_column(2)
+    ctx.dalitz_set_data_size(0, inside.size)
+    ctx.dalitz_cache(0)
+    value = ctx.eval_metric("EVAL")
+    assert value.max() < fmax
+    keep = inside[u[inside] * fmax < value]
+    first = int(np.sum(keep < 1 << 22))
+    assert 1000 < first < keep.size
+    for n in (1, 777, first, first + 1, keep.size):
+        a, b, tried, top_value = ctx.dalitz_generate(0, n, seed, box, fmax)
+        assert np.array_equal(a, m12[keep[:n]]) and np.array_equal(b, m13[keep[:n]])
+        assert tried == (1 if n <= first else 2) << 22 and top_value == fmax
+    # the envelope found from the first pass, whose candidates are then not used again
+    n = keep.size - first
+    a, b, tried, top_value = ctx.dalitz_generate(0, n // 2, seed, box)
+    top_seen = value[inside < 1 << 22].max()
+    np.testing.assert_allclose(top_value, 1.25 * top_seen, rtol=1e-13)
+    later = inside[(inside >= 1 << 22) & (u[inside] * top_value < value)]
+    k = min(later.size, n // 2)
+    assert np.array_equal(a[:k], m12[later[:k]]) and np.array_equal(b[:k], m13[later[:k]])
+    # an envelope below the values, and a box without the plot
+    with pytest.raises(capi.GooFitError, match="raise fmax"):
+        ctx.dalitz_generate(0, 10, seed, box, 0.5 * top_seen)
+    with pytest.raises(capi.GooFitError, match="is zero"):
+        ctx.dalitz_generate(0, 10, seed, [2.95, 3.0, 2.95, 3.0])
+    a2, b2, _, _ = ctx.dalitz_generate(0, 777, seed, box, fmax)
+    assert np.array_equal(a2, m12[keep[:777]]) and np.array_equal(b2, m13[keep[:777]])
