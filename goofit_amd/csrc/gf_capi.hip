@@ -697,7 +697,7 @@ gf_status scan_dalitz(gf_ctx *ctx) {
 // at (m12, m13) and again at (m13, m12), as the cache of a time-dependent node holds them.
 void line_plan(const gf_ctx *ctx, const GfResDesc *res, int n, bool both, GfLinePlan &plan) {
     struct Entry {
-        std::array<int, 4> key;  // swap, pair, spin, norm
+        std::array<int, 5> key;  // swap, pair, spin, norm, Gounaris-Sakurai
         GfLineTerm term;
     };
     std::vector<Entry> all;
@@ -705,14 +705,15 @@ void line_plan(const gf_ctx *ctx, const GfResDesc *res, int n, bool both, GfLine
         for(int i = 0; i < n; i++) {
             const GfResDesc &r = res[i];
             Entry e{};
-            e.key       = {both ? sw : (r.swap != 0), -1, 0, 1};
+            e.key       = {both ? sw : (r.swap != 0), -1, 0, 1, r.kind == GR_GS};
             e.term.res  = i;
             e.term.p    = r.p;
             e.term.kind = r.kind == GR_RBW_SYM ? GR_RBW : r.kind;
             if(r.kind != GR_NONRES) {
                 const unsigned spin = (unsigned)ctx->consts[r.c], cyc = (unsigned)ctx->consts[r.c + 1];
                 // without spin there are no barrier factors: the flag makes no difference
-                e.key = {e.key[0], (int)std::min(cyc, 3u), (int)spin, (spin == 0 || ctx->consts[r.c + 2] != 0.0) ? 1 : 0};
+                e.key = {e.key[0], (int)std::min(cyc, 3u), (int)spin, (spin == 0 || ctx->consts[r.c + 2] != 0.0) ? 1 : 0,
+                         e.key[4]};
                 if(r.kind == GR_RBW_SYM) {  // the second half, one channel on (RBW.cu:80-81)
                     Entry h  = e;
                     h.key[1] = (int)((cyc + 1) % 3);
@@ -733,6 +734,7 @@ void line_plan(const gf_ctx *ctx, const GfResDesc *res, int n, bool both, GfLine
             c.pair         = key[1];
             c.spin         = key[2];
             c.norm         = key[3];
+            c.gs           = key[4];
         }
         GfLineClass &c = plan.cls[plan.nclass - 1];
         c.count++;
@@ -2120,8 +2122,8 @@ gf_status gf_dalitz_cache(gf_ctx *ctx, int dalitz_func, uint64_t res_mask) {
     if(nb > (int64_t)ctx->cu_count * 8)
         nb = (int64_t)ctx->cu_count * 8;
     GfProgArgs a = prog_args(ctx);
-    int rc = gfk::launch_dalitz_cache(a, slot, wc.offset, wc.n, mask, ctx->d_plan + slot,
-                                      (int)(nb < 1 ? 1 : nb), ctx->stream);
+    int rc = gfk::launch_dalitz_cache(a, slot, wc.offset, wc.n, mask, mask + 1 == 1u << d->nres,
+                                      ctx->d_plan + slot, (int)(nb < 1 ? 1 : nb), ctx->stream);
     if(rc)
         return fail(GF_ERR_HIP, "cache launch failed (%d)", rc);
     GF_HIP(hipStreamSynchronize(ctx->stream));
@@ -2437,7 +2439,7 @@ gf_status gf_time_dalitz_cache(gf_ctx *ctx, int dalitz_func, int reps, double *m
     uint32_t mask = d->nres >= 32 ? 0xffffffffu : ((1u << d->nres) - 1u);
     GF_HIP(hipEventRecord(ctx->ev0, ctx->stream));
     for(int r = 0; r < reps; r++) {
-        int rc = gfk::launch_dalitz_cache(a, slot, wc.offset, wc.n, mask, ctx->d_plan + slot,
+        int rc = gfk::launch_dalitz_cache(a, slot, wc.offset, wc.n, mask, true, ctx->d_plan + slot,
                                           (int)(nb < 1 ? 1 : nb), ctx->stream);
         if(rc)
             return fail(GF_ERR_HIP, "cache launch failed (%d)", rc);

@@ -294,26 +294,48 @@ __device__ __forceinline__ double d_fun(double s, double daug2Mass, double daug3
 // At one point: s the pair's mass squared, r = 1 / s, u = q / sqrt(s), q2 = q^2; bf and sf
 // as above.
 
+// 1 / sqrt(x) and 1 / x of a normal x > 0, to about one unit in the last place: the
+// hardware's estimate and two Newton steps.  (The barrier denominators are at least 1 and
+// the propagators' are squares of masses: nothing here comes near the ends of the range
+// for which the library's forms scale their operands.)
+__device__ __forceinline__ double rsqrt_n(double x) {
+    double y = __builtin_amdgcn_rsq(x);
+    y        = fma(y, fma(-0.5 * x * y, y, 0.5), y);
+    return fma(y, fma(-0.5 * x * y, y, 0.5), y);
+}
+__device__ __forceinline__ double rcp_n(double x) {
+    double y = __builtin_amdgcn_rcp(x);
+    y        = fma(y, fma(-x, y, 1.0), y);
+    return fma(y, fma(-x, y, 1.0), y);
+}
+
+// 1 - t / s with the thresholds' rule (below zero: 1).  r = 1 / s; next to the threshold
+// the quotient decides as the reference's division does.
+__device__ __forceinline__ double threshold_factor(double t, double s, double r) {
+    const double d = s - t;
+    double k       = d * r;
+    if(fabs(d) < 1e-14 * s)
+        k = 1 - t / s;
+    return k >= 0 ? k : 1;
+}
+
 // The pair's part: s, 1 / s and the momentum (two_body_cm_mom).
-__device__ __forceinline__ void line_pair(const GF_CONST GfLineClass &c, double m12, double m13, double m23,
-                                          double &s, double &r, double &u, double &q2) {
-    s         = 0 == c.pair ? m12 : (1 == c.pair ? m13 : m23);
-    double k1 = 1 - c.sum2 / s;
-    k1        = k1 >= 0 ? k1 : 1;
-    if(c.dif2 != 0) {  // uniform: equal daughter masses give exactly 1
-        const double k2 = 1 - c.dif2 / s;
-        k1 *= k2 >= 0 ? k2 : 1;
-    }
-    r  = 1.0 / s;
-    u  = 0.5 * sqrt(k1);
-    q2 = 0.25 * s * k1;
+__device__ __forceinline__ void line_pair(const GfLineClass &c, double m12, double m13, double m23, double &s,
+                                          double &r, double &u, double &q2) {
+    s        = 0 == c.pair ? m12 : (1 == c.pair ? m13 : m23);
+    r        = 1.0 / s;
+    double k = threshold_factor(c.sum2, s, r);
+    if(c.dif2 != 0)  // uniform: equal daughter masses give exactly 1
+        k *= threshold_factor(c.dif2, s, r);
+    u  = 0.5 * sqrt(k);
+    q2 = 0.25 * s * k;
 }
 
 // The class's part: barrier and spin factors (dampingFactorSquareNorm, dampingFactorSquare
 // and spinFactor, Resonance.cu:77-155).
-__device__ __forceinline__ void line_class(const GF_CONST GfLinePlan *__restrict__ plan,
-                                           const GF_CONST GfLineClass &c, double m12, double m13, double m23, double s,
-                                           double r, double u, double q2, double &bf, double &sf) {
+__device__ __forceinline__ void line_class(const GF_CONST GfLinePlan *__restrict__ plan, const GfLineClass &c,
+                                           double m12, double m13, double m23, double s, double r, double u, double q2,
+                                           double &bf, double &sf) {
     bf = u;
     sf = 1.0;
     if(0 == c.spin)
@@ -321,7 +343,7 @@ __device__ __forceinline__ void line_class(const GF_CONST GfLinePlan *__restrict
     for(int k = 0; k < c.spin; ++k)
         bf *= q2;
     const double z = c.r2 * q2;
-    double g;  // sqrt(g) multiplies the amplitude
+    double g;  // multiplies the amplitude
     if(c.norm) {
         // the bachelor's momentum in the form of two_body_cm_mother_mom, 0.5 s / M times two
         // square roots that are 1 below s = (M - mc)^2, the end of the plot
@@ -333,12 +355,12 @@ __device__ __forceinline__ void line_class(const GF_CONST GfLinePlan *__restrict
         const double zm = c.rm2 * s * s * k;
         const double dq = 2 == c.spin ? fma(z, z + 3, 9) : 1 + z;
         const double dm = 2 == c.spin ? fma(zm, zm + 3, 9) : 1 + zm;
-        g               = 1.0 / (dq * dm);
-        bf *= g * dm;
+        g               = rsqrt_n(dq * dm);
+        bf *= g * g * dm;
     } else {
         const double pm = two_body_cm_mom(plan->m2, sqrt(s), c.mc);
         const double f  = 2 == c.spin ? 13 * z / ((z - 3) * (z - 3)) + 9 * z * z : 2 * z;
-        g               = f * damping_factor_square(pm, c.spin, plan->rm);
+        g               = sqrt(f * damping_factor_square(pm, c.spin, plan->rm));
         bf *= f;
     }
     const double sAC = 0 == c.pair ? m13 : (1 == c.pair ? m23 : m12);
@@ -346,46 +368,27 @@ __device__ __forceinline__ void line_class(const GF_CONST GfLinePlan *__restrict
     double f         = -fma(r, c.s0, sBC - sAC);
     if(2 == c.spin)
         f = fma(f, f, -(fma(r, c.s2, s - c.s1) * fma(r, c.s4, s - c.s3)) * (1.0 / 3.0));
-    sf = sqrt(g) * f;
+    sf = g * f;
 }
 
-// One resonance's term at the point.
-__device__ __forceinline__ double2 line_term(const GF_CONST GfLinePlan *__restrict__ plan, const GF_CONST GfLineTerm &t,
-                                             double s, double bf, double sf) {
-    double A = t.m2 - s, B = t.kb * bf;
-    if(t.kind == GR_GS) {
-        // hFun takes the masses of daughters 2 and 3 in every channel, as there
-        const double _pi = 3.14159265359;
-        double k1        = 1 - plan->gsum2 / s;
-        k1               = k1 >= 0 ? k1 : 1;
-        const double k2  = 1 - plan->gdif2 / s;
-        k1 *= k2 >= 0 ? k2 : 1;
-        const double rs = sqrt(s), u = 0.5 * sqrt(k1);
-        const double h  = (2 / _pi) * u * gfmath::log_d(rs * fma(2, u, 1) * plan->ginv);
-        A               = fma(t.f0, fma(0.25 * s * k1, h - t.h0, A * t.d0), A);
-        B *= rs;
-    }
-    const double C = t.ks * sf / fma(A, A, B * B);
-    return make_double2(A * C, B * C);
-}
-
-// Every wave of the plan whose resonance is in mask, at one point: emit(row, swap, add,
+// Every wave of the plan whose resonance is in mask (ALL: every one), at one point: emit(row, swap, add,
 // value).  m23 is the same for the swapped point (m13, m12).  All control flow is
-// uniform over the wave.
-template <class Emit>
-__device__ __forceinline__ void line_waves(const GfLinePlan *__restrict__ plan_, double m12, double m13,
-                                           double m23, uint32_t mask, const Emit &emit) {
+// uniform over the wave, and a class or term is read from the plan as a whole (one wait
+// for its scalar loads).
+template <bool ALL, class Emit>
+__device__ __forceinline__ void line_waves(const GfLinePlan *__restrict__ plan_, double m12, double m13, double m23,
+                                           uint32_t mask, const Emit &emit) {
     const GF_CONST GfLinePlan *__restrict__ plan = as_const(plan_);
     double s = 0, r = 0, u = 0, q2 = 0, bf, sf;
     int chan = -1;
     for(int ci = 0; ci < plan->nclass; ++ci) {
-        const GF_CONST GfLineClass &c = plan->cls[ci];
-        if(!(c.res & mask))
+        const GfLineClass c = plan->cls[ci];
+        if(!ALL && !(c.res & mask))
             continue;
         const int k1 = c.first + c.count;
         if(c.pair < 0) {  // nonres, NonRes.cu:8-11
             for(int k = c.first; k < k1; ++k)
-                if((mask >> plan->term[k].res) & 1u)
+                if(ALL || ((mask >> plan->term[k].res) & 1u))
                     emit(plan->term[k].res, c.swap, 0, make_double2(1.0, 0.0));
             continue;
         }
@@ -395,18 +398,32 @@ __device__ __forceinline__ void line_waves(const GfLinePlan *__restrict__ plan_,
             line_pair(c, x, y, m23, s, r, u, q2);
         }
         line_class(plan, c, x, y, m23, s, r, u, q2, bf, sf);
-        // two terms at a time: their divisions are independent chains
-        int k = c.first;
-        for(; k + 1 < k1; k += 2) {
-            const GF_CONST GfLineTerm &t0 = plan->term[k], &t1 = plan->term[k + 1];
-            const double2 v0 = line_term(plan, t0, s, bf, sf), v1 = line_term(plan, t1, s, bf, sf);
-            if((mask >> t0.res) & 1u)
-                emit(t0.res, c.swap, t0.add, v0);
-            if((mask >> t1.res) & 1u)
-                emit(t1.res, c.swap, t1.add, v1);
+        if(c.gs) {
+            // hFun takes the masses of daughters 2 and 3 in every channel, as there
+            const double _pi = 3.14159265359;
+            const double k   = threshold_factor(plan->gsum2, s, r) * threshold_factor(plan->gdif2, s, r);
+            const double rs = sqrt(s), v = 0.5 * sqrt(k);
+            const double h  = (2 / _pi) * v * gfmath::log_d(rs * fma(2, v, 1) * plan->ginv);
+            for(int j = c.first; j < k1; ++j) {
+                const GfLineTerm t = plan->term[j];
+                const double A0 = t.m2 - s, B = t.kb * bf * rs;
+                const double A = fma(t.f0, fma(0.25 * s * k, h - t.h0, A0 * t.d0), A0);
+                const double C = t.ks * sf * rcp_n(fma(A, A, B * B));
+                if(ALL || ((mask >> t.res) & 1u))
+                    emit(t.res, c.swap, t.add, make_double2(A * C, B * C));
+            }
+            continue;
         }
-        if(k < k1 && ((mask >> plan->term[k].res) & 1u))
-            emit(plan->term[k].res, c.swap, plan->term[k].add, line_term(plan, plan->term[k], s, bf, sf));
+        GfLineTerm t = plan->term[c.first];
+        for(int j = c.first; j < k1; ++j) {
+            const GfLineTerm next = plan->term[j + 1];  // its loads are in flight behind this term
+            if(ALL || ((mask >> t.res) & 1u)) {
+                const double A = t.m2 - s, B = t.kb * bf;
+                const double C = t.ks * sf * rcp_n(fma(A, A, B * B));
+                emit(t.res, c.swap, t.add, make_double2(A * C, B * C));
+            }
+            t = next;
+        }
     }
 }
 

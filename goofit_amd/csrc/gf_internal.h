@@ -91,7 +91,7 @@ struct GfLineClass {
     int32_t first, count;  // its terms
     int32_t pair, spin, norm, swap;  // pair -1: the non-resonant wave, 1 inside the plot
     uint32_t res;          // bit i: a term of resonance i
-    int32_t pad;
+    int32_t gs;            // 1: Gounaris-Sakurai shapes
     double sum2, dif2;     // (ma + mb)^2, (ma - mb)^2 of the pair
     double mc;             // the bachelor's mass
     double msum2, mdif2;   // (M + mc)^2, (M - mc)^2
@@ -113,7 +113,7 @@ struct GfLinePlan {
     double m2, rm;              // mother mass squared, mother radius
     double gsum2, gdif2, ginv;  // Gounaris-Sakurai: (m2 + m3)^2, (m2 - m3)^2, 1 / (m2 + m3)
     GfLineClass cls[GF_MAX_TERMS];
-    GfLineTerm term[GF_MAX_TERMS];
+    GfLineTerm term[GF_MAX_TERMS + 1];  // the last one is read ahead, never used
 };
 
 // Time-resolution models of a time-dependent Dalitz node.
@@ -303,7 +303,8 @@ int launch_gen_scan(bool envelope, double value, const int *bcount, const double
 int launch_compact(const uint32_t *bits, const GfGenBox &box, uint64_t key, int64_t base, int nblocks,
                    const int64_t *boff, int64_t limit, double *o12, double *o13, void *stream);
 // plan (here and in launch_gram): the lineshapes' structure; its numbers are filled in first.
-int launch_dalitz_cache(const GfProgArgs &a, int slot, int64_t offset, int64_t n, uint32_t mask, GfLinePlan *plan,
+// all: mask holds every resonance of the plan.
+int launch_dalitz_cache(const GfProgArgs &a, int slot, int64_t offset, int64_t n, uint32_t mask, bool all, GfLinePlan *plan,
                         int nblocks, void *stream);
 // mode 0: grid cells (grid6 host array); 1: points (m12, m13, w device arrays); 2: data cache of `slot`.
 // Writes 768 doubles (tiles RR, II, RI in MFMA register layout) to tiles_dev.

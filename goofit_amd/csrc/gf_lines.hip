@@ -79,9 +79,10 @@ __global__ __launch_bounds__(GF_MAX_TERMS) void k_line_plan(GfLinePlan *plan, co
     r.ks = ks;
 }
 
-// The wave cache.  16 shapes over 1e6 events: 65 us, 1214 vector instructions per wave of 64
-// events (34 us of issue) beside 256 MB of stores (40 us at the fill rate); 290 us with each
-// shape evaluated by itself.
+// The wave cache (ALL: every resonance).  16 shapes over 1e6 events: 58 us, 1045 vector
+// instructions per wave of 64 events (29 us of issue) beside 256 MB of stores (40 us at the
+// fill rate); 290 us with each shape evaluated by itself.
+template <bool ALL>
 __global__ __launch_bounds__(256) void k_dalitz_cache(GfProgArgs A, int slot, int64_t offset, int64_t n, uint32_t mask,
                                                       const GfLinePlan *__restrict__ plan) {
     const GfDalitzSlot dz = gfd::as_const(A.dz)[slot];
@@ -98,7 +99,7 @@ __global__ __launch_bounds__(256) void k_dalitz_cache(GfProgArgs A, int slot, in
         // same m23 (SpecialWaveCalculator.cu:55-58)
         const double m23 = D.motherMass * D.motherMass + D.daug1Mass * D.daug1Mass + D.daug2Mass * D.daug2Mass
                            + D.daug3Mass * D.daug3Mass - m12 - m13;
-        gfd::line_waves(plan, m12, m13, m23, mask, [&](int i, int swap, int add, double2 v) {
+        gfd::line_waves<ALL>(plan, m12, m13, m23, mask, [&](int i, int swap, int add, double2 v) {
             double2 *w = (swap ? wave_b : wave) + (int64_t)i * dz.ncache + e;
             if(add) {
                 v.x += w->x;
@@ -122,11 +123,11 @@ __device__ __forceinline__ void gen_point(const GfGenBox &B, uint64_t key, uint6
 }
 
 // One workgroup takes GF_GEN_BLOCK candidates: all its lanes draw and test them against
-// the plot, the points inside (about a third of a box around it) are gathered in LDS, and
+// the plot, the points inside (about half of a box around it) are gathered in LDS, and
 // only those are evaluated, on full waves -- the lineshapes are nine tenths of the work.
 // Out: the accepted candidates as bits, their number and the largest value (to check the
-// envelope).  Nothing is done once st->have has reached limit.  A pass of 2^22 candidates,
-// 16 shapes: 208 us with every candidate evaluated in its own lane.
+// envelope).  Nothing is done once st->have has reached limit.  A pass of 2^22 candidates
+// with 16 shapes: 126 us; 208 us with every candidate evaluated in its own lane.
 template <bool GEN_EFF>
 __global__ __launch_bounds__(256) void k_dalitz_candidates(GfProgArgs A, const GfLinePlan *__restrict__ plan,
                                                            int p_coup, int eff_pc, double eff_const, int id12,
@@ -176,7 +177,7 @@ __global__ __launch_bounds__(256) void k_dalitz_candidates(GfProgArgs A, const G
         const double m23 = D.motherMass * D.motherMass + D.daug1Mass * D.daug1Mass + D.daug2Mass * D.daug2Mass
                            + D.daug3Mass * D.daug3Mass - m12 - m13;
         double re = 0.0, im = 0.0;
-        gfd::line_waves(plan, m12, m13, m23, ~0u, [&](int r, int, int, double2 b) {
+        gfd::line_waves<true>(plan, m12, m13, m23, ~0u, [&](int r, int, int, double2 b) {
             const double ar = P[2 * r], ai = P[2 * r + 1];
             re = fma(ar, b.x, fma(-ai, b.y, re));
             im = fma(ar, b.y, fma(ai, b.x, im));
@@ -367,8 +368,8 @@ __global__ __launch_bounds__(256) void k_dalitz_cells(GramSrc S, double *m12, do
 // each of three 16x16 output tiles: RR = R^T E R, II = I^T E I, RI = R^T E I, with
 // E = diag(eff * weight).  No barrier until the four waves' tiles are added at the end.
 // A point outside the Dalitz plot adds nothing, so a wave with none inside moves on (two
-// fifths of the waves over a box around the plot).  16 shapes on 1414 x 1414 cells: 129 us
-// (46 us of vector and 24 us of matrix-core issue; the 16.5 KB of LDS per wave leave two
+// fifths of the waves over a box around the plot).  16 shapes on 1414 x 1414 cells: 115 us
+// (40 us of vector and 24 us of matrix-core issue; the 16.5 KB of LDS per wave leave two
 // waves per SIMD, so latency shows), 450-520 us with each shape evaluated by itself over
 // every cell.  Partials: 3 tiles x 64 lanes x 4 values per block.
 template <bool GEN_EFF>
@@ -411,7 +412,7 @@ __global__ __launch_bounds__(GG_BLOCK) __attribute__((amdgpu_waves_per_eu(2))) v
                 continue;
             const double m23  = D.motherMass * D.motherMass + D.daug1Mass * D.daug1Mass + D.daug2Mass * D.daug2Mass
                                + D.daug3Mass * D.daug3Mass - m12 - m13;
-            gfd::line_waves(plan, m12, m13, m23, ~0u, [&](int i, int, int add, double2 b) {
+            gfd::line_waves<true>(plan, m12, m13, m23, ~0u, [&](int i, int, int add, double2 b) {
                 if(add) {
                     b.x += Xr[wave][i][lane];
                     b.y += Xi[wave][i][lane];
@@ -548,13 +549,17 @@ int launch_compact(const uint32_t *bits, const GfGenBox &box, uint64_t key, int6
     return check(hipGetLastError());
 }
 
-int launch_dalitz_cache(const GfProgArgs &a, int slot, int64_t offset, int64_t n, uint32_t mask, GfLinePlan *plan,
+int launch_dalitz_cache(const GfProgArgs &a, int slot, int64_t offset, int64_t n, uint32_t mask, bool all, GfLinePlan *plan,
                         int nblocks, void *stream) {
     int rc = fill_plan(a, plan, (hipStream_t)stream);
     if(rc)
         return rc;
-    hipLaunchKernelGGL(k_dalitz_cache, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, a, slot, offset, n, mask,
-                       plan);
+    if(all)
+        hipLaunchKernelGGL(k_dalitz_cache<true>, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, a, slot, offset, n,
+                           mask, plan);
+    else
+        hipLaunchKernelGGL(k_dalitz_cache<false>, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, a, slot, offset, n,
+                           mask, plan);
     return check(hipGetLastError());
 }
 
