@@ -2487,7 +2487,10 @@ struct gf_mlp {
     gf_ctx *ctx = nullptr;
     GfMlpDev D{};
     int adam_t     = 0;
-    bool use_graph = true;  // replay one captured training step
+    // replay one captured training step instead of launching it: off, since a step's four
+    // launches keep ahead of its 34 us and the replays cost 5 us of gaps a step more (38.8
+    // against 34.1 us at batch 8192, 27 against 22.5 at 1024, and 0.2 ms of capture a call)
+    bool use_graph = false;
     // tabulated proposal
     double *d_cdf = nullptr, *d_pcell = nullptr;
     int G         = 0;
@@ -2498,7 +2501,7 @@ namespace {
 
 void mlp_free(gf_mlp *m) {
     void *p[] = {m->D.P,     m->D.m,       m->D.v,       m->D.grad,     m->D.w2b,     m->D.w2t,   m->D.xy,
-                 m->D.z1,    m->D.z2,      m->D.h1,      m->D.delta2,   m->D.out,     m->D.coef,  m->D.loss,
+                 m->D.z2,    m->D.out,     m->D.coef,    m->D.loss,
                  m->D.part_in, m->D.part_w2, m->D.part_out, m->d_cdf, m->d_pcell, m->D.state};
     for(void *q : p)
         if(q)
@@ -2587,7 +2590,7 @@ gf_status gf_mlp_create(gf_ctx *ctx, uint64_t seed, int batch_cap, gf_mlp **out)
     GfMlpDev &D = m->D;
     D.cap       = round64(batch_cap);
     const size_t cap = (size_t)D.cap, H = GF_MLP_H;
-    const size_t nb = cap / 64;
+    const size_t nb = cap / 16;  // parts of the gradient
     bool ok = hipMalloc((void **)&D.P, GF_MLP_NPARAM * 4) == hipSuccess
               && hipMalloc((void **)&D.m, GF_MLP_NPARAM * 4) == hipSuccess
               && hipMalloc((void **)&D.v, GF_MLP_NPARAM * 4) == hipSuccess
@@ -2595,10 +2598,7 @@ gf_status gf_mlp_create(gf_ctx *ctx, uint64_t seed, int batch_cap, gf_mlp **out)
               && hipMalloc((void **)&D.w2b, H * H * 2) == hipSuccess
               && hipMalloc((void **)&D.w2t, H * H * 2) == hipSuccess
               && hipMalloc((void **)&D.xy, cap * 8) == hipSuccess
-              && hipMalloc((void **)&D.z1, cap * H * 4) == hipSuccess
               && hipMalloc((void **)&D.z2, cap * H * 4) == hipSuccess
-              && hipMalloc((void **)&D.h1, cap * H * 2) == hipSuccess
-              && hipMalloc((void **)&D.delta2, cap * H * 2) == hipSuccess
               && hipMalloc((void **)&D.out, cap * 4) == hipSuccess
               && hipMalloc((void **)&D.coef, cap * 4) == hipSuccess
               && hipMalloc((void **)&D.loss, 64) == hipSuccess
@@ -2681,7 +2681,7 @@ gf_status gf_mlp_forward(gf_mlp *m, const float *xy, int64_t n, float *out) {
         gf_status st    = mlp_copy_xy(m, xy + 2 * off, c);
         if(st)
             return st;
-        if(gfm::launch_forward(m->D, m->D.xy, (int)round64(c), m->D.out, s))
+        if(gfm::launch_forward(m->D, m->D.xy, (int)round64(c), m->D.out, false, s))
             return fail(GF_ERR_HIP, "forward launch failed");
         GF_HIP(hipMemcpyAsync(out + off, m->D.out, (size_t)c * 4, hipMemcpyDeviceToHost, s));
     }
@@ -2704,7 +2704,7 @@ gf_status gf_mlp_gradient(gf_mlp *m, const float *xy, const float *coef, int64_t
     GF_HIP(hipMemcpyAsync(m->D.coef, coef, (size_t)n * 4, hipMemcpyHostToDevice, s));
     if(np > n)
         GF_HIP(hipMemsetAsync(m->D.coef + n, 0, (size_t)(np - n) * 4, s));
-    if(gfm::launch_forward(m->D, m->D.xy, (int)np, m->D.out, s)
+    if(gfm::launch_forward(m->D, m->D.xy, (int)np, m->D.out, true, s)
        || gfm::launch_backward(m->D, m->D.xy, m->D.coef, (int)np, m->D.grad, s))
         return fail(GF_ERR_HIP, "forward/backward launch failed");
     GF_HIP(hipMemcpyAsync(grad, m->D.grad, GF_MLP_NPARAM * 4, hipMemcpyDeviceToHost, s));
@@ -2812,7 +2812,7 @@ gf_status gf_mlp_build_proposal(gf_mlp *m, const double box[4], int grid, double
         st = fail(GF_ERR_HIP, "grid launch failed");
     for(int64_t off = 0; !st && off < nc; off += m->D.cap) {
         const int64_t c = std::min<int64_t>(m->D.cap, nc - off);  // multiple of 64: grid % 8 == 0
-        if(gfm::launch_forward(m->D, gxy + off, (int)c, gout + off, s))
+        if(gfm::launch_forward(m->D, gxy + off, (int)c, gout + off, false, s))
             st = fail(GF_ERR_HIP, "forward launch failed");
     }
     if(!st && (hipMemcpyAsync(f.data(), gout, (size_t)nc * 4, hipMemcpyDeviceToHost, s) != hipSuccess
