@@ -151,6 +151,7 @@ struct gf_ctx {
     int32_t *d_err           = nullptr;  // device error word (bit 0: cache index out of range, bit 1: node kind not compiled in)
     unsigned long long *d_fuse_slots = nullptr;  // in-kernel finish: 2 x GF_MAX_PARTIALS words
     bool fast_dalitz         = false;    // program is [DALITZ, MULTI_POLY, DALITZ_END, END]
+    bool lone_td             = false;    // program is [TDDP, MULTI_POLY, TDDP_END, END]
     bool flat                = false;    // program is one level of 1-D leaves (flat_program)
     double *d_gram_partials  = nullptr;
     size_t cap_gram_partials = 0;
@@ -878,6 +879,9 @@ GfProgArgs prog_args(gf_ctx *ctx) {
     a.decay        = ctx->decay;
     a.td           = ctx->has_td ? 1 : 0;
     a.has_dz       = ctx->dalitz.empty() ? 0 : 1;
+    a.lone_td      = !ctx->lone_td || !ctx->tune[GF_TUNE_FAST_DALITZ] ? 0
+                     : ctx->dalitz[0].res_kind == GT_THREEGAUSS      ? 2
+                                                                     : 1;
     a.err          = ctx->d_err;
     a.seq          = ctx->res_seq;
     a.mark         = nullptr;
@@ -970,6 +974,16 @@ gf_status read_result(gf_ctx *ctx, double *sum, double *comp) {
     if(comp)
         *comp = r.comp;
     return GF_OK;
+}
+
+// Workgroups of an event sweep outside the coherent fast path.  k_td_reduce takes one event
+// per lane and its registers let three workgroups onto a CU: a fourth would run alone,
+// after the others.
+int sweep_blocks(gf_ctx *ctx, const GfProgArgs &a, int metric) {
+    if(!a.lone_td || metric >= GF_METRIC_BINAVG)
+        return event_blocks(ctx, ctx->n);
+    const int64_t cap = (int64_t)ctx->cu_count * std::min(3, ctx->tune[GF_TUNE_BLOCKS_PER_CU]);
+    return (int)std::max<int64_t>(1, std::min<int64_t>({(ctx->n + GF_BLOCK - 1) / GF_BLOCK, cap, GF_MAX_PARTIALS}));
 }
 
 // Parameter and normalisation values for the kernel arguments (false if they do not fit).
@@ -1094,7 +1108,7 @@ gf_status launch_reduce(gf_ctx *ctx, int metric, hipEvent_t mark = nullptr, bool
                                      ctx->d_partials, ctx->d_res_mapped, event_blocks(ctx, ctx->n), ctx->stream);
     else
         rc = gfk::launch_reduce_metric(a, have_inl ? &inl : nullptr, metric, ctx->d_partials, ctx->d_res_mapped,
-                                       event_blocks(ctx, ctx->n), ctx->stream);
+                                       sweep_blocks(ctx, a, metric), ctx->stream);
     if(rc)
         return fail(GF_ERR_HIP, "reduce launch failed (%d)", rc);
     return GF_OK;
@@ -1568,6 +1582,8 @@ gf_status gf_program_set(gf_ctx *ctx, const int32_t *funcs, int nfunc, const dou
     ctx->fast_dalitz = ctx->ins.size() >= 4 && ctx->ins[0].op == GF_LVL_OP(GK_DALITZ, 0)
                        && ctx->ins[1].op == GI_MULTI_POLY && ctx->ins[2].op == GF_LVL_OP(GK_DALITZ_END, 0)
                        && ctx->ins[3].op == GI_END;
+    ctx->lone_td = ctx->ins.size() >= 4 && ctx->ins[0].op == GF_LVL_OP(GK_TDDP, 0) && ctx->ins[1].op == GI_MULTI_POLY
+                   && ctx->ins[2].op == GF_LVL_OP(GK_TDDP_END, 0) && ctx->ins[3].op == GI_END;
     ctx->flat = flat_program(ctx);
     for(const DalitzNode &d : ctx->dalitz) {
         int cols[7] = {d.col_m12, d.col_m13, d.col_num, d.col_time, d.col_sigma, d.col_mis, d.col_tag};
@@ -1675,11 +1691,11 @@ gf_status gf_reduce_metric_noalloc(gf_ctx *ctx, int metric, gf_result *dev_out, 
         return fail(GF_ERR_STATE, "no-allocation scratch of device %d not set up", ctx->device);
     const bool fast = use_fast_dalitz(ctx, metric);
     const bool flat = !fast && use_flat(ctx, metric);
-    const int nblocks = fast ? fast_blocks(ctx, ctx->n) : event_blocks(ctx, ctx->n);
+    GfProgArgs a = prog_args(ctx);
+    const int nblocks = fast ? fast_blocks(ctx, ctx->n) : sweep_blocks(ctx, a, metric);
     if(nblocks > GF_NOALLOC_PARTIALS)
         return fail(GF_ERR_STATE, "no-allocation reduction: %d workgroups exceed the scratch of %d partials", nblocks,
                     GF_NOALLOC_PARTIALS);
-    GfProgArgs a = prog_args(ctx);
     a.seq        = ++ctx->noalloc_seq;
     if(fast)
         a.coh_group = coh_mx_nres(ctx, metric) > 0;

@@ -9,38 +9,6 @@ namespace {
 
 // ------------------------------------------------------ coherent-sum fast path
 
-// Multivariate polynomial of one event (device_MultiPolynomial,
-// src/PDFs/basic/PolynomialPdf.cu:47-118), columns read at row e.
-__device__ __forceinline__ double multipoly_at(const GfIns &in, const GfProgArgs &A,
-                                               const GF_CONST double *__restrict__ P, int64_t e) {
-    const int nobs      = in.a;
-    const int maxDegree = (int)gfd::as_const(A.consts)[in.c] + 1;
-    int numBoxes        = 1;
-    for(int i = 0; i < nobs; ++i)
-        numBoxes *= maxDegree;
-    int coeff = nobs;
-    double r  = P[in.p + coeff];
-    coeff++;
-    for(int i = 1; i < numBoxes; ++i) {
-        double term = 1;
-        int ci = i, sum = 0;
-        for(int o = 0; o < nobs; ++o) {
-            double x = gfd::as_const(A.cols)[gfd::as_const(A.obsid)[in.x + o]][e];
-            x -= P[in.p + o];
-            int pw = ci % maxDegree;
-            ci /= maxDegree;
-            term *= pow(x, (double)pw);
-            sum += pw;
-        }
-        if(sum >= maxDegree)
-            continue;
-        term *= P[in.p + coeff];
-        coeff++;
-        r += term;
-    }
-    return r;
-}
-
 // |sum_i c_i W_i[e]|^2 * eff for a Dalitz node at the root of the tree.  All
 // wave loads of an event are issued before any arithmetic (16 x 16 bytes per lane
 // in flight); the rest is device_DalitzPlot's arithmetic, the coherent sum in

@@ -443,68 +443,103 @@ __device__ __forceinline__ double truth_resolution(double coshterm, double coste
     return ret;
 }
 
-// One Gaussian of the three-Gaussian model (gaussian(), ThreeGaussResolution.cu:11-61):
-// the decay-time terms convolved with a Gaussian of width adjSigma centred on adjTime;
-// cos and sin are expanded to second and third order in x t / tau.
-__device__ __forceinline__ void tg_gaussian(double &P1, double &P2, double &P3, double &P4, double tau, double adjTime,
-                                            double xmixing, double ymixing, double adjSigma, double selbias) {
-    const double sqrt_pi_over_2 = 1.0 / M_2_SQRTPI;
-    const double inv_sqrt_2pi   = sqrt(0.5 * M_1_PI);
-    const double sixth          = 1.0 / 6.0;
-    const double a1  = adjSigma * M_SQRT2;  // 1 / sqrt(A)
-    const double is  = 1 / adjSigma;
-    const double a2  = 0.5 * a1;
-    const double is2 = is * is;
-    const double ng  = inv_sqrt_2pi * is;
-    const double Cc  = 0.5 * adjTime * adjTime * is2;
-    const double Bgn = -adjTime * is2;
-    const double G   = 1 / tau;
-    const double B   = G + Bgn;
-    const double u0  = a2 * (B + selbias);
-    const double u02 = u0 * u0;
-    const double F   = a1 * exp(-Cc + u02);
-    const double Ig0 = sqrt_pi_over_2 * erfc(u0);
-    const double Ig1 = 0.5 * exp(-u02);
-    const double Ig2 = Ig1 * u0 + 0.5 * Ig0;
-    const double Ig3 = Ig1 * (u02 + 1);
-    const double R   = xmixing * G * a1;
-    const double R2  = R * R;
-    const double It0 = F * Ig0;
-    const double It1 = F * R * (Ig1 - u0 * Ig0);
-    const double It2 = F * R2 * (Ig2 - u0 * Ig1 * 2 + u02 * Ig0);
-    const double It3 = F * R2 * R * (Ig3 - u0 * Ig2 * 3 + u02 * Ig1 * 3 - u0 * u02 * Ig0);
-    P2 = ng * (It0 - 0.5 * It2);
-    P4 = ng * (It1 - sixth * It3);
-    const double upy = a2 * (B - ymixing * G + selbias);
-    const double umy = a2 * (B + ymixing * G + selbias);
-    const double Ipy = a1 * exp(-Cc + upy * upy) * sqrt_pi_over_2 * erfc(upy);
-    const double Imy = a1 * exp(-Cc + umy * umy) * sqrt_pi_over_2 * erfc(umy);
-    P1 = ng * 0.5 * (Ipy + Imy);
-    P3 = ng * 0.5 * (Ipy - Imy);
+// exp and erfcx with their constants in constant memory: scalar loads next to their use.
+// (As literals they are moved to the front of the event loops, some 76 scalar registers
+// that are then spilled to vector lanes and read back one half at a time.)
+static __constant__ double exp_table[gfmath::exp_terms]     = {GF_EXP_TABLE};
+static __constant__ double erfcx_table[gfmath::erfcx_terms] = {GF_ERFCX_TABLE};
+template <int N>
+__device__ __forceinline__ void exp_n(const double (&x)[N], double (&y)[N]) {
+    const GF_CONST double *c = as_const(exp_table);
+    asm volatile("" : "+s"(c));  // not loop-invariant
+    gfmath::exp_n(x, y, c);
+}
+template <int N>
+__device__ __forceinline__ void erfcx(const double (&u)[N], double (&y)[N]) {
+    const GF_CONST double *c = as_const(erfcx_table);
+    asm volatile("" : "+s"(c));
+    double a[N], r[N];
+#pragma unroll
+    for(int i = 0; i < N; ++i) {
+        a[i] = gfmath::erfcx_arg(u[i]);
+        r[i] = rcp_n(gfmath::erfcx_den(a[i]));
+    }
+    gfmath::erfcx(a, r, y, c);
 }
 
 // The decay-time terms P1..P4 (cosh, cos, sinh, sin parts) of the three-Gaussian model,
 // device_threegauss_resolution, ThreeGaussResolution.cu:63-115: core, tail and outlier
 // Gaussians (fractions f_c, f_t, 1 - f_c - f_t) with per-event width sigma.  R = the 13
 // parameters: fractions, biases and scales, selection bias, common offsets.
+//
+// Per Gaussian (gaussian(), ThreeGaussResolution.cu:11-61): the terms convolved with a
+// Gaussian of width s centred on the bias; cos and sin are expanded to second and third
+// order in x t / tau.  With w = t / s, X = exp(-w^2/2) and, for a decay rate g, u =
+// (s g - w) / sqrt(2), the integral of exp(-g t') over t' > 0 under the Gaussian is S(g) / 2,
+// S(g) = exp(u^2 - w^2/2) erfc(u) = X erfcx(u); for u < 0, erfc(u) = 2 - erfc(-u) and
+// u^2 - w^2/2 = s g (s g / 2 - w), formed so because u^2 and w^2/2 cancel for t >> s.  With
+// g0 = 1/tau + selection bias, g+- = g0 -+ y/tau, u of g0 and R = sqrt(2) s x / tau, the
+// moments' recursion in u leaves
+//   P1, P3 = (S(g+) +- S(g-)) / 4,
+//   P2 = S/2 - R^2/2 (S (1/2 + u^2)/2 - u h),  P4 = R (h - u S/2) - R^3/6 (h (1 + u^2) - u S (3/2 + u^2)/2),
+// h = X / (2 sqrt(pi)).  Bound by FP64 issue: three erfcx and four exponentials per Gaussian
+// (350 operations), X shared, where three of the library's erfc and five exponentials took
+// some 1000 and the cancelling exponent cost w^2 / 2 roundings.
 struct TimeTerms {
     double P1, P2, P3, P4;
 };
-__device__ __forceinline__ TimeTerms threegauss_terms(const GF_CONST double *__restrict__ R, double tau, double dtime,
-                                                      double xmixing, double ymixing, double sigma) {
-    const double fc = R[0], ft = R[1], fo = 1 - fc - ft;
-    const double bc = R[2] + R[9], bt = R[4] + R[11], bo = R[6] + R[11];
-    const double sc = R[3] * R[10], st = R[5] * R[12], so = R[7] * R[12];
-    const double sb = R[8];
-    double c1, c2, c3, c4, t1, t2, t3, t4, o1, o2, o3, o4;
-    tg_gaussian(c1, c2, c3, c4, tau, dtime - bc * sigma, xmixing, ymixing, sc * sigma, sb);
-    tg_gaussian(t1, t2, t3, t4, tau, dtime - bt * sigma, xmixing, ymixing, st * sigma, sb);
-    tg_gaussian(o1, o2, o3, o4, tau, dtime - bo * sigma, xmixing, ymixing, so * sigma, sb);
-    TimeTerms P;
-    P.P1 = fc * c1 + ft * t1 + fo * o1;
-    P.P2 = fc * c2 + ft * t2 + fo * o2;
-    P.P3 = fc * c3 + ft * t3 + fo * o3;
-    P.P4 = fc * c4 + ft * t4 + fo * o4;
+// The resolution's parameters, of Gaussian k: fraction, bias and scale (in units of sigma).
+struct GaussParams {
+    const GF_CONST double *R;
+    __device__ __forceinline__ double selbias() const { return R[8]; }
+    __device__ __forceinline__ void get(int k, double &f, double &b, double &s) const {
+        const int o = k < 1 ? 0 : 2;  // the tail and the outlier share their offsets
+        f           = k < 2 ? R[k] : 1 - R[0] - R[1];
+        b           = R[2 + 2 * k] + R[9 + o];
+        s           = R[3 + 2 * k] * R[10 + o];
+    }
+};
+template <class Params>
+__device__ __forceinline__ TimeTerms threegauss_terms(const Params &R, double tau, double dtime, double xmixing,
+                                                      double ymixing, double sigma) {
+    const double G = 1 / tau, g0 = G + R.selbias(), gy = ymixing * G;
+    TimeTerms P{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+    for(int k = 0; k < 3; ++k) {
+        double f, b, s;
+        R.get(k, f, b, s);
+        s *= sigma;
+        const double w    = (dtime - b * sigma) * rcp_n(s);
+        const double q[3] = {s * g0, s * (g0 - gy), s * (g0 + gy)};
+        double u[3], S[3], E[4];
+        {
+            const double x[4] = {-0.5 * w * w, q[0] * fma(0.5, q[0], -w), q[1] * fma(0.5, q[1], -w),
+                                 q[2] * fma(0.5, q[2], -w)};
+            exp_n(x, E);
+        }
+        {
+            double a[3];
+#pragma unroll
+            for(int i = 0; i < 3; ++i) {
+                u[i] = M_SQRT1_2 * (q[i] - w);
+                a[i] = fabs(u[i]);
+            }
+            erfcx(a, S);
+        }
+#pragma unroll
+        for(int i = 0; i < 3; ++i) {
+            S[i] *= E[0];
+            S[i] = u[i] >= 0 ? S[i] : fma(2.0, E[1 + i], -S[i]);
+        }
+        const double h   = (0.25 * M_2_SQRTPI) * E[0], S0 = 0.5 * S[0];
+        const double r   = M_SQRT2 * s * xmixing * G, r2 = r * r, u2 = u[0] * u[0];
+        const double It2 = fma(S0, 0.5 + u2, -u[0] * h);
+        const double It3 = fma(h, 1 + u2, -u[0] * S0 * (1.5 + u2));
+        P.P1 = fma(f, 0.25 * (S[1] + S[2]), P.P1);
+        P.P2 = fma(f, fma(-0.5 * r2, It2, S0), P.P2);
+        P.P3 = fma(f, 0.25 * (S[1] - S[2]), P.P3);
+        P.P4 = fma(f * r, fma((-1.0 / 6.0) * r2, It3, fma(-u[0], S0, h)), P.P4);
+    }
     return P;
 }
 // ThreeGaussResolution.cu:117-122: the rate from the terms
@@ -523,7 +558,7 @@ __device__ __forceinline__ double time_resolution(int kind, const GF_CONST doubl
                                                   double abr, double abi, double tau, double dtime, double x,
                                                   double y, double sigma) {
     if(kind == GT_THREEGAUSS)
-        return threegauss_rate(threegauss_terms(R, tau, dtime, x, y, sigma), t1, t2, abr, abi);
+        return threegauss_rate(threegauss_terms(GaussParams{R}, tau, dtime, x, y, sigma), t1, t2, abr, abi);
     return truth_resolution(t1, t2, abr, abi, tau, dtime, x, y);
 }
 

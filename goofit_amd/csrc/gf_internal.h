@@ -156,6 +156,7 @@ struct GfProgArgs {
     GfDecay decay;
     int32_t td;                  // 1: the program holds a time-dependent Dalitz node
     int32_t has_dz;              // 1: the program holds a Dalitz node (either kind)
+    int32_t lone_td;             // host only: > 0 a lone Amp3Body_TD, reduced by k_td_reduce (1 truth, 2 three-Gaussian)
     int32_t *err;                // device error word (bit 0: cache index out of range, bit 1: node kind not compiled in)
     uint32_t seq;                // sequence number k_finish stamps on its GfResult
     // In-kernel finish (lone-Amp3Body and flat reductions; null: k_finish adds the

@@ -52,35 +52,38 @@ struct RegSrc {
     }
 };
 
-// Per-level accumulators of the combining nodes.
+// Per-level accumulators of the combining nodes: the current level's, taken and put back
+// by selects on the wave-uniform level, so that each node kind is compiled once and not
+// once per level (four copies of the time-dependent node had 960 scalar registers spilled
+// to vector lanes).
 template <int EPT>
 struct Acc {
-    double a0[EPT], a1[EPT], a2[EPT], a3[EPT];
+    double v[4][EPT];
+    __device__ __forceinline__ void take(int l, double (&a)[EPT]) const {
+#pragma unroll
+        for(int j = 0; j < EPT; ++j)
+            a[j] = l == 0 ? v[0][j] : l == 1 ? v[1][j] : l == 2 ? v[2][j] : v[3][j];
+    }
+    __device__ __forceinline__ void put(int l, const double (&a)[EPT]) {
+#pragma unroll
+        for(int k = 0; k < 4; ++k)
+#pragma unroll
+            for(int j = 0; j < EPT; ++j)
+                v[k][j] = l == k ? a[j] : v[k][j];
+    }
 };
-template <int L, int EPT>
-__device__ __forceinline__ double (&level(Acc<EPT> &a))[EPT] {
-    if constexpr(L == 0)
-        return a.a0;
-    else if constexpr(L == 1)
-        return a.a1;
-    else if constexpr(L == 2)
-        return a.a2;
-    else
-        return a.a3;
-}
 
 // ------------------------------------------------------------ interpreter
 
-// One combining step on the accumulator of level L.  FEAT: the node kinds compiled
+// One combining step on the accumulator a of its level.  FEAT: the node kinds compiled
 // in -- 0 none of the Dalitz nodes, 1 the time-integrated Dalitz node, 2 also the
 // time-dependent one -- so that each kernel carries only the register budget of
 // the programs it runs (a Dalitz node met by a kernel without it sets bit 1 of
 // the error word instead of being skipped silently).
-template <int L, int EPT, int FEAT, class Src>
+template <int EPT, int FEAT, class Src>
 __device__ __forceinline__ void step(int kind, const GfIns &in, const GfProgArgs &A, const GF_CONST double *__restrict__ P,
                                      const GF_CONST double *__restrict__ Nm, const Src &src, const int64_t (&row)[EPT],
-                                     const bool (&valid)[EPT], Acc<EPT> &acc, double (&T)[EPT]) {
-    double(&a)[EPT] = level<L>(acc);
+                                     const bool (&valid)[EPT], double (&a)[EPT], double (&T)[EPT]) {
     switch(kind) {
     case GK_PUSH0:
 #pragma unroll
@@ -265,7 +268,7 @@ __device__ __forceinline__ void step(int kind, const GfIns &in, const GfProgArgs
                     if(dz.res_kind == GT_THREEGAUSS) {
                         // both mistag calls take the same (taufix, t, xfix, yfix, sigma): their
                         // Gaussian terms are evaluated once and combined twice (same values)
-                        const gfd::TimeTerms Pf = gfd::threegauss_terms(R, taufix, t, xfix, yfix, sg);
+                        const gfd::TimeTerms Pf = gfd::threegauss_terms(gfd::GaussParams{R}, taufix, t, xfix, yfix, sg);
                         ret += mis * gfd::threegauss_rate(Pf, t1, -t2, abr, -abi);
                         ret += mis * gfd::threegauss_rate(Pf, t1, t2, abr, abi);
                     } else {
@@ -312,10 +315,8 @@ __device__ __forceinline__ void run(const GfProgArgs &A, const double *__restric
     const GF_CONST GfIns *__restrict__ prog = gfd::as_const(A.ins);
     Acc<EPT> acc;
 #pragma unroll
-    for(int j = 0; j < EPT; ++j) {
-        acc.a0[j] = acc.a1[j] = acc.a2[j] = acc.a3[j] = 0.0;
-        T[j]                                          = 0.0;
-    }
+    for(int j = 0; j < EPT; ++j)
+        T[j] = acc.v[0][j] = acc.v[1][j] = acc.v[2][j] = acc.v[3][j] = 0.0;
     for(int pc = pc0;; ++pc) {
         const GfIns in = prog[pc];
         switch(in.op) {
@@ -345,8 +346,9 @@ __device__ __forceinline__ void run(const GfProgArgs &A, const double *__restric
 #pragma unroll
             for(int j = 0; j < EPT; ++j) {
                 double x = src.get(in.a, j), e = 0;
-                for(int i = 0; i < in.k; ++i)
-                    e += pow(x, (double)i) * P[in.p + i];
+                gfmath::Powers xi;
+                for(int i = 0; i < in.k; ++i, xi.next(x))
+                    e += xi.value() * P[in.p + i];
                 T[j] = exp(e);
             }
         } break;
@@ -355,8 +357,11 @@ __device__ __forceinline__ void run(const GfProgArgs &A, const double *__restric
             for(int j = 0; j < EPT; ++j) {
                 double x = src.get(in.a, j), e = 0;
                 x -= P[in.p];
-                for(int i = 1; i < in.k; ++i)
-                    e += pow(x, (double)i) * P[in.p + i];
+                gfmath::Powers xi;
+                for(int i = 1; i < in.k; ++i) {
+                    xi.next(x);
+                    e += xi.value() * P[in.p + i];
+                }
                 T[j] = exp(e);
             }
         } break;
@@ -366,23 +371,24 @@ __device__ __forceinline__ void run(const GfProgArgs &A, const double *__restric
             for(int j = 0; j < EPT; ++j)
                 T[j] = gfd::expgaus(src.get(in.a, j), m, s, al);
         } break;
-        case GI_POLY: {
-            const int lowest = (int)Cn[in.c];
-#pragma unroll
-            for(int j = 0; j < EPT; ++j) {
-                double x = src.get(in.a, j), r = 0;
-                for(int i = 0; i < in.k; ++i)
-                    r += P[in.p + i] * pow(x, (double)(lowest + i));
-                T[j] = r;
-            }
-        } break;
+        case GI_POLY:
         case GI_OFF_POLY: {
-            const int lowest = (int)Cn[in.c];
+            // the powers from lowest on (a negative one apart); the two coefficients in
+            // front of an offset polynomial's are no terms of it
+            const int lowest = (int)Cn[in.c], i0 = in.op == GI_OFF_POLY ? 2 : 0;
 #pragma unroll
             for(int j = 0; j < EPT; ++j) {
-                double x = src.get(in.a, j), r = 0;
-                for(int i = 2; i < in.k; ++i)
-                    r += P[in.p + i] * pow(x, (double)(lowest + i - 2));
+                const double x = src.get(in.a, j);
+                double r       = 0;
+                gfmath::Powers xi;
+                for(int k = 0; k < lowest; ++k)
+                    xi.next(x);
+                for(int i = i0; i < in.k; ++i) {
+                    const int n = lowest + i - i0;
+                    r += P[in.p + i] * (n < 0 ? gfmath::powi(x, n) : xi.value());
+                    if(n >= 0)
+                        xi.next(x);
+                }
                 T[j] = r;
             }
         } break;
@@ -406,7 +412,7 @@ __device__ __forceinline__ void run(const GfProgArgs &A, const double *__restric
                         x -= P[in.p + o];
                         int pw = ci % maxDegree;
                         ci /= maxDegree;
-                        term *= pow(x, (double)pw);
+                        term *= gfmath::powi(x, pw);
                         sum += pw;
                     }
                     if(sum >= maxDegree)
@@ -420,18 +426,47 @@ __device__ __forceinline__ void run(const GfProgArgs &A, const double *__restric
         } break;
         default:
             if(in.op >= GI_LVL) {
-                const int kind = (in.op - GI_LVL) >> 2;
-                switch((in.op - GI_LVL) & 3) {
-                case 0: step<0, EPT, FEAT>(kind, in, A, P, Nm, src, row, valid, acc, T); break;
-                case 1: step<1, EPT, FEAT>(kind, in, A, P, Nm, src, row, valid, acc, T); break;
-                case 2: step<2, EPT, FEAT>(kind, in, A, P, Nm, src, row, valid, acc, T); break;
-                default: step<3, EPT, FEAT>(kind, in, A, P, Nm, src, row, valid, acc, T); break;
-                }
+                double a[EPT];
+                acc.take((in.op - GI_LVL) & 3, a);
+                step<EPT, FEAT>((in.op - GI_LVL) >> 2, in, A, P, Nm, src, row, valid, a, T);
+                acc.put((in.op - GI_LVL) & 3, a);
                 break;
             }
             return;
         }
     }
+}
+
+// Multivariate polynomial of one event (device_MultiPolynomial,
+// src/PDFs/basic/PolynomialPdf.cu:47-118), columns read at row e.
+__device__ __forceinline__ double multipoly_at(const GfIns &in, const GfProgArgs &A,
+                                               const GF_CONST double *__restrict__ P, int64_t e) {
+    const int nobs      = in.a;
+    const int maxDegree = (int)gfd::as_const(A.consts)[in.c] + 1;
+    int numBoxes        = 1;
+    for(int i = 0; i < nobs; ++i)
+        numBoxes *= maxDegree;
+    int coeff = nobs;
+    double r  = P[in.p + coeff];
+    coeff++;
+    for(int i = 1; i < numBoxes; ++i) {
+        double term = 1;
+        int ci = i, sum = 0;
+        for(int o = 0; o < nobs; ++o) {
+            double x = gfd::as_const(A.cols)[gfd::as_const(A.obsid)[in.x + o]][e];
+            x -= P[in.p + o];
+            int pw = ci % maxDegree;
+            ci /= maxDegree;
+            term *= gfmath::powi(x, pw);
+            sum += pw;
+        }
+        if(sum >= maxDegree)
+            continue;
+        term *= P[in.p + coeff];
+        coeff++;
+        r += term;
+    }
+    return r;
 }
 
 // the four result registers of a lane of v_mfma_f64_16x16x4f64

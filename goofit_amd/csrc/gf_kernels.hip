@@ -90,6 +90,150 @@ __global__ __launch_bounds__(GF_BLOCK) void k_reduce_metric(GfProgArgs A, GfInli
     store_partial(s, c, partials);
 }
 
+// ------------------------------------------- a time-dependent node at the root
+
+// The reduction of a lone Amp3Body_TD -- [TDDP, MULTI_POLY, TDDP_END, END] -- with run()'s
+// arithmetic (device_Tddp, src/PDFs/physics/Amp3Body_TD.cu:41-257), one event per lane.
+// Bound by reading the waves (2 x 16 bytes per resonance and event) as long as the
+// decay-time terms, some thousand FP64 operations which need no wave, run while they
+// arrive: the first 2 x TD_CHUNK resonances are loaded before the terms, the following
+// ones each as soon as a chunk is used up.  That takes 168 registers, three waves on a
+// SIMD; in 128, for four, a dozen values per event spill and the sweep is slower (216 us).
+// 1e6 events, 16 resonances, three Gaussians: 194 us in the interpreter with the library's
+// exp and erfc, 160 with this file's terms there, 126 here (4.3 TB/s), on grids of three
+// workgroups a CU (134 on four).
+constexpr int TD_CHUNK = 4;
+struct TdChunk {
+    double2 a[TD_CHUNK], b[TD_CHUNK];
+    // past the last resonance: the last one's again, not used
+    __device__ __forceinline__ void load(const GfDalitzSlot &dz, int i0, int nres, int64_t e) {
+        if(i0 >= nres)
+            return;
+#pragma unroll
+        for(int u = 0; u < TD_CHUNK; ++u) {
+            const int64_t o = (int64_t)(i0 + u < nres ? i0 + u : nres - 1) * dz.ncache + e;
+            a[u]            = dz.wave[o];
+            b[u]            = dz.wave_b[o];
+        }
+    }
+    __device__ __forceinline__ void add(const GF_CONST double *__restrict__ C, int i0, int nres, double2 &sa,
+                                        double2 &sb) const {
+#pragma unroll
+        for(int u = 0; u < TD_CHUNK; ++u)
+            if(i0 + u < nres) {
+                const double cr = C[2 * (i0 + u)], ci = C[2 * (i0 + u) + 1];
+                gfd::cmac(sa.x, sa.y, cr, ci, a[u]);
+                gfd::cmac(sb.x, sb.y, cr, ci, b[u]);
+            }
+    }
+};
+
+// What every event needs and no event changes, in LDS: held in registers across the loop
+// (the compiler moves all of it in front) it would cost 40 vector registers of 128.
+struct TdShared {
+    double f[3], b[3], s[3], sb;
+    GfDecay decay;
+    __device__ __forceinline__ double selbias() const { return sb; }
+    __device__ __forceinline__ void get(int k, double &fk, double &bk, double &sk) const {
+        fk = f[k];
+        bk = b[k];
+        sk = s[k];
+    }
+};
+
+template <bool INL, bool GAUSS>
+__global__ __launch_bounds__(GF_BLOCK, 3) void k_td_reduce(GfProgArgs A, GfInline I, int metric, Partial *partials) {
+    const GF_CONST double *__restrict__ P  = gfd::as_const(INL ? I.p : A.params);
+    const GF_CONST double *__restrict__ Nm = gfd::as_const(INL ? I.n : A.norms);
+    const GfIns td        = gfd::as_const(A.ins)[0];
+    const GfIns eff       = gfd::as_const(A.ins)[1];
+    const GfDalitzSlot dz = gfd::as_const(A.dz)[td.x];
+    const auto cols       = gfd::as_const(A.cols);
+    const GF_CONST double *__restrict__ C = P + td.p + 5;
+    const GF_CONST double *__restrict__ R = P + dz.res_p;
+    const int nres     = td.a;
+    const int64_t n    = A.nevents;
+    const double norm  = Nm[1];
+    const bool nll     = metric == gfd::metric_nll;
+    const double xfix = 0.0039, yfix = 0.0065, taufix = 0.4101;
+    __shared__ TdShared sh;
+    if(threadIdx.x == 0) {
+        if(GAUSS)
+            for(int k = 0; k < 3; ++k)
+                gfd::GaussParams{R}.get(k, sh.f[k], sh.b[k], sh.s[k]);
+        sh.sb    = GAUSS ? R[8] : 0.0;
+        sh.decay = A.decay;
+    }
+    __syncthreads();
+    double s = nll ? 1.0 : 0.0, c = 0.0;  // the NLL as a product: (mantissa, exponent)
+    for(int64_t base = (int64_t)blockIdx.x * GF_BLOCK; base < n; base += (int64_t)gridDim.x * GF_BLOCK) {
+        const int64_t row = base + threadIdx.x < n ? base + threadIdx.x : n - 1;
+        const bool valid  = base + threadIdx.x < n;
+        const double m12 = cols[dz.col_m12][row], m13 = cols[dz.col_m13][row];
+        const double t = cols[dz.col_time][row], sg = cols[dz.col_sigma][row];
+        const int tag      = dz.col_tag >= 0 ? (int)cols[dz.col_tag][row] : 0;
+        const double mis   = dz.col_mis >= 0 ? cols[dz.col_mis][row] : 0.0;
+        asm volatile("" ::: "memory");  // sh is read in each pass
+        const GfDecay &D   = sh.decay;
+        const bool inside  = gfd::in_dalitz(m12, m13, D.motherMass, D.daug1Mass, D.daug2Mass, D.daug3Mass);
+        int64_t e          = A.identity_num ? row : (int64_t)floor(0.5 + cols[dz.col_num][row]);
+        if(e < 0 || e >= dz.ncache) {
+            if(inside && valid)
+                atomicOr(A.err, 1);
+            e = 0;
+        }
+        TdChunk w0, w1;
+        w0.load(dz, 0, nres, e);
+        w1.load(dz, TD_CHUNK, nres, e);
+        const double tau = P[td.p], x0 = P[td.p + 1], y0 = P[td.p + 2], dx = P[td.p + 3], dy = P[td.p + 4];
+        const double x = tag == 1 ? x0 + dx : (tag == -1 ? x0 - dx : x0);
+        const double y = tag == 1 ? y0 + dy : (tag == -1 ? y0 - dy : y0);
+        gfd::TimeTerms Pt{}, Pf{};
+        if constexpr(GAUSS) {
+            Pt = gfd::threegauss_terms(sh, tau, t, x, y, sg);
+            if(mis > 0)
+                Pf = gfd::threegauss_terms(sh, taufix, t, xfix, yfix, sg);
+        }
+        double2 sa = make_double2(0.0, 0.0), sb = make_double2(0.0, 0.0);
+        for(int i0 = 0; i0 < nres; i0 += 2 * TD_CHUNK) {
+            w0.add(C, i0, nres, sa, sb);
+            w0.load(dz, i0 + 2 * TD_CHUNK, nres, e);
+            w1.add(C, i0 + TD_CHUNK, nres, sa, sb);
+            w1.load(dz, i0 + 3 * TD_CHUNK, nres, e);
+        }
+        const double nA = sa.x * sa.x + sa.y * sa.y;
+        const double nB = sb.x * sb.x + sb.y * sb.y;
+        const double t1 = nA + nB, t2 = nA - nB;
+        const double abr = sa.x * sb.x + sa.y * sb.y;  // A conj(B)
+        const double abi = sa.y * sb.x - sa.x * sb.y;
+        double ret;
+        if constexpr(GAUSS)
+            ret = gfd::threegauss_rate(Pt, t1, t2, abr, abi);
+        else
+            ret = gfd::truth_resolution(t1, t2, abr, abi, tau, t, x, y);
+        if(mis > 0) {  // A <-> B with fixed lifetime and mixing (Amp3Body_TD.cu:226-248)
+            ret *= (1 - 2 * mis);
+            if constexpr(GAUSS) {
+                ret += mis * gfd::threegauss_rate(Pf, t1, -t2, abr, -abi);
+                ret += mis * gfd::threegauss_rate(Pf, t1, t2, abr, abi);
+            } else {
+                ret += mis * gfd::truth_resolution(t1, -t2, abr, -abi, taufix, t, xfix, yfix);
+                ret += mis * gfd::truth_resolution(t1, t2, abr, abi, taufix, t, xfix, yfix);
+            }
+        }
+        const double v = inside ? ret * multipoly_at(eff, A, P, row) : 0.0;
+        if(!valid)
+            continue;
+        if(nll)
+            gfd::nll_add(s, c, v, norm);
+        else
+            gfd::kb_add(s, c, gfd::metric(metric, v, 0.0, 0.0, norm, A.total_events));
+    }
+    if(nll)
+        s = gfd::nll_total(s, c), c = 0.0;
+    store_partial(s, c, partials);
+}
+
 // ------------------------------------------------------------ flat trees
 
 // The event columns of a flat program (at most GF_FLAT_COLS), loaded for the whole
@@ -457,6 +601,15 @@ int launch_reduce_metric(const GfProgArgs &a, const GfInline *inl, int metric, P
     // programs without Dalitz nodes: the kernels compiled without them
     const dim3 g(nblocks), b(GF_BLOCK);
     const GfInline none{};
+    if(a.lone_td && metric < GF_METRIC_BINAVG_CODE) {
+        switch((a.lone_td - 1) * 2 + (inl ? 1 : 0)) {
+        case 0: hipLaunchKernelGGL((k_td_reduce<false, false>), g, b, 0, s, a, none, metric, partials); break;
+        case 1: hipLaunchKernelGGL((k_td_reduce<true, false>), g, b, 0, s, a, *inl, metric, partials); break;
+        case 2: hipLaunchKernelGGL((k_td_reduce<false, true>), g, b, 0, s, a, none, metric, partials); break;
+        default: hipLaunchKernelGGL((k_td_reduce<true, true>), g, b, 0, s, a, *inl, metric, partials); break;
+        }
+        return launch_finish(a, partials, nblocks, result, s);
+    }
     switch(feature_level(a) * 2 + (inl ? 1 : 0)) {
     case 0: hipLaunchKernelGGL((k_reduce_metric<2, false, 0>), g, b, 0, s, a, none, metric, partials); break;
     case 1: hipLaunchKernelGGL((k_reduce_metric<2, true, 0>), g, b, 0, s, a, *inl, metric, partials); break;

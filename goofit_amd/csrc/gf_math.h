@@ -1,5 +1,5 @@
-// gf_math.h -- FP64 log for the likelihood metrics, and the NLL of many events as
-// one logarithm.
+// gf_math.h -- FP64 log for the likelihood metrics, the NLL of many events as one
+// logarithm, whole powers, and the scaled complementary error function.
 //
 // Every event of every likelihood sweep takes one logarithm per parameter point
 // (-log of the normalised PDF value), and the multi-point sweeps -- up to 16
@@ -101,5 +101,101 @@ GF_MATH_HD inline void nll_add(double &m, int &e, double v) {
 }
 // sum of -log(v_k) = -(log m + e ln 2)
 GF_MATH_HD inline double nll_total(double m, double e) { return -fma(e, ln2_hi, fma(e, ln2_lo, log_d(m))); }
+
+// Powers x^0, x^1, x^2, ... of the polynomials, each within half a unit in the last place
+// and 2^-100 (the running power kept as an unevaluated sum h + l): four operations a power,
+// where the library's pow, which knows nothing of whole exponents, takes some 200 each time.
+// Once h is infinite or l lost to it, h is the power (overflow and non-finite x as pow).
+struct Powers {
+    double h = 1.0, l = 0.0;
+    GF_MATH_HD void next(double x) {
+        const double p = h * x;
+        l              = fma(h, x, -p) + l * x;
+        h              = p;
+    }
+    GF_MATH_HD double value() const {
+        const double s = h + l;
+        return s == s ? s : h;
+    }
+};
+// x^n of a whole n, uniform over the wave; a negative one as the reciprocal of h + l.
+GF_MATH_HD inline double powi(double x, int n) {
+    Powers p;
+    for(int i = n < 0 ? -n : n; i > 0; --i)
+        p.next(x);
+    if(n >= 0)
+        return p.value();
+    const double r = 1.0 / p.h;
+    const double t = fma(r, fma(-p.h, r, 1.0) - p.l * r, r);
+    return t == t ? t : r;
+}
+
+// exp(x), N arguments side by side so that each constant is read once: x = k ln 2 + r with
+// |r| <= ln(2)/2 (two-part ln 2: k ln2_hi is exact), exp r = 1 + r + r^2 p(r), p the
+// Chebyshev series of (exp r - 1 - r) / r^2 cut at degree 9 (1.3e-17 of exp r), then one
+// ldexp.  Below one unit in the last place; overflow, underflow to 0 through the
+// subnormals, infinities and NaN as the library's.  c = the table: 1 / ln 2, ln2_hi,
+// ln2_lo, the coefficients of p, the highest first.
+#define GF_EXP_TABLE \
+    0x1.71547652b82fep+0, 0x1.62e42ffp-1, -0x1.718432a1b0e26p-35, 0x1.af4ddf7e0398cp-26, \
+    0x1.28917e26a6626p-22, 0x1.71de02365785cp-19, 0x1.a019b91328958p-16, 0x1.a01a01abe6830p-13, \
+    0x1.6c16c1788a55fp-10, 0x1.11111111100dep-7, 0x1.5555555553d67p-5, 0x1.5555555555557p-3, \
+    0x1.0000000000001p-1
+constexpr int exp_terms = 13;
+template <int N, class Table>
+GF_MATH_HD inline void exp_n(const double (&x)[N], double (&y)[N], Table c) {
+    double k[N], r[N];
+    for(int i = 0; i < N; ++i) {
+        const double v = x[i] < -1000.0 ? -1000.0 : x[i] > 1000.0 ? 1000.0 : x[i];
+        k[i]           = rint(v * c[0]);
+        r[i]           = fma(-k[i], c[2], fma(-k[i], c[1], v));
+        y[i]           = c[3];
+    }
+    for(int t = 4; t < exp_terms; ++t) {
+        const double ct = c[t];
+        for(int i = 0; i < N; ++i)
+            y[i] = fma(y[i], r[i], ct);
+    }
+    for(int i = 0; i < N; ++i)
+        y[i] = ldexp(fma(r[i], fma(r[i], y[i], 1.0), 1.0), (int)k[i]);
+}
+
+// erfcx(u) = exp(u^2) erfc(u), the tail of a Gaussian without its exponential, for u >= 0:
+// (1 + u) erfcx(u) runs from 1 at u = 0 to 1/sqrt(pi) at infinity and is smooth in t =
+// (u - K) / (u + K), which maps [0, inf) to [-1, 1) (Shepherd and Laframboise, Math. Comp.
+// 36 (1981) 249, with K = 3.75 and 1 + 2u); its Chebyshev series in t, cut below 3e-17 of
+// it, is the polynomial of degree 23 below, computed in 60 digits from erfc and written in
+// powers of t, the highest first.  One reciprocal serves both quotients: r = 1 /
+// erfcx_den(u) from the caller, c = the table (a copy where the caller can read it fastest).
+// Within 2.5 units in the last place (0.6 rms) over [0, 1e150]; above, where erfcx u is
+// 1/(sqrt(pi) u) to rounding and the denominator would overflow, the value at 1e150.  NaN
+// propagates.  30 FP64 operations and the reciprocal, no branch; the device library's erfc
+// evaluates its ranges' polynomials under a divergent branch and an exponential of its own.
+#define GF_ERFCX_TABLE \
+    0x1.b67d3cbe87cfdp-33, -0x1.3ac6917ca74d1p-30, -0x1.4b3c756e41a2cp-29, 0x1.df8b7453833dcp-27, \
+    0x1.135c3e7c71fe8p-26, -0x1.d4cee07a03890p-24, -0x1.160006d6a62aap-24, 0x1.a2af86b4cd31ep-21, \
+    -0x1.518d8f65de133p-23, -0x1.66b4424d30f98p-18, 0x1.0fce79c4fa4c0p-17, 0x1.cf4eb0935ef46p-16, \
+    -0x1.fc0bd8648af46p-14, 0x1.2839e4434b916p-14, 0x1.c58868fcff65ap-11, -0x1.044be4278f554p-8, \
+    0x1.4a003abc297dbp-7, -0x1.1b08f7c015a79p-6, 0x1.333761f87299dp-6, -0x1.964c5507e5c25p-9, \
+    -0x1.4cfc268c884b0p-5, 0x1.d6351b9255894p-4, -0x1.a79726791d142p-3, 0x1.6212fee9586e8p-1
+constexpr int erfcx_terms = 24;
+GF_MATH_HD inline double erfcx_arg(double u) { return u > 1e150 ? 1e150 : u; }
+GF_MATH_HD inline double erfcx_den(double u) { return (u + 3.75) * (1.0 + u); }
+// N arguments side by side: each coefficient is read once
+template <int N, class Table>
+GF_MATH_HD inline void erfcx(const double (&u)[N], const double (&r)[N], double (&y)[N], Table c) {
+    double t[N];
+    for(int i = 0; i < N; ++i) {
+        t[i] = (u[i] - 3.75) * ((1.0 + u[i]) * r[i]);
+        y[i] = c[0];
+    }
+    for(int k = 1; k < erfcx_terms; ++k) {
+        const double ck = c[k];
+        for(int i = 0; i < N; ++i)
+            y[i] = fma(y[i], t[i], ck);
+    }
+    for(int i = 0; i < N; ++i)
+        y[i] *= (u[i] + 3.75) * r[i];
+}
 
 }  // namespace gfmath
