@@ -153,6 +153,7 @@ struct gf_ctx {
     bool fast_dalitz         = false;    // program is [DALITZ, MULTI_POLY, DALITZ_END, END]
     bool lone_td             = false;    // program is [TDDP, MULTI_POLY, TDDP_END, END]
     bool flat                = false;    // program is one level of 1-D leaves (flat_program)
+    bool flat_prod           = false;    // ... and that level, if there is one, is a ProdPdf
     double *d_gram_partials  = nullptr;
     size_t cap_gram_partials = 0;
     double *d_gram_tiles     = nullptr;  // 768
@@ -882,6 +883,7 @@ GfProgArgs prog_args(gf_ctx *ctx) {
     a.lone_td      = !ctx->lone_td || !ctx->tune[GF_TUNE_FAST_DALITZ] ? 0
                      : ctx->dalitz[0].res_kind == GT_THREEGAUSS      ? 2
                                                                      : 1;
+    a.flat_prod    = ctx->flat_prod ? 1 : 0;
     a.err          = ctx->d_err;
     a.seq          = ctx->res_seq;
     a.mark         = nullptr;
@@ -1009,7 +1011,8 @@ bool use_flat(const gf_ctx *ctx, int metric) {
 }
 
 // Events per lane of the flat kernel: 4 hides more latency on large sets (1e7 events of
-// the 3-D ProdPdf: 123 us against 140 us with 2), 2 keeps small sets on more workgroups.
+// the 3-D ProdPdf: 123 us against 140 us with 2; 71 us in logarithms, k_reduce_prod), 2
+// keeps small sets on more workgroups.
 int flat_ept(const gf_ctx *ctx) {
     const int t = ctx->tune[GF_TUNE_FLAT];
     return t == 1 ? (ctx->n >= ((int64_t)1 << 20) ? 4 : 2) : t;
@@ -1584,7 +1587,10 @@ gf_status gf_program_set(gf_ctx *ctx, const int32_t *funcs, int nfunc, const dou
                        && ctx->ins[3].op == GI_END;
     ctx->lone_td = ctx->ins.size() >= 4 && ctx->ins[0].op == GF_LVL_OP(GK_TDDP, 0) && ctx->ins[1].op == GI_MULTI_POLY
                    && ctx->ins[2].op == GF_LVL_OP(GK_TDDP_END, 0) && ctx->ins[3].op == GI_END;
-    ctx->flat = flat_program(ctx);
+    ctx->flat      = flat_program(ctx);
+    ctx->flat_prod = ctx->flat && (ctx->ins[0].op < GI_LVL || ctx->ins[0].op == GF_LVL_OP(GK_PUSH1, 0))
+                     && std::count_if(ctx->ins.begin(), ctx->ins.end(),
+                                      [](const GfIns &i) { return i.op < GI_LVL && i.op != GI_END; }) <= GF_PROD_LEAVES;
     for(const DalitzNode &d : ctx->dalitz) {
         int cols[7] = {d.col_m12, d.col_m13, d.col_num, d.col_time, d.col_sigma, d.col_mis, d.col_tag};
         for(int c : cols)

@@ -287,13 +287,81 @@ __device__ __forceinline__ void flat_leaf(const GfIns &in, const GF_CONST double
     }
 }
 
+// A flat program over the events in src: run()'s arithmetic with one accumulator.
+template <int EPT>
+__device__ __forceinline__ void flat_run(const GF_CONST GfIns *__restrict__ prog, const GF_CONST double *__restrict__ P,
+                                         const GF_CONST double *__restrict__ Nm, const FlatSrc<EPT> &src,
+                                         double (&T)[EPT]) {
+            double acc[EPT];
+#pragma unroll
+            for(int j = 0; j < EPT; ++j)
+                T[j] = acc[j] = 0.0;
+            for(int pc = 0;; ++pc) {
+                const GfIns in = prog[pc];
+                if(in.op == GI_END)
+                    break;
+                if(in.op < GI_LVL) {
+                    flat_leaf<EPT>(in, P, src, T);
+                    continue;
+                }
+                switch((in.op - GI_LVL) >> 2) {
+                case GK_PUSH0:
+#pragma unroll
+                    for(int j = 0; j < EPT; ++j)
+                        acc[j] = 0.0;
+                    break;
+                case GK_PUSH1:
+#pragma unroll
+                    for(int j = 0; j < EPT; ++j)
+                        acc[j] = 1.0;
+                    break;
+                case GK_ADD_ACC: {
+                    const double w = P[in.p], nm = Nm[in.n];
+#pragma unroll
+                    for(int j = 0; j < EPT; ++j)
+                        acc[j] += w * T[j] * nm;
+                } break;
+                case GK_ADD_LAST: {
+                    double tw = 0;
+                    for(int i = 0; i < in.k; ++i)
+                        tw += P[in.p + i];
+                    const double nm = Nm[in.n];
+#pragma unroll
+                    for(int j = 0; j < EPT; ++j)
+                        acc[j] += (1 - tw) * T[j] * nm;
+                } break;
+                case GK_ADDEXT_END: {
+                    double tw = 0;
+                    for(int i = 0; i < in.k; ++i)
+                        tw += P[in.p + i];
+#pragma unroll
+                    for(int j = 0; j < EPT; ++j)
+                        T[j] = acc[j] / tw;
+                } break;
+                case GK_PROD_ACC: {
+                    const double nm = Nm[in.n];
+#pragma unroll
+                    for(int j = 0; j < EPT; ++j) {
+                        double cur = T[j] * nm;
+                        acc[j] *= cur;
+                    }
+                } break;
+                default:  // GK_POP
+#pragma unroll
+                    for(int j = 0; j < EPT; ++j)
+                        T[j] = acc[j];
+                    break;
+                }
+            }
+}
+
 // The reduction of a flat program -- one leaf, or one AddPdf / ProdPdf level over
 // Gaussian, Exp, Exp-with-offset and ExpGaus leaves, reading columns 0 .. ncols-1
 // (ncols <= GF_FLAT_COLS) -- with run()'s arithmetic in the same order (the same
 // bits as k_reduce_metric) but one accumulator instead of a stack of levels, no
 // Dalitz or polynomial cases, and the tile's columns loaded up front.
 template <int EPT, bool INL>
-__global__ __launch_bounds__(GF_BLOCK) void k_reduce_flat(GfProgArgs A, GfInline I, int metric, int ncols,
+__global__ __launch_bounds__(GF_BLOCK, 4) void k_reduce_flat(GfProgArgs A, GfInline I, int metric, int ncols,
                                                           Partial *partials) {
     const GF_CONST double *__restrict__ P    = gfd::as_const(INL ? I.p : A.params);
     const GF_CONST double *__restrict__ Nm   = gfd::as_const(INL ? I.n : A.norms);
@@ -327,67 +395,8 @@ __global__ __launch_bounds__(GF_BLOCK) void k_reduce_flat(GfProgArgs A, GfInline
                 for(int j = 0; j < EPT; ++j)
                     src.v[j][k] = col[row[j]];
             }
-        double T[EPT], acc[EPT];
-#pragma unroll
-        for(int j = 0; j < EPT; ++j)
-            T[j] = acc[j] = 0.0;
-        for(int pc = 0;; ++pc) {
-            const GfIns in = prog[pc];
-            if(in.op == GI_END)
-                break;
-            if(in.op < GI_LVL) {
-                flat_leaf<EPT>(in, P, src, T);
-                continue;
-            }
-            switch((in.op - GI_LVL) >> 2) {
-            case GK_PUSH0:
-#pragma unroll
-                for(int j = 0; j < EPT; ++j)
-                    acc[j] = 0.0;
-                break;
-            case GK_PUSH1:
-#pragma unroll
-                for(int j = 0; j < EPT; ++j)
-                    acc[j] = 1.0;
-                break;
-            case GK_ADD_ACC: {
-                const double w = P[in.p], nm = Nm[in.n];
-#pragma unroll
-                for(int j = 0; j < EPT; ++j)
-                    acc[j] += w * T[j] * nm;
-            } break;
-            case GK_ADD_LAST: {
-                double tw = 0;
-                for(int i = 0; i < in.k; ++i)
-                    tw += P[in.p + i];
-                const double nm = Nm[in.n];
-#pragma unroll
-                for(int j = 0; j < EPT; ++j)
-                    acc[j] += (1 - tw) * T[j] * nm;
-            } break;
-            case GK_ADDEXT_END: {
-                double tw = 0;
-                for(int i = 0; i < in.k; ++i)
-                    tw += P[in.p + i];
-#pragma unroll
-                for(int j = 0; j < EPT; ++j)
-                    T[j] = acc[j] / tw;
-            } break;
-            case GK_PROD_ACC: {
-                const double nm = Nm[in.n];
-#pragma unroll
-                for(int j = 0; j < EPT; ++j) {
-                    double cur = T[j] * nm;
-                    acc[j] *= cur;
-                }
-            } break;
-            default:  // GK_POP
-#pragma unroll
-                for(int j = 0; j < EPT; ++j)
-                    T[j] = acc[j];
-                break;
-            }
-        }
+        double T[EPT];
+        flat_run<EPT>(prog, P, Nm, src, T);
 #pragma unroll
         for(int j = 0; j < EPT; ++j) {
             if(nll) {
@@ -402,6 +411,215 @@ __global__ __launch_bounds__(GF_BLOCK) void k_reduce_flat(GfProgArgs A, GfInline
     }
     if(nll)
         s = gfd::nll_total(s, c), c = 0.0;
+    if(A.fuse_slots)
+        finish_in_kernel(s, c, A);
+    else
+        store_partial(s, c, partials);
+}
+
+// The NLL of one leaf or of a product of leaves on a large set.  Such a sweep is bound by FP64
+// issue in k_reduce_flat's form (257 operations an event for a Gaussian, an exponential and
+// an ExpGaus, which are 24 bytes: 112 us for 1e7 events); here the leaves' exponents are
+// added and not exponentiated, an ExpGaus leaves its erfcx, and a tile's exponents and factors
+// meet in one compensated sum and one product: 71 us (3.4 TB/s).  125 registers, four waves on
+// a SIMD; loading the next tile ahead takes a wave's place (155 registers: 81 us), two
+// events a lane with the next two ahead also 81.  Taken from 2^20 events on, where k_reduce_flat
+// goes to four events per lane; below, a call is bound by its launch.
+//
+// A wave's tile takes this way only if no partial product of the reference's form leaves the
+// normal range by far -- each exponent below 600 / leaves, the norms (positive) within
+// 2^+-60 -- so that neither form overflows, underflows or meets a NaN.  The events of any
+// other tile are evaluated one by one as k_reduce_flat does (a PDF value that underflows to 0
+// adds 0).
+struct ProdPlan {
+    int ngauss, nexp, nexpgaus;  // leaves by kind, Gaussians first, then exponentials
+    double K, lim;                      // the event-independent factor, the exponents' bound (0: none passes)
+    int col[GF_PROD_LEAVES];
+    double p[GF_PROD_LEAVES][5];        // mean, width^2, 1 / width^2; offset, alpha; see prod_plan
+};
+
+__device__ __forceinline__ void prod_plan(ProdPlan &S, const GF_CONST GfIns *__restrict__ prog,
+                                          const GF_CONST double *__restrict__ P,
+                                          const GF_CONST double *__restrict__ Nm) {
+    double K    = Nm[1];
+    bool inside = K > 0x1p-60 && K < 0x1p60;
+    int count[3] = {0, 0, 0}, n = 0;
+    for(int kind = 0; kind < 3; ++kind)
+        for(int pc = 0; prog[pc].op != GI_END; ++pc) {
+            const GfIns in = prog[pc];
+            if(in.op >= GI_LVL) {
+                if(kind == 0 && (in.op - GI_LVL) >> 2 == GK_PROD_ACC)
+                    K *= Nm[in.n];
+            } else if(kind == (in.op == GI_GAUSS ? 0 : in.op == GI_EXPGAUS ? 2 : 1)) {
+                double *q  = S.p[n];
+                S.col[n++] = in.a;
+                ++count[kind];
+                if(kind == 0) {
+                    q[0] = P[in.p];
+                    q[1] = P[in.p + 1] * P[in.p + 1];
+                    q[2] = 1 / q[1];
+                } else if(kind == 1) {
+                    q[0] = in.op == GI_EXP_OFF ? P[in.p] : 0.0;
+                    q[1] = in.op == GI_EXP_OFF ? P[in.p + 1] : P[in.p];
+                } else {  // expgaus(): exp(q3 (q4 - 2 x)) erfc((q0 - x) / q1)
+                    const double m = P[in.p], sg = P[in.p + 1], al = P[in.p + 2];
+                    q[0] = m + al * sg * sg;
+                    q[1] = sg * 1.4142135623;
+                    q[2] = 1 / q[1];
+                    q[3] = 0.5 * al;
+                    q[4] = 2 * m + al * sg * sg;
+                    K *= q[3];
+                }
+            }
+            inside = inside && K > 0x1p-60 && K < 0x1p60;
+        }
+    S.ngauss   = count[0];
+    S.nexp     = count[1];
+    S.nexpgaus = count[2];
+    S.K        = K;
+    S.lim      = inside ? 600.0 / n : 0.0;
+}
+
+template <int EPT, bool INL>
+__global__ __launch_bounds__(GF_BLOCK, 4) void k_reduce_prod(GfProgArgs A, GfInline I, int ncols, Partial *partials) {
+    const GF_CONST double *__restrict__ P   = gfd::as_const(INL ? I.p : A.params);
+    const GF_CONST double *__restrict__ Nm  = gfd::as_const(INL ? I.n : A.norms);
+    const GF_CONST GfIns *__restrict__ prog = gfd::as_const(A.ins);
+    const auto cols                         = gfd::as_const(A.cols);
+    __shared__ unsigned left[GF_BLOCK / 64][GF_PROD_PASSES / 32];  // passes whose tile was not taken, per wave
+    const int wave = threadIdx.x >> 6;
+    for(int i = threadIdx.x; i < GF_BLOCK / 64 * (GF_PROD_PASSES / 32); i += GF_BLOCK)
+        (&left[0][0])[i] = 0;
+    __shared__ ProdPlan S;
+    if(threadIdx.x == 0)
+        prod_plan(S, prog, P, Nm);
+    __syncthreads();
+    const int64_t n    = A.nevents;
+    const int64_t tile = (int64_t)GF_BLOCK * EPT;
+    const double norm  = Nm[1];
+    const int ng = __builtin_amdgcn_readfirstlane(S.ngauss), ne = ng + __builtin_amdgcn_readfirstlane(S.nexp);
+    const int nl = ne + __builtin_amdgcn_readfirstlane(S.nexpgaus);
+    double s = 1.0, c = 0.0, es = 0.0, ec = 0.0;  // the factors' product, the exponents' sum
+    FlatSrc<EPT> src;
+#pragma unroll
+    for(int j = 0; j < EPT; ++j)
+#pragma unroll
+        for(int k = 0; k < GF_FLAT_COLS; ++k)
+            src.v[j][k] = 0.0;
+    int pass = 0;
+    for(int64_t base = (int64_t)blockIdx.x * tile; base < n; base += (int64_t)gridDim.x * tile, ++pass) {
+        const bool full = base + tile <= n;
+#pragma unroll
+        for(int k = 0; k < GF_FLAT_COLS; ++k)
+            if(k < ncols) {
+                const double *__restrict__ col = cols[k] + base;
+#pragma unroll
+                for(int j = 0; j < EPT; ++j) {
+                    const int o = j * GF_BLOCK + threadIdx.x;
+                    src.v[j][k] = col[full || base + o < n ? o : n - 1 - base];
+                }
+            }
+        asm volatile("" ::: "memory");  // the plan is read where it is used
+        const double lim = S.lim;
+        double E[EPT], G[EPT];
+        bool ok = true;
+#pragma unroll
+        for(int j = 0; j < EPT; ++j) {
+            E[j] = 0.0;
+            G[j] = S.K;
+        }
+        for(int l = 0; l < ng; ++l) {
+            const int a    = __builtin_amdgcn_readfirstlane(S.col[l]);
+            const double m = S.p[l][0], v = S.p[l][1], r = S.p[l][2];
+#pragma unroll
+            for(int j = 0; j < EPT; ++j) {
+                const double d = src.get(a, j) - m, t = -0.5 * d * d, q = t * r;
+                const double e = fma(fma(-q, v, t), r, q);  // t / v, rounded once
+                ok             = ok && fabs(e) < lim;
+                E[j] += e;
+            }
+        }
+        for(int l = ng; l < ne; ++l) {
+            const int a     = __builtin_amdgcn_readfirstlane(S.col[l]);
+            const double x0 = S.p[l][0], al = S.p[l][1];
+#pragma unroll
+            for(int j = 0; j < EPT; ++j) {
+                const double e = al * (src.get(a, j) - x0);
+                ok             = ok && fabs(e) < lim;
+                E[j] += e;
+            }
+        }
+        // exp(e) erfc(u): for u >= 0 exp(e - u^2) erfcx(u), else exp(e) (2 - exp(-u^2) erfcx(-u))
+        for(int l = ne; l < nl; ++l) {
+            const int a = __builtin_amdgcn_readfirstlane(S.col[l]);
+            double u[EPT], y[EPT], t[EPT], g[EPT];
+            {
+                const double c0 = S.p[l][0], v = S.p[l][1], r = S.p[l][2], h = S.p[l][3], c2 = S.p[l][4];
+#pragma unroll
+                for(int j = 0; j < EPT; ++j) {
+                    const double x = src.get(a, j), d = c0 - x, q = d * r;
+                    double e       = h * (c2 - 2 * x);
+                    u[j]           = fma(fma(-q, v, d), r, q);
+                    ok             = ok && fabs(u[j]) < lim;  // and erfcx's reciprocal in range
+                    e              = u[j] >= 0 ? fma(-u[j], u[j], e) : e;
+                    ok             = ok && fabs(e) < lim;
+                    E[j] += e;
+                    t[j] = -u[j] * u[j];
+                    y[j] = fabs(u[j]);
+                }
+            }
+            gfd::exp_n(t, g);
+#pragma unroll
+            for(int j = 0; j < EPT; ++j)
+                g[j] = u[j] >= 0 ? 0.0 : g[j];
+            gfd::erfcx(y, t);
+#pragma unroll
+            for(int j = 0; j < EPT; ++j)
+                G[j] *= u[j] >= 0 ? t[j] : fma(-g[j], t[j], 2.0);
+        }
+        if(__all(ok)) {
+            double e = 0.0, g = 1.0;
+#pragma unroll
+            for(int j = 0; j < EPT; ++j) {
+                const bool valid = full || base + j * GF_BLOCK + threadIdx.x < n;
+                e += valid ? E[j] : 0.0;
+                g *= valid ? G[j] : 1.0;
+            }
+            const double t = es + e, b = t - es;
+            ec += (es - (t - b)) + (e - b);
+            es = t;
+            gfmath::nll_add(s, c, g);
+            continue;
+        }
+        if((threadIdx.x & 63) == 0)
+            left[wave][pass >> 5] |= 1u << (pass & 31);
+    }
+    // The tiles left over, after the loop: inside it the compiler holds the library functions'
+    // constants in vector registers throughout (187 registers, two waves on a SIMD).
+    __syncthreads();
+    for(int w = 0; w <= (pass - 1) >> 5; ++w) {
+        unsigned bits = __builtin_amdgcn_readfirstlane(left[wave][w]);
+        while(bits) {
+            const int t = 32 * w + __builtin_ctz(bits);
+            bits &= bits - 1;
+            for(int j = 0; j < EPT; ++j) {
+                const int64_t row = ((int64_t)t * gridDim.x + blockIdx.x) * tile + j * GF_BLOCK + threadIdx.x;
+                if(row >= n)
+                    continue;
+                FlatSrc<1> one;
+                double T[1];
+#pragma unroll
+                for(int k = 0; k < GF_FLAT_COLS; ++k)
+                    one.v[0][k] = k < ncols ? cols[k][row] : 0.0;
+                flat_run<1>(prog, P, Nm, one, T);
+                gfd::nll_add(s, c, T[0], norm);
+            }
+        }
+    }
+    s = gfd::nll_total(s, c);
+    c = 0.0;
+    gfd::kb_add(s, c, -es);
+    c -= ec;
     if(A.fuse_slots)
         finish_in_kernel(s, c, A);
     else
@@ -627,6 +845,14 @@ int launch_reduce_flat(const GfProgArgs &a, const GfInline *inl, int metric, int
         return -1;
     const dim3 g(nblocks), b(GF_BLOCK);
     const GfInline none{};
+    if(ept == 4 && a.flat_prod && metric == gfd::metric_nll
+       && a.nevents <= (int64_t)GF_PROD_PASSES * nblocks * GF_BLOCK * 4) {
+        if(inl)
+            hipLaunchKernelGGL((k_reduce_prod<4, true>), g, b, 0, s, a, *inl, ncols, partials);
+        else
+            hipLaunchKernelGGL((k_reduce_prod<4, false>), g, b, 0, s, a, none, ncols, partials);
+        return launch_finish(a, partials, nblocks, result, s);
+    }
     switch((ept == 4 ? 2 : 0) + (inl ? 1 : 0)) {
     case 0: hipLaunchKernelGGL((k_reduce_flat<2, false>), g, b, 0, s, a, none, metric, ncols, partials); break;
     case 1: hipLaunchKernelGGL((k_reduce_flat<2, true>), g, b, 0, s, a, *inl, metric, ncols, partials); break;

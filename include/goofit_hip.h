@@ -114,8 +114,9 @@ enum gf_tune {
     GF_TUNE_FLAT               = 6, /* a tree that is one leaf, or one product or sum of 1-D leaves
                                        (Gaussian, Exp, ExpGaus) over at most 4 columns, runs a dedicated
                                        kernel that loads every column of a tile before evaluating it, with
-                                       2 or 4 events per lane (the value), or 1: 4 from 2^20 events on,
-                                       2 below; 0: the general interpreter (default 1) */
+                                       2 or 4 events per lane (the value; at 4 the NLL of a leaf or
+                                       product adds exponents and not values), or 1: 4 from 2^20
+                                       events on, 2 below; 0: the general interpreter (default 1) */
     GF_TUNE_FUSED_FINISH       = 7, /* 1: the coherent-sum and flat reductions add their workgroups'
                                        partials inside the sweep (the last workgroup to finish does it,
                                        in k_finish's order: the same bits) instead of in a second launch;
