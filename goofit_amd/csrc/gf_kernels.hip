@@ -427,8 +427,8 @@ __global__ __launch_bounds__(GF_BLOCK, 4) void k_reduce_flat(GfProgArgs A, GfInl
 // goes to four events per lane; below, a call is bound by its launch.
 //
 // A wave's tile takes this way only if no partial product of the reference's form leaves the
-// normal range by far -- each exponent below 600 / leaves, the norms (positive) within
-// 2^+-60 -- so that neither form overflows, underflows or meets a NaN.  The events of any
+// normal range by far -- each exponent below 600 / leaves, an ExpGaus' erfc above 1e-296, the
+// norms (positive) within 2^+-60 -- so that neither form overflows, underflows or meets a NaN.  The events of any
 // other tile are evaluated one by one as k_reduce_flat does (a PDF value that underflows to 0
 // adds 0).
 struct ProdPlan {
@@ -560,7 +560,7 @@ __global__ __launch_bounds__(GF_BLOCK, 4) void k_reduce_prod(GfProgArgs A, GfInl
                     const double x = src.get(a, j), d = c0 - x, q = d * r;
                     double e       = h * (c2 - 2 * x);
                     u[j]           = fma(fma(-q, v, d), r, q);
-                    ok             = ok && fabs(u[j]) < lim;  // and erfcx's reciprocal in range
+                    ok             = ok && u[j] > -lim && u[j] < 26.0;  // erfc(u) a normal number
                     e              = u[j] >= 0 ? fma(-u[j], u[j], e) : e;
                     ok             = ok && fabs(e) < lim;
                     E[j] += e;
