@@ -381,8 +381,8 @@ __device__ __forceinline__ void run(const GfProgArgs &A, const double *__restric
                 const double x = src.get(in.a, j);
                 double r       = 0;
                 gfmath::Powers xi;
-                for(int k = 0; k < lowest; ++k)
-                    xi.next(x);
+                if(lowest > 0)
+                    xi.start(x, (unsigned)lowest);
                 for(int i = i0; i < in.k; ++i) {
                     const int n = lowest + i - i0;
                     r += P[in.p + i] * (n < 0 ? gfmath::powi(x, n) : xi.value());
@@ -412,7 +412,7 @@ __device__ __forceinline__ void run(const GfProgArgs &A, const double *__restric
                         x -= P[in.p + o];
                         int pw = ci % maxDegree;
                         ci /= maxDegree;
-                        term *= gfmath::powi(x, pw);
+                        term *= gfmath::power(x, pw);
                         sum += pw;
                     }
                     if(sum >= maxDegree)
@@ -457,7 +457,7 @@ __device__ __forceinline__ double multipoly_at(const GfIns &in, const GfProgArgs
             x -= P[in.p + o];
             int pw = ci % maxDegree;
             ci /= maxDegree;
-            term *= gfmath::powi(x, pw);
+            term *= gfmath::power(x, pw);
             sum += pw;
         }
         if(sum >= maxDegree)

@@ -102,27 +102,57 @@ GF_MATH_HD inline void nll_add(double &m, int &e, double v) {
 // sum of -log(v_k) = -(log m + e ln 2)
 GF_MATH_HD inline double nll_total(double m, double e) { return -fma(e, ln2_hi, fma(e, ln2_lo, log_d(m))); }
 
-// Powers x^0, x^1, x^2, ... of the polynomials, each within half a unit in the last place
-// and 2^-100 (the running power kept as an unevaluated sum h + l): four operations a power,
-// where the library's pow, which knows nothing of whole exponents, takes some 200 each time.
-// Once h is infinite or l lost to it, h is the power (overflow and non-finite x as pow).
+// Powers x^n, x^(n+1), ... of the polynomials, each within half a unit in the last place and
+// some 2^-100 (the power kept as an unevaluated sum h + l): five operations a power, where
+// the library's pow, which knows nothing of whole exponents, takes some 200 each time.
+// Where l is no number (overflow, infinite x) h alone is the power, as pow gives it.
 struct Powers {
     double h = 1.0, l = 0.0;
-    GF_MATH_HD void next(double x) {
-        const double p = h * x;
-        l              = fma(h, x, -p) + l * x;
+    GF_MATH_HD void times(double bh, double bl) {
+        const double p = h * bh;
+        l              = fma(h, bh, -p) + (h * bl + l * bh);
         h              = p;
+    }
+    GF_MATH_HD void next(double x) { times(x, 0.0); }
+    // from x^0 to x^n by squarings: any exponent in at most 32 steps
+    GF_MATH_HD void start(double x, unsigned n) {
+        Powers b;
+        b.next(x);
+        while(n) {
+            if(n & 1) {
+                times(b.h, b.l);
+                round();
+            }
+            if((n >>= 1)) {
+                b.times(b.h, b.l);
+                b.round();
+            }
+        }
+    }
+    // h again the nearest double to the sum (l grows by a rounding of h a step)
+    GF_MATH_HD void round() {
+        const double s = h + l;
+        if(s == s && s != 0) {
+            l -= s - h;
+            h = s;
+        }
     }
     GF_MATH_HD double value() const {
         const double s = h + l;
         return s == s ? s : h;
     }
 };
-// x^n of a whole n, uniform over the wave; a negative one as the reciprocal of h + l.
+// x^n by n multiplications, for the small n >= 0 of a polynomial's terms
+GF_MATH_HD inline double power(double x, int n) {
+    Powers p;
+    for(; n > 0; --n)
+        p.next(x);
+    return p.value();
+}
+// x^n of any whole n, uniform over the wave; a negative one as the reciprocal of h + l.
 GF_MATH_HD inline double powi(double x, int n) {
     Powers p;
-    for(int i = n < 0 ? -n : n; i > 0; --i)
-        p.next(x);
+    p.start(x, n < 0 ? 0u - (unsigned)n : (unsigned)n);
     if(n >= 0)
         return p.value();
     const double r = 1.0 / p.h;

@@ -56,7 +56,7 @@ int main(int argc, char **argv) {
     const long long N = argc > 1 ? std::atoll(argv[1]) : 1000000;
     std::mt19937_64 rng(argc > 2 ? std::strtoull(argv[2], nullptr, 10) : 1);
     std::uniform_real_distribution<double> u(0.0, 1.0);
-    Worst e_all, e_small, x_low, x_mid, x_high, pw, pn;
+    Worst e_all, e_small, x_low, x_mid, x_high, pw, pn, pl;
     for(long long i = 0; i < N; ++i) {
         double x = -707.0 + 1416.0 * u(rng);
         e_all.add(x, exp_1(x), expl((long double)x));
@@ -74,7 +74,12 @@ int main(int argc, char **argv) {
         for(int k = 0; k < n; ++k)
             p *= x;
         pw.add(x, gfmath::powi(x, n), p);
+        pw.add(x, gfmath::power(x, n), p);
         pn.add(x, gfmath::powi(x, -n), 1 / p);
+        // exponents to 2^31 of x with |log x^n| < 700 (not by n multiplications)
+        const int big = (int)std::pow(2.0, 31 * u(rng) - 1e-9);
+        x             = 1 + (2 * u(rng) - 1) * std::fmin(0.4, 500.0 / big);
+        pl.add(x, gfmath::powi(x, big), powl(x, big));
     }
     e_all.print("exp_range");
     e_small.print("exp_small");
@@ -83,6 +88,7 @@ int main(int argc, char **argv) {
     x_high.print("erfcx_high");
     pw.print("powi");
     pn.print("powi_negative");
+    pl.print("powi_large");
     for(double x : {0.0, -0.0, 1.0, 710.0, -746.0, -745.0, 1e300, -1e300, (double)HUGE_VAL, -(double)HUGE_VAL, (double)NAN})
         std::printf("special exp x=%.17g y=%.17g library=%.17g\n", x, exp_1(x), std::exp(x));
     for(double x : {0.0, 1e200, (double)HUGE_VAL, (double)NAN})
