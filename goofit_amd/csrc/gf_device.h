@@ -484,7 +484,9 @@ __device__ __forceinline__ void erfcx(const double (&u)[N], double (&y)[N]) {
 //   P2 = S/2 - R^2/2 (S (1/2 + u^2)/2 - u h),  P4 = R (h - u S/2) - R^3/6 (h (1 + u^2) - u S (3/2 + u^2)/2),
 // h = X / (2 sqrt(pi)).  Bound by FP64 issue: three erfcx and four exponentials per Gaussian
 // (350 operations), X shared, where three of the library's erfc and five exponentials took
-// some 1000 and the cancelling exponent cost w^2 / 2 roundings.
+// some 1000 and the cancelling exponent cost w^2 / 2 roundings (P1 of exponential times at
+// widths of 0.03 to 0.08, against 40 digits: 2.3e-14 rms and 7e-15 mean then, 1.4e-16 and
+// 3e-17 now).
 struct TimeTerms {
     double P1, P2, P3, P4;
 };

@@ -102,7 +102,7 @@ const char *gf_last_error(void);
 enum gf_tune {
     GF_TUNE_INLINE_ARGS        = 0, /* 1: parameter and normalisation values travel in the kernel
                                        arguments (no upload copy); 0: device buffers (default 1) */
-    GF_TUNE_FAST_DALITZ        = 1, /* 1: dedicated coherent-sum kernel for a lone Amp3Body (default 1) */
+    GF_TUNE_FAST_DALITZ        = 1, /* 1: dedicated kernels for a lone Amp3Body or Amp3Body_TD (default 1) */
     GF_TUNE_BLOCKS_PER_CU      = 2, /* interpreter reduction grid cap, workgroups per CU (1..64, default 4) */
     GF_TUNE_FAST_BLOCKS_PER_CU = 3, /* coherent-sum kernel grid cap, workgroups per CU (1..64, default 3) */
     GF_TUNE_SPIN_US            = 4, /* a reduction's caller polls the result for up to this many
