@@ -100,7 +100,7 @@ __global__ __launch_bounds__(GF_BLOCK) void k_reduce_metric(GfProgArgs A, GfInli
 // ones each as soon as a chunk is used up.  That takes 168 registers, three waves on a
 // SIMD; in 128, for four, a dozen values per event spill and the sweep is slower (216 us).
 // 1e6 events, 16 resonances, three Gaussians: 194 us in the interpreter with the library's
-// exp and erfc, 160 with this file's terms there, 126 here (4.3 TB/s), on grids of three
+// exp and erfc, 160 with these terms there, 129 here (4.2 TB/s), on grids of three
 // workgroups a CU (134 on four).
 constexpr int TD_CHUNK = 4;
 struct TdChunk {
