@@ -153,7 +153,7 @@ struct gf_ctx {
     bool fast_dalitz         = false;    // program is [DALITZ, MULTI_POLY, DALITZ_END, END]
     bool lone_td             = false;    // program is [TDDP, MULTI_POLY, TDDP_END, END]
     bool flat                = false;    // program is one level of 1-D leaves (flat_program)
-    bool flat_prod           = false;    // ... and that level, if there is one, is a ProdPdf
+    int flat_prod            = 0;        // ... and that level, if there is one, is a ProdPdf: its instructions
     double *d_gram_partials  = nullptr;
     size_t cap_gram_partials = 0;
     double *d_gram_tiles     = nullptr;  // 768
@@ -864,6 +864,22 @@ gf_status flush_uploads(gf_ctx *ctx) {
     return GF_OK;
 }
 
+// k_reduce_prod's part of its bound that no event changes: the norms and the ExpGaus leaves'
+// rates / 2, multiplied one by one, stay within 2^+-60.
+bool prod_norms(const gf_ctx *ctx) {
+    double K    = ctx->norms[1];
+    bool inside = K > 0x1p-60 && K < 0x1p60;
+    for(int i = 0; i < ctx->flat_prod; i++) {
+        const GfIns &in = ctx->ins[i];
+        if(in.op == GI_EXPGAUS)
+            K *= 0.5 * ctx->params[in.p + 2];
+        else if(in.op == GF_LVL_OP(GK_PROD_ACC, 0))
+            K *= ctx->norms[in.n];
+        inside = inside && K > 0x1p-60 && K < 0x1p60;
+    }
+    return inside;
+}
+
 GfProgArgs prog_args(gf_ctx *ctx) {
     GfProgArgs a;
     a.ins          = ctx->d_ins;
@@ -883,7 +899,7 @@ GfProgArgs prog_args(gf_ctx *ctx) {
     a.lone_td      = !ctx->lone_td || !ctx->tune[GF_TUNE_FAST_DALITZ] ? 0
                      : ctx->dalitz[0].res_kind == GT_THREEGAUSS      ? 2
                                                                      : 1;
-    a.flat_prod    = ctx->flat_prod ? 1 : 0;
+    a.flat_prod    = ctx->flat_prod && prod_norms(ctx) ? ctx->flat_prod : 0;
     a.err          = ctx->d_err;
     a.seq          = ctx->res_seq;
     a.mark         = nullptr;
@@ -1011,7 +1027,7 @@ bool use_flat(const gf_ctx *ctx, int metric) {
 }
 
 // Events per lane of the flat kernel: 4 hides more latency on large sets (1e7 events of
-// the 3-D ProdPdf: 123 us against 140 us with 2; 71 us in logarithms, k_reduce_prod), 2
+// the 3-D ProdPdf: 112 us against 140 us with 2; 70 us in logarithms, k_reduce_prod), 2
 // keeps small sets on more workgroups.
 int flat_ept(const gf_ctx *ctx) {
     const int t = ctx->tune[GF_TUNE_FLAT];
@@ -1588,9 +1604,13 @@ gf_status gf_program_set(gf_ctx *ctx, const int32_t *funcs, int nfunc, const dou
     ctx->lone_td = ctx->ins.size() >= 4 && ctx->ins[0].op == GF_LVL_OP(GK_TDDP, 0) && ctx->ins[1].op == GI_MULTI_POLY
                    && ctx->ins[2].op == GF_LVL_OP(GK_TDDP_END, 0) && ctx->ins[3].op == GI_END;
     ctx->flat      = flat_program(ctx);
-    ctx->flat_prod = ctx->flat && (ctx->ins[0].op < GI_LVL || ctx->ins[0].op == GF_LVL_OP(GK_PUSH1, 0))
-                     && std::count_if(ctx->ins.begin(), ctx->ins.end(),
-                                      [](const GfIns &i) { return i.op < GI_LVL && i.op != GI_END; }) <= GF_PROD_LEAVES;
+    ctx->flat_prod = 0;
+    if(ctx->flat && (ctx->ins[0].op < GI_LVL || ctx->ins[0].op == GF_LVL_OP(GK_PUSH1, 0))) {
+        int leaves = 0, nins = 0;
+        for(; ctx->ins[nins].op != GI_END; nins++)
+            leaves += ctx->ins[nins].op < GI_LVL;
+        ctx->flat_prod = leaves <= GF_PROD_LEAVES ? nins : 0;
+    }
     for(const DalitzNode &d : ctx->dalitz) {
         int cols[7] = {d.col_m12, d.col_m13, d.col_num, d.col_time, d.col_sigma, d.col_mis, d.col_tag};
         for(int c : cols)

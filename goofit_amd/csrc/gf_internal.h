@@ -138,7 +138,6 @@ struct GfDalitzSlot {
 };
 
 #define GF_PROD_LEAVES 16  // leaves of a product that k_reduce_prod takes
-#define GF_PROD_PASSES 8192  // passes of its grid over the events (8e9 events on 1024 workgroups)
 
 // Everything an event-evaluating kernel needs, passed by value as the kernel
 // argument.  Arrays indexed by a program operand (column pointers, Dalitz
@@ -160,7 +159,7 @@ struct GfProgArgs {
     int32_t td;                  // 1: the program holds a time-dependent Dalitz node
     int32_t has_dz;              // 1: the program holds a Dalitz node (either kind)
     int32_t lone_td;             // host only: > 0 a lone Amp3Body_TD, reduced by k_td_reduce (1 truth, 2 three-Gaussian)
-    int32_t flat_prod;           // host only: a flat program is one leaf or a product of at most GF_PROD_LEAVES
+    int32_t flat_prod;           // > 0: k_reduce_prod may take the program, of that many instructions
     int32_t *err;                // device error word (bit 0: cache index out of range, bit 1: node kind not compiled in)
     uint32_t seq;                // sequence number k_finish stamps on its GfResult
     // In-kernel finish (lone-Amp3Body and flat reductions; null: k_finish adds the

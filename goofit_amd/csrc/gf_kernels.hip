@@ -421,63 +421,88 @@ __global__ __launch_bounds__(GF_BLOCK, 4) void k_reduce_flat(GfProgArgs A, GfInl
 // issue in k_reduce_flat's form (257 operations an event for a Gaussian, an exponential and
 // an ExpGaus, which are 24 bytes: 112 us for 1e7 events); here the leaves' exponents are
 // added and not exponentiated, an ExpGaus leaves its erfcx, and a tile's exponents and factors
-// meet in one compensated sum and one product: 71 us (3.4 TB/s).  125 registers, four waves on
+// meet in one compensated sum and one product: 70 us (3.4 TB/s).  121 registers, four waves on
 // a SIMD; loading the next tile ahead takes a wave's place (155 registers: 81 us), two
 // events a lane with the next two ahead also 81.  Taken from 2^20 events on, where k_reduce_flat
-// goes to four events per lane; below, a call is bound by its launch.
+// goes to four events per lane: 16 us against 19 there, with the first tile's columns requested
+// before the plan is formed.
 //
-// A wave's tile takes this way only if no partial product of the reference's form leaves the
-// normal range by far -- each exponent below 600 / leaves, an ExpGaus' erfc above 1e-296, the
-// norms (positive) within 2^+-60 -- so that neither form overflows, underflows or meets a NaN.  The events of any
-// other tile are evaluated one by one as k_reduce_flat does (a PDF value that underflows to 0
-// adds 0).
+// An event takes this way if no partial product of the reference's form can leave the normal
+// range: its leaves' negative exponents add up to more than -616, the positive ones to less than
+// 600, an ExpGaus' u < 24 (erfc above 1e-253, its exponential below e^577), the norms (positive)
+// within 2^+-60, so each within 2^+-120 (the caller's part: prod_norms).  It adds nothing if one
+// of its leaves is certain to round to 0 (an exponent below -750, an ExpGaus' u > 28): the
+// product is then 0, or NaN if another leaf is infinite.  The loop tests less: the exponents'
+// sum above -520, each Exp's below 80 / their number and each ExpGaus' below 1.  Any other event
+// is noted and evaluated after the loop as k_reduce_flat does, on full waves.  A wave that meets
+// more than GF_PROD_MISSES of them in a tile, or has noted GF_PROD_NOTES, evaluates this tile and
+// its remaining ones so.  What is left of k_reduce_flat's speed on samples that meet these bounds, at
+// 1e7 events: 72 us where any share of the events is certain to be 0, 70 with decay times to 330
+// widths of the resolution, 137 (k_reduce_flat 115) where a fifth of all events lies between; at 2^20
+// events 16, 16 and 27 (19).  (Giving up a whole tile for one event, and bounding u from below:
+// 239, 175 and 241; 37, 35 and 37.)
 struct ProdPlan {
     int ngauss, nexp, nexpgaus;  // leaves by kind, Gaussians first, then exponentials
-    double K, lim;                      // the event-independent factor, the exponents' bound (0: none passes)
+    double K, rise;                     // the event-independent factor, the bound of an Exp's exponent
     int col[GF_PROD_LEAVES];
     double p[GF_PROD_LEAVES][5];        // mean, width^2, 1 / width^2; offset, alpha; see prod_plan
 };
+#define GF_PROD_MISSES 96
+#define GF_PROD_NOTES 1024
 
-__device__ __forceinline__ void prod_plan(ProdPlan &S, const GF_CONST GfIns *__restrict__ prog,
+// By the lanes of one wave, an instruction each (a product's program has at most 2 x
+// GF_PROD_LEAVES + 3 of them): one lane alone took 3 us of its dependent loads and divisions.
+__device__ __forceinline__ void prod_plan(ProdPlan &S, const GF_CONST GfIns *__restrict__ prog, int nins,
                                           const GF_CONST double *__restrict__ P,
                                           const GF_CONST double *__restrict__ Nm) {
-    double K    = Nm[1];
-    bool inside = K > 0x1p-60 && K < 0x1p60;
-    int count[3] = {0, 0, 0}, n = 0;
-    for(int kind = 0; kind < 3; ++kind)
-        for(int pc = 0; prog[pc].op != GI_END; ++pc) {
-            const GfIns in = prog[pc];
-            if(in.op >= GI_LVL) {
-                if(kind == 0 && (in.op - GI_LVL) >> 2 == GK_PROD_ACC)
-                    K *= Nm[in.n];
-            } else if(kind == (in.op == GI_GAUSS ? 0 : in.op == GI_EXPGAUS ? 2 : 1)) {
-                double *q  = S.p[n];
-                S.col[n++] = in.a;
-                ++count[kind];
-                if(kind == 0) {
-                    q[0] = P[in.p];
-                    q[1] = P[in.p + 1] * P[in.p + 1];
-                    q[2] = 1 / q[1];
-                } else if(kind == 1) {
-                    q[0] = in.op == GI_EXP_OFF ? P[in.p] : 0.0;
-                    q[1] = in.op == GI_EXP_OFF ? P[in.p + 1] : P[in.p];
-                } else {  // expgaus(): exp(q3 (q4 - 2 x)) erfc((q0 - x) / q1)
-                    const double m = P[in.p], sg = P[in.p + 1], al = P[in.p + 2];
-                    q[0] = m + al * sg * sg;
-                    q[1] = sg * 1.4142135623;
-                    q[2] = 1 / q[1];
-                    q[3] = 0.5 * al;
-                    q[4] = 2 * m + al * sg * sg;
-                    K *= q[3];
-                }
+    static_assert(2 * GF_PROD_LEAVES + 3 <= 64, "an instruction per lane");
+    const int lane = threadIdx.x;
+    GfIns in{};
+    in.op = GI_END;
+    if(lane < nins)
+        in = prog[lane];
+    const bool leaf = in.op != GI_END && in.op < GI_LVL;
+    const int kind  = in.op == GI_GAUSS ? 0 : in.op == GI_EXPGAUS ? 2 : 1;
+    int first = 0, count[3];
+    double K = lane == 0 ? Nm[1] : 1.0;
+    for(int k = 0; k < 3; ++k) {
+        const unsigned long long m = __ballot(leaf && kind == k);
+        count[k]                   = __popcll(m);
+        if(leaf && kind == k) {
+            const int at = first + __popcll(m & ((1ull << lane) - 1ull));
+            double *q    = S.p[at];
+            S.col[at]    = in.a;
+            if(k == 0) {
+                const double v = P[in.p + 1] * P[in.p + 1];
+                q[0] = P[in.p];
+                q[1] = v;
+                q[2] = 1 / v;
+            } else if(k == 1) {
+                q[0] = in.op == GI_EXP_OFF ? P[in.p] : 0.0;
+                q[1] = in.op == GI_EXP_OFF ? P[in.p + 1] : P[in.p];
+            } else {  // expgaus(): exp(q3 (q4 - 2 x)) erfc((q0 - x) / q1)
+                const double m = P[in.p], sg = P[in.p + 1], al = P[in.p + 2], w = sg * 1.4142135623;
+                q[0] = m + al * sg * sg;
+                q[1] = w;
+                q[2] = 1 / w;
+                q[3] = 0.5 * al;
+                q[4] = 2 * m + al * sg * sg;
+                K *= q[3];
             }
-            inside = inside && K > 0x1p-60 && K < 0x1p60;
         }
-    S.ngauss   = count[0];
-    S.nexp     = count[1];
-    S.nexpgaus = count[2];
-    S.K        = K;
-    S.lim      = inside ? 600.0 / n : 0.0;
+        first += count[k];
+    }
+    if(in.op >= GI_LVL && (in.op - GI_LVL) >> 2 == GK_PROD_ACC)
+        K = Nm[in.n];
+    for(int off = 32; off > 0; off >>= 1)
+        K *= __shfl_xor(K, off, 64);
+    if(lane == 0) {
+        S.ngauss   = count[0];
+        S.nexp     = count[1];
+        S.nexpgaus = count[2];
+        S.K        = K;
+        S.rise     = 80.0 / count[1];
+    }
 }
 
 template <int EPT, bool INL>
@@ -486,19 +511,12 @@ __global__ __launch_bounds__(GF_BLOCK, 4) void k_reduce_prod(GfProgArgs A, GfInl
     const GF_CONST double *__restrict__ Nm  = gfd::as_const(INL ? I.n : A.norms);
     const GF_CONST GfIns *__restrict__ prog = gfd::as_const(A.ins);
     const auto cols                         = gfd::as_const(A.cols);
-    __shared__ unsigned left[GF_BLOCK / 64][GF_PROD_PASSES / 32];  // passes whose tile was not taken, per wave
-    const int wave = threadIdx.x >> 6;
-    for(int i = threadIdx.x; i < GF_BLOCK / 64 * (GF_PROD_PASSES / 32); i += GF_BLOCK)
-        (&left[0][0])[i] = 0;
     __shared__ ProdPlan S;
-    if(threadIdx.x == 0)
-        prod_plan(S, prog, P, Nm);
-    __syncthreads();
+    __shared__ unsigned note[GF_BLOCK / 64][GF_PROD_NOTES];  // 64 (pass EPT + event of the lane) + lane
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int64_t n    = A.nevents;
     const int64_t tile = (int64_t)GF_BLOCK * EPT;
     const double norm  = Nm[1];
-    const int ng = __builtin_amdgcn_readfirstlane(S.ngauss), ne = ng + __builtin_amdgcn_readfirstlane(S.nexp);
-    const int nl = ne + __builtin_amdgcn_readfirstlane(S.nexpgaus);
     double s = 1.0, c = 0.0, es = 0.0, ec = 0.0;  // the factors' product, the exponents' sum
     FlatSrc<EPT> src;
 #pragma unroll
@@ -506,9 +524,7 @@ __global__ __launch_bounds__(GF_BLOCK, 4) void k_reduce_prod(GfProgArgs A, GfInl
 #pragma unroll
         for(int k = 0; k < GF_FLAT_COLS; ++k)
             src.v[j][k] = 0.0;
-    int pass = 0;
-    for(int64_t base = (int64_t)blockIdx.x * tile; base < n; base += (int64_t)gridDim.x * tile, ++pass) {
-        const bool full = base + tile <= n;
+    const auto load = [&](int64_t base, bool full) {
 #pragma unroll
         for(int k = 0; k < GF_FLAT_COLS; ++k)
             if(k < ncols) {
@@ -519,10 +535,24 @@ __global__ __launch_bounds__(GF_BLOCK, 4) void k_reduce_prod(GfProgArgs A, GfInl
                     src.v[j][k] = col[full || base + o < n ? o : n - 1 - base];
                 }
             }
+    };
+    const int64_t base0 = (int64_t)blockIdx.x * tile, stride = (int64_t)gridDim.x * tile;
+    const int npass     = base0 < n ? (int)((n - base0 + stride - 1) / stride) : 0;
+    if(npass)
+        load(base0, base0 + tile <= n);
+    if(wave == 0)
+        prod_plan(S, prog, A.flat_prod, P, Nm);
+    __syncthreads();
+    const int ng = __builtin_amdgcn_readfirstlane(S.ngauss), ne = ng + __builtin_amdgcn_readfirstlane(S.nexp);
+    const int nl = ne + __builtin_amdgcn_readfirstlane(S.nexpgaus);
+    int pass = 0, notes = 0;
+    while(pass < npass) {
+        const int64_t base = base0 + pass * stride;
+        const bool full    = base + tile <= n;
         asm volatile("" ::: "memory");  // the plan is read where it is used
-        const double lim = S.lim;
-        double E[EPT], G[EPT];
-        bool ok = true;
+        double E[EPT], G[EPT];  // exponents, factors
+        const double rise = S.rise;
+        bool ok           = full;
 #pragma unroll
         for(int j = 0; j < EPT; ++j) {
             E[j] = 0.0;
@@ -534,9 +564,7 @@ __global__ __launch_bounds__(GF_BLOCK, 4) void k_reduce_prod(GfProgArgs A, GfInl
 #pragma unroll
             for(int j = 0; j < EPT; ++j) {
                 const double d = src.get(a, j) - m, t = -0.5 * d * d, q = t * r;
-                const double e = fma(fma(-q, v, t), r, q);  // t / v, rounded once
-                ok             = ok && fabs(e) < lim;
-                E[j] += e;
+                E[j] += fma(fma(-q, v, t), r, q);  // t / v, rounded once
             }
         }
         for(int l = ng; l < ne; ++l) {
@@ -545,11 +573,12 @@ __global__ __launch_bounds__(GF_BLOCK, 4) void k_reduce_prod(GfProgArgs A, GfInl
 #pragma unroll
             for(int j = 0; j < EPT; ++j) {
                 const double e = al * (src.get(a, j) - x0);
-                ok             = ok && fabs(e) < lim;
+                ok             = ok && e < rise;
                 E[j] += e;
             }
         }
-        // exp(e) erfc(u): for u >= 0 exp(e - u^2) erfcx(u), else exp(e) (2 - exp(-u^2) erfcx(-u))
+        // exp(e) erfc(u): for u >= 0 exp(e - u^2) erfcx(u), else exp(e) (2 - exp(-u^2) erfcx(-u)),
+        // for any u below 0: far below, the second term is 0
         for(int l = ne; l < nl; ++l) {
             const int a = __builtin_amdgcn_readfirstlane(S.col[l]);
             double u[EPT], y[EPT], t[EPT], g[EPT];
@@ -560,9 +589,8 @@ __global__ __launch_bounds__(GF_BLOCK, 4) void k_reduce_prod(GfProgArgs A, GfInl
                     const double x = src.get(a, j), d = c0 - x, q = d * r;
                     double e       = h * (c2 - 2 * x);
                     u[j]           = fma(fma(-q, v, d), r, q);
-                    ok             = ok && u[j] > -lim && u[j] < 26.0;  // erfc(u) a normal number
                     e              = u[j] >= 0 ? fma(-u[j], u[j], e) : e;
-                    ok             = ok && fabs(e) < lim;
+                    ok             = ok && u[j] < 24.0 && e < 1.0;
                     E[j] += e;
                     t[j] = -u[j] * u[j];
                     y[j] = fabs(u[j]);
@@ -577,44 +605,89 @@ __global__ __launch_bounds__(GF_BLOCK, 4) void k_reduce_prod(GfProgArgs A, GfInl
             for(int j = 0; j < EPT; ++j)
                 G[j] *= u[j] >= 0 ? t[j] : fma(-g[j], t[j], 2.0);
         }
-        if(__all(ok)) {
-            double e = 0.0, g = 1.0;
+#pragma unroll
+        for(int j = 0; j < EPT; ++j)
+            ok = ok && E[j] > -520.0;
+        if(!__all(ok)) {  // which events, by the bounds themselves
+            unsigned long long miss[EPT];
+            int misses = 0;
 #pragma unroll
             for(int j = 0; j < EPT; ++j) {
-                const bool valid = full || base + j * GF_BLOCK + threadIdx.x < n;
-                e += valid ? E[j] : 0.0;
-                g *= valid ? G[j] : 1.0;
+                bool in = E[j] == E[j], zero = !(base + j * GF_BLOCK + threadIdx.x < n);
+                double fall = 0.0, rise = 0.0;  // the negative and the positive exponents' sums
+                for(int l = 0; l < nl; ++l) {
+                    const double x = src.get(__builtin_amdgcn_readfirstlane(S.col[l]), j);
+                    double e;
+                    if(l < ng) {
+                        e    = -0.5 * (x - S.p[l][0]) * (x - S.p[l][0]) * S.p[l][2];
+                        zero = zero || e < -750.0;
+                    } else if(l < ne) {
+                        e    = S.p[l][1] * (x - S.p[l][0]);
+                        zero = zero || e < -750.0;
+                    } else {
+                        const double u = (S.p[l][0] - x) * S.p[l][2];
+                        e              = S.p[l][3] * (S.p[l][4] - 2 * x);
+                        zero           = zero || e < -750.0 || u > 28.0;
+                        in             = in && u < 24.0;
+                        e              = u >= 0 ? e - u * u : e;
+                    }
+                    fall += e < 0 ? e : 0.0;
+                    rise += e < 0 ? 0.0 : e;
+                }
+                in      = in && fall > -616.0 && rise < 600.0;
+                miss[j] = __ballot(!in && !zero);
+                misses += __popcll(miss[j]);
+                E[j] = in && !zero ? E[j] : 0.0;
+                G[j] = in && !zero ? G[j] : 1.0;
             }
-            const double t = es + e, b = t - es;
-            ec += (es - (t - b)) + (e - b);
-            es = t;
-            gfmath::nll_add(s, c, g);
-            continue;
+            if(misses > GF_PROD_MISSES || notes + misses > GF_PROD_NOTES)
+                break;
+#pragma unroll
+            for(int j = 0; j < EPT; ++j) {
+                if((miss[j] >> lane) & 1)
+                    note[wave][notes + __popcll(miss[j] & ((1ull << lane) - 1ull))] = 64 * (pass * EPT + j) + lane;
+                notes += __popcll(miss[j]);
+            }
         }
-        if((threadIdx.x & 63) == 0)
-            left[wave][pass >> 5] |= 1u << (pass & 31);
+        double e = 0.0, g = 1.0;
+#pragma unroll
+        for(int j = 0; j < EPT; ++j) {
+            e += E[j];
+            g *= G[j];
+        }
+        const double t = es + e, b = t - es;
+        ec += (es - (t - b)) + (e - b);
+        es = t;
+        gfmath::nll_add(s, c, g);
+        if(++pass < npass)
+            load(base + stride, base + stride + tile <= n);
     }
-    // The tiles left over, after the loop: inside it the compiler holds the library functions'
-    // constants in vector registers throughout (187 registers, two waves on a SIMD).
-    __syncthreads();
-    for(int w = 0; w <= (pass - 1) >> 5; ++w) {
-        unsigned bits = __builtin_amdgcn_readfirstlane(left[wave][w]);
-        while(bits) {
-            const int t = 32 * w + __builtin_ctz(bits);
-            bits &= bits - 1;
-            for(int j = 0; j < EPT; ++j) {
-                const int64_t row = ((int64_t)t * gridDim.x + blockIdx.x) * tile + j * GF_BLOCK + threadIdx.x;
-                if(row >= n)
-                    continue;
-                FlatSrc<1> one;
-                double T[1];
+    // The other form, after the loop: inside it the compiler holds the library functions' constants
+    // in vector registers throughout (187 registers, two waves on a SIMD).  First the tiles from
+    // the one on at which the wave stopped, which is still in registers, then the notes.
+    for(bool kept = true; pass < npass; ++pass, kept = false) {
+        const int64_t base = base0 + pass * stride;
+        if(!kept)
+            load(base, base + tile <= n);
+        double T[EPT];
+        flat_run<EPT>(prog, P, Nm, src, T);
 #pragma unroll
-                for(int k = 0; k < GF_FLAT_COLS; ++k)
-                    one.v[0][k] = k < ncols ? cols[k][row] : 0.0;
-                flat_run<1>(prog, P, Nm, one, T);
-                gfd::nll_add(s, c, T[0], norm);
-            }
-        }
+        for(int j = 0; j < EPT; ++j)
+            if(base + j * GF_BLOCK + threadIdx.x < n)
+                gfd::nll_add(s, c, T[j], norm);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for(int i = 0; i < notes; i += 64) {
+        const unsigned id = note[wave][i + lane < notes ? i + lane : 0];
+        const int64_t row = base0 + (int64_t)(id / (64 * EPT)) * stride + id / 64 % EPT * GF_BLOCK + 64 * wave + id % 64;
+        FlatSrc<1> one;
+        double T[1];
+#pragma unroll
+        for(int k = 0; k < GF_FLAT_COLS; ++k)
+            one.v[0][k] = k < ncols ? cols[k][row] : 0.0;
+        flat_run<1>(prog, P, Nm, one, T);
+        if(i + lane < notes)
+            gfd::nll_add(s, c, T[0], norm);
     }
     s = gfd::nll_total(s, c);
     c = 0.0;
@@ -845,8 +918,7 @@ int launch_reduce_flat(const GfProgArgs &a, const GfInline *inl, int metric, int
         return -1;
     const dim3 g(nblocks), b(GF_BLOCK);
     const GfInline none{};
-    if(ept == 4 && a.flat_prod && metric == gfd::metric_nll
-       && a.nevents <= (int64_t)GF_PROD_PASSES * nblocks * GF_BLOCK * 4) {
+    if(ept == 4 && a.flat_prod && metric == gfd::metric_nll) {
         if(inl)
             hipLaunchKernelGGL((k_reduce_prod<4, true>), g, b, 0, s, a, *inl, ncols, partials);
         else
