@@ -83,6 +83,8 @@ struct DalitzNode {
     int res_func = -1;    // resolution function index
     int res_kind = GT_TRUTH;
     int res_p = 0;        // params index of the resolution's first parameter
+    GfLinePlan plan;      // its lineshapes
+    bool plan_sent = false;  // a long plan's structure is on the device
 };
 
 }  // namespace
@@ -115,7 +117,9 @@ struct gf_ctx {
     GfIns *d_ins = nullptr;
     size_t cap_params = 0, cap_consts = 0, cap_norms = 0, cap_obsid = 0, cap_ins = 0;
     GfDalitzSlot *d_dz = nullptr;
-    GfLinePlan *d_plan = nullptr;  // one per Dalitz node, then one for a stack of lineshapes (gf_tddp_gram)
+    // lineshape plans too long for a kernel's arguments: one per Dalitz node, then one for a stack
+    // of lineshapes (gf_tddp_gram)
+    GfLinePlan *d_plan = nullptr;
     GfDecay decay{};
 
     std::map<int, WaveCache> caches;
@@ -580,6 +584,59 @@ bool cursor_at(Compiler &C, int func, Cur &q) {
     return true;
 }
 
+// The structure of a lineshape plan for the n resonances in res: their terms sorted into
+// classes (GfLinePlan).  both: every resonance at (m12, m13) and again at (m13, m12), as the cache of a time-dependent node holds them.
+void line_plan(const gf_ctx *ctx, const GfResDesc *res, int n, bool both, GfLinePlan &plan) {
+    struct Entry {
+        std::array<int, 5> key;  // swap, pair, spin, norm, Gounaris-Sakurai
+        GfLineTerm term;
+    };
+    std::vector<Entry> all;
+    for(int sw = 0; sw < (both ? 2 : 1); sw++)
+        for(int i = 0; i < n; i++) {
+            const GfResDesc &r = res[i];
+            Entry e{};
+            e.key       = {both ? sw : (r.swap != 0), -1, 0, 1, r.kind == GR_GS};
+            e.term.res  = i;
+            e.term.p    = r.p;
+            e.term.kind = r.kind == GR_RBW_SYM ? GR_RBW : r.kind;
+            if(r.kind != GR_NONRES) {
+                const unsigned spin = (unsigned)ctx->consts[r.c], cyc = (unsigned)ctx->consts[r.c + 1];
+                // without spin there are no barrier factors: the flag makes no difference
+                e.key = {e.key[0], (int)std::min(cyc, 3u), (int)spin, (spin == 0 || ctx->consts[r.c + 2] != 0.0) ? 1 : 0,
+                         e.key[4]};
+                if(r.kind == GR_RBW_SYM) {  // the second half, one channel on (RBW.cu:80-81)
+                    Entry h  = e;
+                    h.key[1] = (int)((cyc + 1) % 3);
+                    all.push_back(h);
+                }
+            }
+            all.push_back(e);
+        }
+    std::stable_sort(all.begin(), all.end(), [](const Entry &a, const Entry &b) { return a.key < b.key; });
+    memset(&plan, 0, sizeof(plan));
+    std::set<std::pair<int, int>> seen;  // rows with a term already
+    for(size_t k = 0; k < all.size(); k++) {
+        const auto &key = all[k].key;
+        if(k == 0 || key != all[k - 1].key) {
+            GfLineClass &c = plan.cls[plan.nclass++];
+            c.first        = (int)k;
+            c.swap         = key[0];
+            c.pair         = key[1];
+            c.spin         = key[2];
+            c.norm         = key[3];
+            c.gs           = key[4];
+        }
+        GfLineClass &c = plan.cls[plan.nclass - 1];
+        c.count++;
+        c.res |= 1u << all[k].term.res;
+        plan.term[k]     = all[k].term;
+        plan.term[k].cls = plan.nclass - 1;
+        plan.term[k].add = seen.insert({key[0], all[k].term.res}).second ? 0 : 1;
+    }
+    plan.nterm = (int)all.size();
+}
+
 // Discover the Dalitz nodes (resonance layout, efficiency index, observable columns).
 gf_status scan_dalitz(gf_ctx *ctx) {
     ctx->dalitz.clear();
@@ -689,68 +746,56 @@ gf_status scan_dalitz(gf_ctx *ctx) {
         // Amp3Body: the last function of the subtree (Amp3Body.cu:198-202);
         // Amp3Body_TD: the root of the efficiency subtree (Amp3Body_TD.cu:518)
         d.eff_func = td ? d.eff_root : q.f - 1;
+        line_plan(ctx, d.res.data(), d.nres, d.td, d.plan);
         ctx->dalitz.push_back(d);
     }
     return GF_OK;
 }
 
-// The structure of a lineshape plan for the n resonances in res: their terms sorted into
-// classes (GfLinePlan; the numbers are filled in on the device).  both: every resonance
-// at (m12, m13) and again at (m13, m12), as the cache of a time-dependent node holds them.
-void line_plan(const gf_ctx *ctx, const GfResDesc *res, int n, bool both, GfLinePlan &plan) {
-    struct Entry {
-        std::array<int, 5> key;  // swap, pair, spin, norm, Gounaris-Sakurai
-        GfLineTerm term;
-    };
-    std::vector<Entry> all;
-    for(int sw = 0; sw < (both ? 2 : 1); sw++)
-        for(int i = 0; i < n; i++) {
-            const GfResDesc &r = res[i];
-            Entry e{};
-            e.key       = {both ? sw : (r.swap != 0), -1, 0, 1, r.kind == GR_GS};
-            e.term.res  = i;
-            e.term.p    = r.p;
-            e.term.kind = r.kind == GR_RBW_SYM ? GR_RBW : r.kind;
-            if(r.kind != GR_NONRES) {
-                const unsigned spin = (unsigned)ctx->consts[r.c], cyc = (unsigned)ctx->consts[r.c + 1];
-                // without spin there are no barrier factors: the flag makes no difference
-                e.key = {e.key[0], (int)std::min(cyc, 3u), (int)spin, (spin == 0 || ctx->consts[r.c + 2] != 0.0) ? 1 : 0,
-                         e.key[4]};
-                if(r.kind == GR_RBW_SYM) {  // the second half, one channel on (RBW.cu:80-81)
-                    Entry h  = e;
-                    h.key[1] = (int)((cyc + 1) % 3);
-                    all.push_back(h);
-                }
+// The terms of a plan that belong to the resonances in mask as a kernel's argument, with the
+// current numbers; false if they are too many.
+bool plan_in_args(const gf_ctx *ctx, const GfLinePlan &plan, uint32_t mask, GfLinePlanArg &arg) {
+    int n = 0;
+    for(int k = 0; k < plan.nterm; k++)
+        n += (mask >> plan.term[k].res) & 1u;
+    if(n > GF_ARG_TERMS)
+        return false;
+    memset(&arg, 0, sizeof(arg));
+    for(int c = 0; c < plan.nclass; c++) {
+        const GfLineClass &from = plan.cls[c];
+        if(!(from.res & mask))
+            continue;
+        GfLineClass &to = arg.cls[arg.nclass];
+        to              = from;
+        to.first        = arg.nterm;
+        to.count        = 0;
+        to.res          = from.res & mask;
+        for(int k = from.first; k < from.first + from.count; k++)
+            if((mask >> plan.term[k].res) & 1u) {
+                arg.term[arg.nterm]       = plan.term[k];
+                arg.term[arg.nterm++].cls = arg.nclass;
+                to.count++;
             }
-            all.push_back(e);
-        }
-    std::stable_sort(all.begin(), all.end(), [](const Entry &a, const Entry &b) { return a.key < b.key; });
-    memset(&plan, 0, sizeof(plan));
-    std::set<std::pair<int, int>> seen;  // rows with a term already
-    for(size_t k = 0; k < all.size(); k++) {
-        const auto &key = all[k].key;
-        if(k == 0 || key != all[k - 1].key) {
-            GfLineClass &c = plan.cls[plan.nclass++];
-            c.first        = (int)k;
-            c.swap         = key[0];
-            c.pair         = key[1];
-            c.spin         = key[2];
-            c.norm         = key[3];
-            c.gs           = key[4];
-        }
-        GfLineClass &c = plan.cls[plan.nclass - 1];
-        c.count++;
-        c.res |= 1u << all[k].term.res;
-        plan.term[k]     = all[k].term;
-        plan.term[k].cls = plan.nclass - 1;
-        plan.term[k].add = seen.insert({key[0], all[k].term.res}).second ? 0 : 1;
+        arg.nclass++;
     }
-    plan.nterm = (int)all.size();
+    for(int t = 0; t < arg.nterm; t++)
+        gfd::line_plan_term(arg, t, ctx->params.data(), ctx->decay);
+    return true;
+}
+
+// The lineshapes of node d in mask for a kernel: in arg, or the node's whole plan on the device.
+gf_status plan_ref(gf_ctx *ctx, DalitzNode &d, int slot, uint32_t mask, GfLinePlanArg &arg, GfLinePlanRef &ref) {
+    ref = {plan_in_args(ctx, d.plan, mask, arg) ? &arg : nullptr, ctx->d_plan + slot};
+    if(ref.arg || d.plan_sent)
+        return GF_OK;
+    GF_HIP(hipMemcpyAsync(ref.dev, &d.plan, sizeof(d.plan), hipMemcpyHostToDevice, ctx->stream));
+    GF_HIP(hipStreamSynchronize(ctx->stream));
+    d.plan_sent = true;
+    return GF_OK;
 }
 
 gf_status upload_dalitz_table(gf_ctx *ctx) {
     GfDalitzSlot slots[GF_MAX_DALITZ];
-    std::vector<GfLinePlan> plans(GF_MAX_DALITZ);
     memset(slots, 0, sizeof(slots));
     for(size_t s = 0; s < ctx->dalitz.size(); s++) {
         const DalitzNode &d = ctx->dalitz[s];
@@ -768,11 +813,8 @@ gf_status upload_dalitz_table(gf_ctx *ctx) {
         slots[s].col_tag    = d.col_tag;
         slots[s].res_kind   = d.res_kind;
         slots[s].res_p      = d.res_p;
-        line_plan(ctx, d.res.data(), d.nres, d.td, plans[s]);
     }
     GF_HIP(hipMemcpyAsync(ctx->d_dz, slots, sizeof(slots), hipMemcpyHostToDevice, ctx->stream));
-    GF_HIP(hipMemcpyAsync(ctx->d_plan, plans.data(), GF_MAX_DALITZ * sizeof(GfLinePlan), hipMemcpyHostToDevice,
-                          ctx->stream));
     GF_HIP(hipStreamSynchronize(ctx->stream));
     return GF_OK;
 }
@@ -1220,12 +1262,12 @@ void tiles_to_matrix(gf_ctx *ctx, const double *tiles, int nres, double *out) {
 }
 
 // Gram of the node's lineshapes over grid cells (mode 0), points (1) or its data
-// cache (2) into out (nres x nres complex).  stack/nstack (device plan of at most
-// GF_MAX_RES rows) replaces the node's lineshapes when given;
+// cache (2) into out (nres x nres complex).  stack/nstack (a plan of at most GF_MAX_RES
+// rows) replaces the node's lineshapes when given;
 // td_grid selects the time-dependent grid's m13 bin count.
-gf_status run_gram(gf_ctx *ctx, const DalitzNode &d, int slot, int mode, const double *grid6, const double *m12,
+gf_status run_gram(gf_ctx *ctx, DalitzNode &d, int slot, int mode, const double *grid6, const double *m12,
                    const double *m13, const double *w, int64_t np, int eff_func, double *out,
-                   GfLinePlan *stack = nullptr, int nstack = 0, int td_grid = 0) {
+                   const GfLinePlan *stack = nullptr, int nstack = 0, int td_grid = 0) {
     gf_status st = ensure_layout(ctx);
     if(st)
         return st;
@@ -1249,8 +1291,16 @@ gf_status run_gram(gf_ctx *ctx, const DalitzNode &d, int slot, int mode, const d
     if(st)
         return st;
     GfProgArgs a         = prog_args(ctx);
-    GfLinePlan *plan     = stack ? stack : ctx->d_plan + slot;
     const int nres       = stack ? nstack : d.nres;
+    GfLinePlanArg arg;
+    GfLinePlanRef plan{nullptr, nullptr};  // mode 2 reads the cache
+    if(stack) {  // the stream is waited for below
+        plan = {plan_in_args(ctx, *stack, ~0u, arg) ? &arg : nullptr, ctx->d_plan + GF_MAX_DALITZ};
+        if(!plan.arg)
+            GF_HIP(hipMemcpyAsync(plan.dev, stack, sizeof(*stack), hipMemcpyHostToDevice, ctx->stream));
+    } else if(mode != 2 && (st = plan_ref(ctx, d, slot, ~0u, arg, plan))) {
+        return st;
+    }
     int rc = gfk::launch_gram(a, mode, grid6, m12, m13, w, np, slot, d.col_m12, d.col_m13, eff_pc, eff_cval, td_grid,
                               plan, nres, ctx->d_gram_partials, ctx->d_gram_tiles, (int)nb, ctx->stream);
     if(rc)
@@ -2163,9 +2213,13 @@ gf_status gf_dalitz_cache(gf_ctx *ctx, int dalitz_func, uint64_t res_mask) {
     int64_t nb = (wc.n + 255) / 256;
     if(nb > (int64_t)ctx->cu_count * 8)
         nb = (int64_t)ctx->cu_count * 8;
+    GfLinePlanArg arg;
+    GfLinePlanRef plan;
+    if((st = plan_ref(ctx, *d, slot, mask, arg, plan)))
+        return st;
     GfProgArgs a = prog_args(ctx);
-    int rc = gfk::launch_dalitz_cache(a, slot, wc.offset, wc.n, mask, mask + 1 == 1u << d->nres,
-                                      ctx->d_plan + slot, (int)(nb < 1 ? 1 : nb), ctx->stream);
+    int rc = gfk::launch_dalitz_cache(a, slot, wc.offset, wc.n, mask, mask + 1 == 1u << d->nres, plan,
+                                      (int)(nb < 1 ? 1 : nb), ctx->stream);
     if(rc)
         return fail(GF_ERR_HIP, "cache launch failed (%d)", rc);
     GF_HIP(hipStreamSynchronize(ctx->stream));
@@ -2315,7 +2369,7 @@ gf_status gf_tddp_gram(gf_ctx *ctx, int tddp_func, const double grid6[6], double
     const int ng = (int)groups.size();
     std::vector<std::complex<double>> G((size_t)m * m);
     std::vector<char> have((size_t)m * m, 0);
-    GfLinePlan *dstack = ctx->d_plan + GF_MAX_DALITZ, stack_plan;
+    GfLinePlan stack;
     gf_status st = GF_OK;
     for(int u = 0; u < ng && !st; u++) {
         for(int v = (ng == 1 ? 0 : u + 1); v < ng && !st; v++) {
@@ -2330,16 +2384,11 @@ gf_status gf_tddp_gram(gf_ctx *ctx, int tddp_func, const double grid6[6], double
             std::vector<GfResDesc> st_res(idx.size());
             for(size_t k = 0; k < idx.size(); k++)
                 st_res[k] = all[idx[k]];
-            line_plan(ctx, st_res.data(), (int)st_res.size(), false, stack_plan);
-            if(hipMemcpyAsync(dstack, &stack_plan, sizeof(stack_plan), hipMemcpyHostToDevice, ctx->stream) != hipSuccess
-               || hipStreamSynchronize(ctx->stream) != hipSuccess) {
-                st = fail(GF_ERR_HIP, "copy of the Gram stack failed");
-                break;
-            }
+            line_plan(ctx, st_res.data(), (int)st_res.size(), false, stack);
             const int ns = (int)idx.size();
             std::vector<double> out(2 * (size_t)ns * ns);
             st = run_gram(ctx, *d, slot, 0, grid6, nullptr, nullptr, nullptr, (int64_t)n12 * (int64_t)n13,
-                          d->eff_func, out.data(), dstack, ns, 1);
+                          d->eff_func, out.data(), &stack, ns, 1);
             for(int i = 0; i < ns && !st; i++)
                 for(int j = 0; j < ns; j++) {
                     const size_t at = (size_t)idx[i] * m + idx[j];
@@ -2479,10 +2528,14 @@ gf_status gf_time_dalitz_cache(gf_ctx *ctx, int dalitz_func, int reps, double *m
         nb = (int64_t)ctx->cu_count * 8;
     GfProgArgs a  = prog_args(ctx);
     uint32_t mask = d->nres >= 32 ? 0xffffffffu : ((1u << d->nres) - 1u);
+    GfLinePlanArg arg;
+    GfLinePlanRef plan;
+    if((st = plan_ref(ctx, *d, slot, mask, arg, plan)))
+        return st;
     GF_HIP(hipEventRecord(ctx->ev0, ctx->stream));
     for(int r = 0; r < reps; r++) {
-        int rc = gfk::launch_dalitz_cache(a, slot, wc.offset, wc.n, mask, true, ctx->d_plan + slot,
-                                          (int)(nb < 1 ? 1 : nb), ctx->stream);
+        int rc = gfk::launch_dalitz_cache(a, slot, wc.offset, wc.n, mask, true, plan, (int)(nb < 1 ? 1 : nb),
+                                          ctx->stream);
         if(rc)
             return fail(GF_ERR_HIP, "cache launch failed (%d)", rc);
     }
@@ -3128,20 +3181,26 @@ gf_status gf_dalitz_generate(gf_ctx *ctx, int dalitz_func, int64_t n, uint64_t s
         }
     };
     double *o12 = host_out ? W.out : m12, *o13 = host_out ? W.out + n : m13;
+    GfLinePlanArg arg;
+    GfLinePlanRef plan;
+    if((st = plan_ref(ctx, *d, slot, ~0u, arg, plan))) {
+        release();
+        return st;
+    }
     GfProgArgs a = prog_args(ctx);
     const GfGenBox gbox{box[0], box[1], box[2], box[3]};
     const uint64_t key = gfd::mix64(seed ^ 0x6A09E667F3BCC909ull);
     int64_t have = 0, base = 0;
     hipStream_t s = ctx->stream;
     auto pass = [&](bool envelope, int64_t at, int64_t limit, int k) {
-        return gfk::launch_dalitz_candidates(a, ctx->d_plan + slot, d->p_coup, eff_pc, eff_cval, d->col_m12, d->col_m13,
+        return gfk::launch_dalitz_candidates(a, plan, d->p_coup, eff_pc, eff_cval, d->col_m12, d->col_m13,
                                              gbox, key, at, nb, W.state, limit, W.bits, W.count, W.bmax, s)
                    || gfk::launch_gen_scan(envelope, 0.0, W.count, W.bmax, nb, limit, W.boff, W.state, W.d_pass + k, s)
                    || (!envelope
                        && gfk::launch_compact(W.bits, gbox, key, at, nb, W.boff, limit, o12, o13, s));
     };
     const bool find = !(fmax > 0.0);
-    if(gfk::launch_line_plan(a, ctx->d_plan + slot, s)
+    if(gfk::launch_line_plan(a, plan, s)
        || gfk::launch_gen_scan(false, find ? INFINITY : fmax, nullptr, nullptr, 0, 0, nullptr, W.state, nullptr, s)
        || (find && pass(true, 0, 1, round - 1))) {
         release();

@@ -209,7 +209,7 @@ __device__ __forceinline__ bool in_dalitz(double m12, double m13, double bigM, d
 }
 
 // twoBodyCMmom, src/PDFs/physics/resonances/Resonance.cu:48-60
-__device__ __forceinline__ double two_body_cm_mom(double rMassSq, double d1m, double d2m) {
+__host__ __device__ __forceinline__ double two_body_cm_mom(double rMassSq, double d1m, double d2m) {
     double kin1 = 1 - (d1m + d2m) * (d1m + d2m) / rMassSq;
     kin1        = kin1 >= 0 ? sqrt(kin1) : 1;
     double kin2 = 1 - (d1m - d2m) * (d1m - d2m) / rMassSq;
@@ -218,7 +218,7 @@ __device__ __forceinline__ double two_body_cm_mom(double rMassSq, double d1m, do
 }
 
 // twoBodyCMMothermom, Resonance.cu:62-75
-__device__ __forceinline__ double two_body_cm_mother_mom(double rMassSq, double dm, double d3m) {
+__host__ __device__ __forceinline__ double two_body_cm_mother_mom(double rMassSq, double dm, double d3m) {
     double kin1 = 1 - (dm + d3m) * (dm + d3m) / rMassSq;
     kin1        = kin1 >= 0 ? sqrt(kin1) : 1;
     double kin2 = 1 - (dm - d3m) * (dm - d3m) / rMassSq;
@@ -229,7 +229,7 @@ __device__ __forceinline__ double two_body_cm_mother_mom(double rMassSq, double 
 // x^(2 spin + 1) for spin 0, 1, 2 by multiplication (the reference calls pow with
 // the double exponent 2 spin + 1; products differ from pow by a few ulp, far
 // inside the likelihood tolerance, and avoid FP64 pow's log/exp sequence).
-__device__ __forceinline__ double odd_power(double x, int spin) {
+__host__ __device__ __forceinline__ double odd_power(double x, int spin) {
     const double x2 = x * x;
     double r        = x;
     for(int k = 0; k < spin; ++k)
@@ -246,33 +246,34 @@ __device__ __forceinline__ double damping_factor_square(double cmmom, int spin, 
 }
 
 // dampingFactorSquareNorm, Resonance.cu:88-97
-__device__ __forceinline__ double damping_factor_square_norm(double cmmom, int spin, double mRadius) {
+__host__ __device__ __forceinline__ double damping_factor_square_norm(double cmmom, int spin, double mRadius) {
     double square  = mRadius * mRadius * cmmom * cmmom;
     double dfsq    = 1 + square;
     double dfsqres = dfsq + 8 + 2 * square + square * square;
     return (spin == 2) ? dfsqres : dfsq;
 }
 
-// hFun, dh_dsFun, fsFun, dFun: Resonance.cu:5-46 (pi truncated to 3.14159265359 as there)
-__device__ __forceinline__ double h_fun(double s, double daug2Mass, double daug3Mass) {
+// hFun, dh_dsFun, fsFun, dFun: Resonance.cu:5-46 (pi truncated to 3.14159265359 as there; the
+// logarithm is gf_math.h's, so that a plan filled in on the host has the device's bits)
+__host__ __device__ __forceinline__ double h_fun(double s, double daug2Mass, double daug3Mass) {
     const double _pi = 3.14159265359;
     double sm        = daug2Mass + daug3Mass;
     double sqrt_s    = sqrt(s);
     double k_s       = two_body_cm_mom(s, daug2Mass, daug3Mass);
-    return ((2 / _pi) * (k_s / sqrt_s) * log((sqrt_s + 2 * k_s) / (sm)));
+    return ((2 / _pi) * (k_s / sqrt_s) * gfmath::log_d((sqrt_s + 2 * k_s) / (sm)));
 }
-__device__ __forceinline__ double dh_ds_fun(double s, double daug2Mass, double daug3Mass) {
+__host__ __device__ __forceinline__ double dh_ds_fun(double s, double daug2Mass, double daug3Mass) {
     const double _pi = 3.14159265359;
     double k_s       = two_body_cm_mom(s, daug2Mass, daug3Mass);
     return h_fun(s, daug2Mass, daug3Mass) * (1.0 / (8.0 * (k_s * k_s)) - 1.0 / (2.0 * s)) + 1.0 / (2.0 * _pi * s);
 }
-__device__ __forceinline__ double d_fun(double s, double daug2Mass, double daug3Mass) {
+__host__ __device__ __forceinline__ double d_fun(double s, double daug2Mass, double daug3Mass) {
     const double _pi = 3.14159265359;
     double sm        = daug2Mass + daug3Mass;
     double sm24      = sm * sm / 4.0;
     double m         = sqrt(s);
     double k_m2      = two_body_cm_mom(s, daug2Mass, daug3Mass);
-    return 3.0 / _pi * sm24 / (k_m2 * k_m2) * log((m + 2 * k_m2) / sm) + m / (2 * _pi * k_m2)
+    return 3.0 / _pi * sm24 / (k_m2 * k_m2) * gfmath::log_d((m + 2 * k_m2) / sm) + m / (2 * _pi * k_m2)
            - sm24 * m / (_pi * (k_m2 * k_m2 * k_m2));
 }
 
@@ -286,13 +287,76 @@ __device__ __forceinline__ double d_fun(double s, double daug2Mass, double daug3
 // and F = D(q0) / D(q) (or D'(q) without normalisation), F_mother likewise.  So B =
 // kb bf and the amplitude's factor is ks sf, where bf = q^(2 spin + 1) / (D(q) sqrt(s)) and
 // sf = S / sqrt(D(q) D(p)) depend on the point only and kb, ks on the mass and width only:
-// line_class forms the former once for all resonances of a class, k_line_plan the latter
+// line_class forms the former once for all resonances of a class, line_plan_term the latter
 // once per launch, and a resonance costs one division per point.  (Evaluating each
 // shape apart took 422 FP64 operations and a dozen square roots and divisions.)
 // The momenta keep the thresholds' rules: a factor 1 - (ma + mb)^2 / s below zero is 1.
 
-// At one point: s the pair's mass squared, r = 1 / s, u = q / sqrt(s), q2 = q^2; bf and sf
-// as above.
+// The numbers of a plan's term t, with its class's and the plan's own if it is the first,
+// from the current masses, widths (P) and decay constants: the nominal-mass parts of
+// plainBW and gouSak.
+template <class Plan>
+__host__ __device__ __forceinline__ void line_plan_term(Plan &plan, int t, const double *__restrict__ P,
+                                                        const GfDecay &d) {
+    if(t == 0) {
+        const double a = d.daug2Mass + d.daug3Mass, b = d.daug2Mass - d.daug3Mass;
+        plan.m2    = d.motherMass * d.motherMass;
+        plan.rm    = d.mother_meson_radius;
+        plan.gsum2 = a * a;
+        plan.gdif2 = b * b;
+        plan.ginv  = 1.0 / a;
+    }
+    if(t >= plan.nterm)
+        return;
+    GfLineTerm &r   = plan.term[t];
+    GfLineClass &c  = plan.cls[r.cls];
+    const int pair  = c.pair, spin = c.spin;
+    if(pair < 0)
+        return;
+    const double M = d.motherMass;
+    // daughters and bachelor of the pair (RBW.cu:13-16), and the spin factor's A, B, C
+    const double da = 2 == pair ? d.daug2Mass : d.daug1Mass;
+    const double db = 0 == pair ? d.daug2Mass : d.daug3Mass;
+    const double mA = 0 == pair ? d.daug1Mass : (1 == pair ? d.daug3Mass : d.daug2Mass);
+    const double mB = 0 == pair ? d.daug2Mass : (1 == pair ? d.daug1Mass : d.daug3Mass);
+    const double mC = 0 == pair ? d.daug3Mass : (1 == pair ? d.daug2Mass : d.daug1Mass);
+    if(t == c.first) {
+        const double t1 = M * M - mC * mC, t2 = mA * mA - mB * mB;
+        c.sum2  = (da + db) * (da + db);
+        c.dif2  = (da - db) * (da - db);
+        c.mc    = mC;
+        c.msum2 = (M + mC) * (M + mC);
+        c.mdif2 = (M - mC) * (M - mC);
+        c.r2    = d.meson_radius * d.meson_radius;
+        c.rm2   = d.mother_meson_radius * d.mother_meson_radius * 0.25 / (M * M);
+        c.s0    = t1 * t2;
+        c.s1    = 2 * M * M + 2 * mC * mC;
+        c.s2    = t1 * t1;
+        c.s3    = 2 * mA * mA + 2 * mB * mB;
+        c.s4    = t2 * t2;
+    }
+    const double m  = P[r.p], w = P[r.p + 1], m2 = m * m;
+    const double q0 = two_body_cm_mom(m2, da, db);
+    double kb       = (r.kind == GR_GS ? sqrt(m2) : m2) * w / odd_power(q0, spin);
+    double ks       = 1.0;
+    if(spin != 0 && c.norm) {
+        const double p0 = two_body_cm_mother_mom(m2, M, mC);
+        const double f  = damping_factor_square_norm(q0, spin, d.meson_radius);
+        kb *= f;
+        ks = sqrt(f) * sqrt(damping_factor_square_norm(p0, spin, d.mother_meson_radius));
+    }
+    if(r.kind == GR_GS) {
+        // dFun and fsFun at the nominal mass (GS.cu:53-57)
+        const double k0 = two_body_cm_mom(m2, d.daug2Mass, d.daug3Mass);
+        ks *= 1.0 + d_fun(m2, d.daug2Mass, d.daug3Mass) * w / sqrt(m2);
+        r.f0 = w * m2 / (k0 * k0 * k0);
+        r.h0 = h_fun(m2, d.daug2Mass, d.daug3Mass);
+        r.d0 = k0 * k0 * dh_ds_fun(m2, d.daug2Mass, d.daug3Mass);
+    }
+    r.m2 = m2;
+    r.kb = kb;
+    r.ks = ks;
+}
 
 // 1 / sqrt(x) and 1 / x of a normal x > 0, to about one unit in the last place: the
 // hardware's estimate and two Newton steps.  (The barrier denominators are at least 1 and
@@ -319,7 +383,8 @@ __device__ __forceinline__ double threshold_factor(double t, double s, double r)
     return k >= 0 ? k : 1;
 }
 
-// The pair's part: s, 1 / s and the momentum (two_body_cm_mom).
+// The pair's part at one point: s the pair's mass squared, r = 1 / s and the momentum
+// (two_body_cm_mom), u = q / sqrt(s) and q2 = q^2.
 __device__ __forceinline__ void line_pair(const GfLineClass &c, double m12, double m13, double m23, double &s,
                                           double &r, double &u, double &q2) {
     s        = 0 == c.pair ? m12 : (1 == c.pair ? m13 : m23);
@@ -331,9 +396,10 @@ __device__ __forceinline__ void line_pair(const GfLineClass &c, double m12, doub
     q2 = 0.25 * s * k;
 }
 
-// The class's part: barrier and spin factors (dampingFactorSquareNorm, dampingFactorSquare
-// and spinFactor, Resonance.cu:77-155).
-__device__ __forceinline__ void line_class(const GF_CONST GfLinePlan *__restrict__ plan, const GfLineClass &c,
+// The class's part: bf and sf as above, from the barrier and spin factors
+// (dampingFactorSquareNorm, dampingFactorSquare and spinFactor, Resonance.cu:77-155).
+template <class Plan>
+__device__ __forceinline__ void line_class(const GF_CONST Plan *__restrict__ plan, const GfLineClass &c,
                                            double m12, double m13, double m23, double s, double r, double u, double q2,
                                            double &bf, double &sf) {
     bf = u;
@@ -371,14 +437,17 @@ __device__ __forceinline__ void line_class(const GF_CONST GfLinePlan *__restrict
     sf = g * f;
 }
 
+// A plan in a kernel's arguments or on the device.
+__device__ __forceinline__ const GF_CONST GfLinePlanArg *plan_at(const GfLinePlanArg &p) { return as_const(&p); }
+__device__ __forceinline__ const GF_CONST GfLinePlan *plan_at(const GfLinePlan *p) { return as_const(p); }
+
 // Every wave of the plan whose resonance is in mask (ALL: every one), at one point: emit(row, swap, add,
 // value).  m23 is the same for the swapped point (m13, m12).  All control flow is
 // uniform over the wave, and a class or term is read from the plan as a whole (one wait
 // for its scalar loads).
-template <bool ALL, class Emit>
-__device__ __forceinline__ void line_waves(const GfLinePlan *__restrict__ plan_, double m12, double m13, double m23,
+template <bool ALL, class Plan, class Emit>
+__device__ __forceinline__ void line_waves(const GF_CONST Plan *__restrict__ plan, double m12, double m13, double m23,
                                            uint32_t mask, const Emit &emit) {
-    const GF_CONST GfLinePlan *__restrict__ plan = as_const(plan_);
     double s = 0, r = 0, u = 0, q2 = 0, bf, sf;
     int chan = -1;
     for(int ci = 0; ci < plan->nclass; ++ci) {

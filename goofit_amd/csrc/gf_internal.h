@@ -83,10 +83,13 @@ struct GfResDesc {
 // same pair, spin, normalisation flag and orientation (swap) form a class: everything
 // that depends on the point and not on the mass and width (momenta, barrier factors,
 // the spin factor) is formed once per class, and a resonance adds one term (a plain or
-// Gounaris-Sakurai denominator).  The structure comes from the host with the program;
-// k_line_plan fills in the numbers from the current masses, widths and decay constants
-// before each use.
+// Gounaris-Sakurai denominator).  The structure is the program's; the numbers are
+// filled in from the current masses, widths and decay constants for each use
+// (gfd::line_plan_term).  A plan of at most GF_ARG_TERMS terms travels in the kernel
+// arguments, 3.3 KB; only a longer one is kept on the device and filled in there, by
+// k_line_plan, which costs 4 us in front of the kernel that uses it.
 #define GF_MAX_TERMS (4 * GF_MAX_RES)  // both halves of symmetrised shapes, A and B waves
+#define GF_ARG_TERMS 16
 struct GfLineClass {
     int32_t first, count;  // its terms
     int32_t pair, spin, norm, swap;  // pair -1: the non-resonant wave, 1 inside the plot
@@ -108,12 +111,21 @@ struct GfLineTerm {
     double kb, ks; // factors of the denominator's imaginary part and of the amplitude
     double f0, h0, d0;  // Gounaris-Sakurai: f(s) = f0 (k^2 (h(s) - h0) + (m^2 - s) d0)
 };
-struct GfLinePlan {
+template <int N>
+struct GfLinePlanOf {
     int32_t nclass, nterm;
     double m2, rm;              // mother mass squared, mother radius
     double gsum2, gdif2, ginv;  // Gounaris-Sakurai: (m2 + m3)^2, (m2 - m3)^2, 1 / (m2 + m3)
-    GfLineClass cls[GF_MAX_TERMS];
-    GfLineTerm term[GF_MAX_TERMS + 1];  // the last one is read ahead, never used
+    GfLineClass cls[N];
+    GfLineTerm term[N + 1];  // the last one is read ahead, never used
+};
+using GfLinePlan    = GfLinePlanOf<GF_MAX_TERMS>;
+using GfLinePlanArg = GfLinePlanOf<GF_ARG_TERMS>;
+// A plan as the launchers take it: in the arguments, numbers and all (arg), or else dev,
+// the structure alone, filled in by launch_line_plan.
+struct GfLinePlanRef {
+    const GfLinePlanArg *arg;
+    GfLinePlan *dev;
 };
 
 // Time-resolution models of a time-dependent Dalitz node.
@@ -295,10 +307,11 @@ int launch_batch_points(const GfProgArgs &a, int nres, const GfBatchWork *work, 
                         double *result, uint32_t *counter, uint32_t *stamp, void *stream);
 // Accept-reject generation in passes of nblocks x GF_GEN_BLOCK candidates of a counter-based
 // stream: candidates (accepted ones as bits, per-block counts and largest values), the scan
-// of the counts, the ordered write of the accepted.  plan: filled in by launch_line_plan.
+// of the counts, the ordered write of the accepted.  plan: filled in by launch_line_plan
+// (nothing to do where it travels in the arguments).
 // eff_pc >= 0: efficiency subprogram; -1: efficiency 1; -2: the constant eff_const.
-int launch_line_plan(const GfProgArgs &a, GfLinePlan *plan, void *stream);
-int launch_dalitz_candidates(const GfProgArgs &a, const GfLinePlan *plan, int p_coup, int eff_pc, double eff_const,
+int launch_line_plan(const GfProgArgs &a, const GfLinePlanRef &plan, void *stream);
+int launch_dalitz_candidates(const GfProgArgs &a, const GfLinePlanRef &plan, int p_coup, int eff_pc, double eff_const,
                              int id12, int id13, const GfGenBox &box, uint64_t key, int64_t base, int nblocks,
                              const GfGenState *st, int64_t limit, uint32_t *bits, int *bcount, double *bmax,
                              void *stream);
@@ -306,16 +319,16 @@ int launch_gen_scan(bool envelope, double value, const int *bcount, const double
                     int64_t *boff, GfGenState *st, GfGenPass *out, void *stream);
 int launch_compact(const uint32_t *bits, const GfGenBox &box, uint64_t key, int64_t base, int nblocks,
                    const int64_t *boff, int64_t limit, double *o12, double *o13, void *stream);
-// plan (here and in launch_gram): the lineshapes' structure; its numbers are filled in first.
-// all: mask holds every resonance of the plan.
-int launch_dalitz_cache(const GfProgArgs &a, int slot, int64_t offset, int64_t n, uint32_t mask, bool all, GfLinePlan *plan,
-                        int nblocks, void *stream);
+// plan (here and in launch_gram): the lineshapes, filled in first.  mask: the resonances
+// taken from a plan on the device (all: every one); one in the arguments holds them alone.
+int launch_dalitz_cache(const GfProgArgs &a, int slot, int64_t offset, int64_t n, uint32_t mask, bool all,
+                        const GfLinePlanRef &plan, int nblocks, void *stream);
 // mode 0: grid cells (grid6 host array); 1: points (m12, m13, w device arrays); 2: data cache of `slot`.
 // Writes 768 doubles (tiles RR, II, RI in MFMA register layout) to tiles_dev.
 // td_grid: the grid of a time-dependent node (m13 bin count grid6[5]).
 int launch_gram(const GfProgArgs &a, int mode, const double *grid6, const double *m12, const double *m13,
                 const double *w, int64_t npoints, int slot, int id_m12, int id_m13, int eff_pc, double eff_const,
-                int td_grid, GfLinePlan *plan, int nres, double *partials, double *tiles_dev, int nblocks,
+                int td_grid, const GfLinePlanRef &plan, int nres, double *partials, double *tiles_dev, int nblocks,
                 void *stream);
 // Points per workgroup pass of the Gram kernel and its workgroups per CU (LDS).
 #define GG_BLOCK 256

@@ -9,82 +9,25 @@
 //  * k_dalitz_candidates / k_compact: accept-reject generation from an Amp3Body.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "gf_interp.h"
 
 namespace {
 
 // ------------------------------------------------------------- Dalitz cache
 
-// The numbers of a lineshape plan from the current masses, widths and decay constants,
-// one lane per term (GfLinePlan; the nominal-mass parts of plainBW and gouSak).
+// The numbers of a plan kept on the device, one lane per term.
 __global__ __launch_bounds__(GF_MAX_TERMS) void k_line_plan(GfLinePlan *plan, const double *__restrict__ P, GfDecay d) {
-    const int t = threadIdx.x;
-    if(t == 0) {
-        const double a = d.daug2Mass + d.daug3Mass, b = d.daug2Mass - d.daug3Mass;
-        plan->m2    = d.motherMass * d.motherMass;
-        plan->rm    = d.mother_meson_radius;
-        plan->gsum2 = a * a;
-        plan->gdif2 = b * b;
-        plan->ginv  = 1.0 / a;
-    }
-    if(t >= plan->nterm)
-        return;
-    GfLineTerm &r   = plan->term[t];
-    GfLineClass &c  = plan->cls[r.cls];
-    const int pair  = c.pair, spin = c.spin;
-    if(pair < 0)
-        return;
-    const double M = d.motherMass;
-    // daughters and bachelor of the pair (RBW.cu:13-16), and the spin factor's A, B, C
-    const double da = 2 == pair ? d.daug2Mass : d.daug1Mass;
-    const double db = 0 == pair ? d.daug2Mass : d.daug3Mass;
-    const double mA = 0 == pair ? d.daug1Mass : (1 == pair ? d.daug3Mass : d.daug2Mass);
-    const double mB = 0 == pair ? d.daug2Mass : (1 == pair ? d.daug1Mass : d.daug3Mass);
-    const double mC = 0 == pair ? d.daug3Mass : (1 == pair ? d.daug2Mass : d.daug1Mass);
-    if(t == c.first) {
-        const double t1 = M * M - mC * mC, t2 = mA * mA - mB * mB;
-        c.sum2  = (da + db) * (da + db);
-        c.dif2  = (da - db) * (da - db);
-        c.mc    = mC;
-        c.msum2 = (M + mC) * (M + mC);
-        c.mdif2 = (M - mC) * (M - mC);
-        c.r2    = d.meson_radius * d.meson_radius;
-        c.rm2   = d.mother_meson_radius * d.mother_meson_radius * 0.25 / (M * M);
-        c.s0    = t1 * t2;
-        c.s1    = 2 * M * M + 2 * mC * mC;
-        c.s2    = t1 * t1;
-        c.s3    = 2 * mA * mA + 2 * mB * mB;
-        c.s4    = t2 * t2;
-    }
-    const double m  = P[r.p], w = P[r.p + 1], m2 = m * m;
-    const double q0 = gfd::two_body_cm_mom(m2, da, db);
-    double kb       = (r.kind == GR_GS ? sqrt(m2) : m2) * w / gfd::odd_power(q0, spin);
-    double ks       = 1.0;
-    if(spin != 0 && c.norm) {
-        const double p0 = gfd::two_body_cm_mother_mom(m2, M, mC);
-        const double f  = gfd::damping_factor_square_norm(q0, spin, d.meson_radius);
-        kb *= f;
-        ks = sqrt(f) * sqrt(gfd::damping_factor_square_norm(p0, spin, d.mother_meson_radius));
-    }
-    if(r.kind == GR_GS) {
-        // dFun and fsFun at the nominal mass (GS.cu:53-57)
-        const double k0 = gfd::two_body_cm_mom(m2, d.daug2Mass, d.daug3Mass);
-        ks *= 1.0 + gfd::d_fun(m2, d.daug2Mass, d.daug3Mass) * w / sqrt(m2);
-        r.f0 = w * m2 / (k0 * k0 * k0);
-        r.h0 = gfd::h_fun(m2, d.daug2Mass, d.daug3Mass);
-        r.d0 = k0 * k0 * gfd::dh_ds_fun(m2, d.daug2Mass, d.daug3Mass);
-    }
-    r.m2 = m2;
-    r.kb = kb;
-    r.ks = ks;
+    gfd::line_plan_term(*plan, threadIdx.x, P, d);
 }
 
 // The wave cache (ALL: every resonance).  16 shapes over 1e6 events: 58 us, 1045 vector
 // instructions per wave of 64 events (29 us of issue) beside 256 MB of stores (40 us at the
 // fill rate); 290 us with each shape evaluated by itself.
-template <bool ALL>
+template <bool ALL, class Plan>
 __global__ __launch_bounds__(256) void k_dalitz_cache(GfProgArgs A, int slot, int64_t offset, int64_t n, uint32_t mask,
-                                                      const GfLinePlan *__restrict__ plan) {
+                                                      const Plan plan) {
     const GfDalitzSlot dz = gfd::as_const(A.dz)[slot];
     const GfDecay D       = A.decay;
     double2 *wave         = const_cast<double2 *>(dz.wave);
@@ -99,7 +42,7 @@ __global__ __launch_bounds__(256) void k_dalitz_cache(GfProgArgs A, int slot, in
         // same m23 (SpecialWaveCalculator.cu:55-58)
         const double m23 = D.motherMass * D.motherMass + D.daug1Mass * D.daug1Mass + D.daug2Mass * D.daug2Mass
                            + D.daug3Mass * D.daug3Mass - m12 - m13;
-        gfd::line_waves<ALL>(plan, m12, m13, m23, mask, [&](int i, int swap, int add, double2 v) {
+        gfd::line_waves<ALL>(gfd::plan_at(plan), m12, m13, m23, mask, [&](int i, int swap, int add, double2 v) {
             double2 *w = (swap ? wave_b : wave) + (int64_t)i * dz.ncache + e;
             if(add) {
                 v.x += w->x;
@@ -128,8 +71,8 @@ __device__ __forceinline__ void gen_point(const GfGenBox &B, uint64_t key, uint6
 // Out: the accepted candidates as bits, their number and the largest value (to check the
 // envelope).  Nothing is done once st->have has reached limit.  A pass of 2^22 candidates
 // with 16 shapes: 126 us; 208 us with every candidate evaluated in its own lane.
-template <bool GEN_EFF>
-__global__ __launch_bounds__(256) void k_dalitz_candidates(GfProgArgs A, const GfLinePlan *__restrict__ plan,
+template <bool GEN_EFF, class Plan>
+__global__ __launch_bounds__(256) void k_dalitz_candidates(GfProgArgs A, const Plan plan,
                                                            int p_coup, int eff_pc, double eff_const, int id12,
                                                            int id13, GfGenBox B, uint64_t key, int64_t base,
                                                            const GfGenState *__restrict__ st, int64_t limit,
@@ -177,7 +120,7 @@ __global__ __launch_bounds__(256) void k_dalitz_candidates(GfProgArgs A, const G
         const double m23 = D.motherMass * D.motherMass + D.daug1Mass * D.daug1Mass + D.daug2Mass * D.daug2Mass
                            + D.daug3Mass * D.daug3Mass - m12 - m13;
         double re = 0.0, im = 0.0;
-        gfd::line_waves<true>(plan, m12, m13, m23, ~0u, [&](int r, int, int, double2 b) {
+        gfd::line_waves<true>(gfd::plan_at(plan), m12, m13, m23, ~0u, [&](int r, int, int, double2 b) {
             const double ar = P[2 * r], ai = P[2 * r + 1];
             re = fma(ar, b.x, fma(-ai, b.y, re));
             im = fma(ar, b.y, fma(ai, b.x, im));
@@ -372,9 +315,9 @@ __global__ __launch_bounds__(256) void k_dalitz_cells(GramSrc S, double *m12, do
 // (40 us of vector and 24 us of matrix-core issue; the 16.5 KB of LDS per wave leave two
 // waves per SIMD, so latency shows), 450-520 us with each shape evaluated by itself over
 // every cell.  Partials: 3 tiles x 64 lanes x 4 values per block.
-template <bool GEN_EFF>
+template <bool GEN_EFF, class Plan>
 __global__ __launch_bounds__(GG_BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void k_gram(
-    GfProgArgs A, GramSrc S, const GfLinePlan *__restrict__ plan, int nres, double *partials) {
+    GfProgArgs A, GramSrc S, const Plan plan, int nres, double *partials) {
     __shared__ double Xr[GG_BLOCK / 64][16][GG_LD];
     __shared__ double Xi[GG_BLOCK / 64][16][GG_LD];
     __shared__ double Ew[GG_BLOCK / 64][64];
@@ -412,7 +355,7 @@ __global__ __launch_bounds__(GG_BLOCK) __attribute__((amdgpu_waves_per_eu(2))) v
                 continue;
             const double m23  = D.motherMass * D.motherMass + D.daug1Mass * D.daug1Mass + D.daug2Mass * D.daug2Mass
                                + D.daug3Mass * D.daug3Mass - m12 - m13;
-            gfd::line_waves<true>(plan, m12, m13, m23, ~0u, [&](int i, int, int add, double2 b) {
+            gfd::line_waves<true>(gfd::plan_at(plan), m12, m13, m23, ~0u, [&](int i, int, int add, double2 b) {
                 if(add) {
                     b.x += Xr[wave][i][lane];
                     b.y += Xi[wave][i][lane];
@@ -512,26 +455,35 @@ __global__ __launch_bounds__(256) void k_gram_final(const double *__restrict__ p
 
 namespace gfk {
 
-static int fill_plan(const GfProgArgs &a, GfLinePlan *plan, hipStream_t s) {
-    hipLaunchKernelGGL(k_line_plan, dim3(1), dim3(GF_MAX_TERMS), 0, s, plan, a.params, a.decay);
+int launch_line_plan(const GfProgArgs &a, const GfLinePlanRef &plan, void *stream) {
+    if(plan.arg)
+        return 0;
+    hipLaunchKernelGGL(k_line_plan, dim3(1), dim3(GF_MAX_TERMS), 0, (hipStream_t)stream, plan.dev, a.params, a.decay);
     return check(hipGetLastError());
 }
 
-
-int launch_line_plan(const GfProgArgs &a, GfLinePlan *plan, void *stream) {
-    return fill_plan(a, plan, (hipStream_t)stream);
+// f(plan) with the plan in the form in which the kernels take it.
+template <class F>
+static void with_plan(const GfLinePlanRef &plan, const F &f) {
+    if(plan.arg)
+        f(*plan.arg);
+    else
+        f((const GfLinePlan *)plan.dev);
 }
 
-int launch_dalitz_candidates(const GfProgArgs &a, const GfLinePlan *plan, int p_coup, int eff_pc, double eff_const,
+int launch_dalitz_candidates(const GfProgArgs &a, const GfLinePlanRef &plan, int p_coup, int eff_pc, double eff_const,
                              int id12, int id13, const GfGenBox &box, uint64_t key, int64_t base, int nblocks,
                              const GfGenState *st, int64_t limit, uint32_t *bits, int *bcount, double *bmax,
                              void *stream) {
-    if(eff_pc >= 0)
-        hipLaunchKernelGGL(k_dalitz_candidates<true>, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, a, plan,
-                           p_coup, eff_pc, eff_const, id12, id13, box, key, base, st, limit, bits, bcount, bmax);
-    else
-        hipLaunchKernelGGL(k_dalitz_candidates<false>, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, a, plan,
-                           p_coup, eff_pc, eff_const, id12, id13, box, key, base, st, limit, bits, bcount, bmax);
+    with_plan(plan, [&](const auto &p) {
+        using Plan = std::decay_t<decltype(p)>;
+        if(eff_pc >= 0)
+            hipLaunchKernelGGL((k_dalitz_candidates<true, Plan>), dim3(nblocks), dim3(256), 0, (hipStream_t)stream, a, p,
+                               p_coup, eff_pc, eff_const, id12, id13, box, key, base, st, limit, bits, bcount, bmax);
+        else
+            hipLaunchKernelGGL((k_dalitz_candidates<false, Plan>), dim3(nblocks), dim3(256), 0, (hipStream_t)stream, a, p,
+                               p_coup, eff_pc, eff_const, id12, id13, box, key, base, st, limit, bits, bcount, bmax);
+    });
     return check(hipGetLastError());
 }
 
@@ -549,23 +501,26 @@ int launch_compact(const uint32_t *bits, const GfGenBox &box, uint64_t key, int6
     return check(hipGetLastError());
 }
 
-int launch_dalitz_cache(const GfProgArgs &a, int slot, int64_t offset, int64_t n, uint32_t mask, bool all, GfLinePlan *plan,
-                        int nblocks, void *stream) {
-    int rc = fill_plan(a, plan, (hipStream_t)stream);
+int launch_dalitz_cache(const GfProgArgs &a, int slot, int64_t offset, int64_t n, uint32_t mask, bool all,
+                        const GfLinePlanRef &plan, int nblocks, void *stream) {
+    hipStream_t s = (hipStream_t)stream;
+    const dim3 g(nblocks), b(256);
+    const GfLinePlan *dev = plan.dev;
+    const int rc          = launch_line_plan(a, plan, stream);
     if(rc)
         return rc;
-    if(all)
-        hipLaunchKernelGGL(k_dalitz_cache<true>, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, a, slot, offset, n,
-                           mask, plan);
+    if(plan.arg)
+        hipLaunchKernelGGL((k_dalitz_cache<true, GfLinePlanArg>), g, b, 0, s, a, slot, offset, n, mask, *plan.arg);
+    else if(all)
+        hipLaunchKernelGGL((k_dalitz_cache<true, const GfLinePlan *>), g, b, 0, s, a, slot, offset, n, mask, dev);
     else
-        hipLaunchKernelGGL(k_dalitz_cache<false>, dim3(nblocks), dim3(256), 0, (hipStream_t)stream, a, slot, offset, n,
-                           mask, plan);
+        hipLaunchKernelGGL((k_dalitz_cache<false, const GfLinePlan *>), g, b, 0, s, a, slot, offset, n, mask, dev);
     return check(hipGetLastError());
 }
 
 int launch_gram(const GfProgArgs &a, int mode, const double *grid6, const double *m12, const double *m13,
                 const double *w, int64_t npoints, int slot, int id_m12, int id_m13, int eff_pc, double eff_const,
-                int td_grid, GfLinePlan *plan, int nres, double *partials, double *tiles_dev, int nblocks,
+                int td_grid, const GfLinePlanRef &plan, int nres, double *partials, double *tiles_dev, int nblocks,
                 void *stream) {
     GramSrc S;
     S.mode = mode;
@@ -590,13 +545,16 @@ int launch_gram(const GfProgArgs &a, int mode, const double *grid6, const double
     S.eff_pc    = eff_pc;
     S.eff_const = eff_const;
     hipStream_t s = (hipStream_t)stream;
-    int rc = mode == 2 ? 0 : fill_plan(a, plan, s);
+    int rc = mode == 2 ? 0 : launch_line_plan(a, plan, s);
     if(rc)
         return rc;
-    if(eff_pc >= 0)
-        hipLaunchKernelGGL(k_gram<true>, dim3(nblocks), dim3(GG_BLOCK), 0, s, a, S, plan, nres, partials);
-    else
-        hipLaunchKernelGGL(k_gram<false>, dim3(nblocks), dim3(GG_BLOCK), 0, s, a, S, plan, nres, partials);
+    with_plan(plan, [&](const auto &p) {
+        using Plan = std::decay_t<decltype(p)>;
+        if(eff_pc >= 0)
+            hipLaunchKernelGGL((k_gram<true, Plan>), dim3(nblocks), dim3(GG_BLOCK), 0, s, a, S, p, nres, partials);
+        else
+            hipLaunchKernelGGL((k_gram<false, Plan>), dim3(nblocks), dim3(GG_BLOCK), 0, s, a, S, p, nres, partials);
+    });
     if((rc = check(hipGetLastError())))
         return rc;
     hipLaunchKernelGGL(k_gram_final, dim3(768 / 8), dim3(256), 0, s, partials, nblocks, tiles_dev);

@@ -5,6 +5,8 @@ time-dependent waves.
 Tolerance: a wave is a product of a dozen correctly rounded factors, so engine and oracle
 agree to some 1e-15 relative except where the pair's threshold factor 1 - (ma + mb)^2 / s
 cancels, which multiplies the rounding by s / (s - (ma + mb)^2): below 1e3 on these samples."""
+import time
+
 import numpy as np
 import pytest
 
@@ -25,6 +27,10 @@ SHAPES = {
     "gs": [("GS", 0.7758, 0.15, s, p, True) for s in (0, 1, 2) for p in (0, 1, 2)] + [("NONRES", 0, 0, 0, 0, True)],
     "symmetrised": [("SYM", 0.9, 0.1, s, p, n) for s in (0, 1, 2) for p in (0, 2) for n in (True, False)],
     "one": [("NONRES", 0, 0, 0, 0, True)],
+    # a plan's terms in the kernels' arguments, 16 of them, and one more
+    "args": [("RBW", 0.7 + 0.05 * k, 0.1, k % 3, k % 3, True) for k in range(14)] + [("SYM", 0.9, 0.1, 1, 0, True)],
+    "args and one": [("GS", 0.7758, 0.15, 1, 2, True)] + [("RBW", 0.7 + 0.05 * k, 0.1, k % 3, k % 3, True) for k in range(14)]
+    + [("SYM", 0.9, 0.1, 1, 0, True)],
 }
 
 
@@ -110,7 +116,9 @@ def test_waves_and_integrals(ctx, shapes, decay):
 
 @pytest.mark.parametrize("shapes", ["spins", "gs", "symmetrised"])
 def test_time_dependent_waves(ctx, shapes):
-    """The B waves: every lineshape at the reversed point (a pair below its threshold there)."""
+    """The B waves: every lineshape at the reversed point (a pair below its threshold there).  Alone,
+    a resonance's terms are in the kernel's arguments, with the others on the device: the same
+    bits."""
     n, decay = 1000, UNEQUAL
     top, res = _model(SHAPES[shapes], decay, td=True)
     m12, m13 = _events(n, decay, 5)
@@ -128,6 +136,12 @@ def test_time_dependent_waves(ctx, shapes):
         a, b = M.op.tddp_wave(0, f, aos)
         _close(ctx.dalitz_get_cache(0, i, n), a)
         _close(ctx.dalitz_get_cache(0, len(funcs) + i, n), b)
+    before = [ctx.dalitz_get_cache(0, i, n) for i in range(2 * len(funcs))]
+    ctx.dalitz_set_data_size(0, n)
+    for i in range(len(funcs)):
+        ctx.dalitz_cache(0, 1 << i)
+    for i, w in enumerate(before):
+        assert np.array_equal(ctx.dalitz_get_cache(0, i, n), w)
 
 
 def _mix64(z):
@@ -190,3 +204,28 @@ def test_generated_events_are_the_stream(ctx):
         ctx.dalitz_generate(0, 10, seed, [2.95, 3.0, 2.95, 3.0])
     a2, b2, _, _ = ctx.dalitz_generate(0, 777, seed, box, fmax)
     assert np.array_equal(a2, m12[keep[:777]]) and np.array_equal(b2, m13[keep[:777]])
+
+
+def test_refresh_of_one_resonance_is_not_slow(ctx):
+    """One resonance of sixteen over a small sample is the work of a model's only one: what is
+    prepared for a call must not grow with the others (a sixth more with all of their constants
+    formed on the device in front of it)."""
+    us = {}
+    for nres in (1, 16) * 3:
+        top, _ = _model([("RBW", 0.7 + 0.05 * k, 0.1, k % 3, k % 3, True) for k in range(nres)], EQUAL)
+        n = 1000
+        m12, m13 = _events(n, EQUAL, 3)
+        M = O.Model(top, np.zeros((1, 3)), decay=EQUAL)
+        M.op.sync_params()
+        ctx.set_program(*M.op.prog.arrays())
+        ctx.set_decay(EQUAL)
+        ctx.upload_columns([m12, m13, np.arange(n, dtype=np.float64)])
+        ctx.set_identity_column(2)
+        ctx.dalitz_set_data_size(0, n)
+        t = []
+        for _ in range(200):
+            a = time.perf_counter()
+            ctx.dalitz_cache(0, 1)
+            t.append(time.perf_counter() - a)
+        us[nres] = min(us.get(nres, np.inf), 1e6 * np.median(t))
+    assert us[16] <= 1.08 * us[1], us
