@@ -27,8 +27,9 @@
 
 // Instruction codes of the compiled program.  Leaf codes compute T; the
 // combining steps act on the accumulator of one nesting level and are encoded
-// as GI_LVL + 4*kind + level, so each (kind, level) pair is its own case with
-// the accumulator fixed at compile time (no register array indexed at run time).
+// as GI_LVL + 4*kind + level: a sum's or product's (kind, level) pair is its own case
+// with the accumulator fixed at compile time, a Dalitz node takes its level's by
+// selects (no register array is indexed at run time either way).
 enum GfOp : int32_t {
     GI_END = 0,
     GI_GAUSS,          // T = exp(-0.5*(x-m)*(x-m)/(s*s))

@@ -52,10 +52,14 @@ struct RegSrc {
     }
 };
 
-// Per-level accumulators of the combining nodes: the current level's, taken and put back
-// by selects on the wave-uniform level, so that each node kind is compiled once and not
-// once per level (four copies of the time-dependent node had 960 scalar registers spilled
-// to vector lanes).
+// Per-level accumulators of the combining nodes.  The few operations of a sum or product are a
+// case per level, on that level's registers.  A Dalitz node is compiled once, its level's
+// accumulator taken and put back by selects on the wave-uniform level (four copies of the
+// time-dependent node had 960 scalar registers spilled to vector lanes); with selects for
+// sums and products too, trees three levels deep took a seventh longer (1000 events 23.0 us,
+// 20.4 as cases; an integral over 2e5 cells 30.4 and 25.8), with a switch on the level and one
+// on the kind 21.7 and 27.4.  The time-dependent kernels keep the selects: the
+// cases spill there (3e5 events 57.6 us, 59.4 as cases).
 template <int EPT>
 struct Acc {
     double v[4][EPT];
@@ -75,15 +79,10 @@ struct Acc {
 
 // ------------------------------------------------------------ interpreter
 
-// One combining step on the accumulator a of its level.  FEAT: the node kinds compiled
-// in -- 0 none of the Dalitz nodes, 1 the time-integrated Dalitz node, 2 also the
-// time-dependent one -- so that each kernel carries only the register budget of
-// the programs it runs (a Dalitz node met by a kernel without it sets bit 1 of
-// the error word instead of being skipped silently).
-template <int EPT, int FEAT, class Src>
-__device__ __forceinline__ void step(int kind, const GfIns &in, const GfProgArgs &A, const GF_CONST double *__restrict__ P,
-                                     const GF_CONST double *__restrict__ Nm, const Src &src, const int64_t (&row)[EPT],
-                                     const bool (&valid)[EPT], double (&a)[EPT], double (&T)[EPT]) {
+// One step of a sum or product on the accumulator a of its level.
+template <int EPT>
+__device__ __forceinline__ void sum_step(int kind, const GfIns &in, const GF_CONST double *__restrict__ P,
+                                         const GF_CONST double *__restrict__ Nm, double (&a)[EPT], double (&T)[EPT]) {
     switch(kind) {
     case GK_PUSH0:
 #pragma unroll
@@ -135,6 +134,23 @@ __device__ __forceinline__ void step(int kind, const GfIns &in, const GfProgArgs
         for(int j = 0; j < EPT; ++j)
             T[j] = a[j];
         break;
+    default: break;
+    }
+}
+
+// One step of a Dalitz node (or of a sum or product, where no case of its own takes it) on the
+// accumulator a of its level.  FEAT: the node kinds compiled
+// in -- 0 none of the Dalitz nodes, 1 the time-integrated Dalitz node, 2 also the
+// time-dependent one -- so that each kernel carries only the register budget of
+// the programs it runs (a Dalitz node met by a kernel without it sets bit 1 of
+// the error word instead of being skipped silently).
+template <int EPT, int FEAT, class Src>
+__device__ __forceinline__ void node_step(int kind, const GfIns &in, const GfProgArgs &A,
+                                          const GF_CONST double *__restrict__ P,
+                                          const GF_CONST double *__restrict__ Nm, const Src &src,
+                                          const int64_t (&row)[EPT], const bool (&valid)[EPT], double (&a)[EPT],
+                                          double (&T)[EPT]) {
+    switch(kind) {
     case GK_DALITZ: {
         if constexpr(FEAT < 1) {
             atomicOr(A.err, 2);
@@ -297,7 +313,7 @@ __device__ __forceinline__ void step(int kind, const GfIns &in, const GfProgArgs
             atomicOr(A.err, 2);
         }
         break;
-    default: break;
+    default: sum_step<EPT>(kind, in, P, Nm, a, T); break;
     }
 }
 
@@ -319,7 +335,8 @@ __device__ __forceinline__ void run(const GfProgArgs &A, const double *__restric
         T[j] = acc.v[0][j] = acc.v[1][j] = acc.v[2][j] = acc.v[3][j] = 0.0;
     for(int pc = pc0;; ++pc) {
         const GfIns in = prog[pc];
-        switch(in.op) {
+        // the time-dependent kernels take every level's step by the default case
+        switch(FEAT == 2 && in.op >= GI_LVL ? GF_LVL_OP(GK_DALITZ, 0) : in.op) {
         case GI_END: return;
         case GI_GAUSS: {
             const double m = P[in.p], s = P[in.p + 1];
@@ -424,12 +441,26 @@ __device__ __forceinline__ void run(const GfProgArgs &A, const double *__restric
                 T[j] = r;
             }
         } break;
+#define GF_SUM_CASE(k)                                                     \
+    case GF_LVL_OP(k, 0): sum_step<EPT>(k, in, P, Nm, acc.v[0], T); break; \
+    case GF_LVL_OP(k, 1): sum_step<EPT>(k, in, P, Nm, acc.v[1], T); break; \
+    case GF_LVL_OP(k, 2): sum_step<EPT>(k, in, P, Nm, acc.v[2], T); break; \
+    case GF_LVL_OP(k, 3): sum_step<EPT>(k, in, P, Nm, acc.v[3], T); break;
+            GF_SUM_CASE(GK_PUSH0)
+            GF_SUM_CASE(GK_PUSH1)
+            GF_SUM_CASE(GK_ADD_ACC)
+            GF_SUM_CASE(GK_ADD_LAST)
+            GF_SUM_CASE(GK_ADDEXT_END)
+            GF_SUM_CASE(GK_PROD_ACC)
+            GF_SUM_CASE(GK_POP)
+#undef GF_SUM_CASE
         default:
             if(in.op >= GI_LVL) {
+                const int kind = (in.op - GI_LVL) >> 2, lvl = (in.op - GI_LVL) & 3;
                 double a[EPT];
-                acc.take((in.op - GI_LVL) & 3, a);
-                step<EPT, FEAT>((in.op - GI_LVL) >> 2, in, A, P, Nm, src, row, valid, a, T);
-                acc.put((in.op - GI_LVL) & 3, a);
+                acc.take(lvl, a);
+                node_step<EPT, FEAT>(kind, in, A, P, Nm, src, row, valid, a, T);
+                acc.put(lvl, a);
                 break;
             }
             return;

@@ -319,3 +319,46 @@ def test_nll_with_subnormal_and_zero_pdf_values(ctx):
         ctx.set_tuning(capi.TUNE_FUSED_FINISH, 1)
     assert len(set(got.values())) == 1, got
     assert math.isclose(got[1, 1][0], ref, rel_tol=NLL_RTOL), (got[1, 1], ref)
+
+
+def _nested(kinds, x, y, k=0):
+    """A tree of len(kinds) levels: the first child of each node is the next level's, the
+    second a leaf.  S a sum with fractions, E one with yields, P a product."""
+    v = lambda name, value: O.Var(f"{name}{k}", value)
+    leaf = lambda i: (O.Exp(f"e{k}_{i}", x, O.Var(f"a{k}_{i}", -0.3 - 0.1 * i)) if (k + i) % 2
+                      else O.Gaussian(f"g{k}_{i}", y, O.Var(f"m{k}_{i}", 0.1), O.Var(f"s{k}_{i}", 0.9 + 0.1 * k)))
+    if not kinds:
+        return leaf(0)
+    parts = [_nested(kinds[1:], x, y, k + 1), leaf(1), leaf(2)]
+    if kinds[0] == "P":
+        return O.Prod(f"p{k}", parts[:2])
+    if kinds[0] == "S":
+        return O.Add(f"s{k}", [v("f", 0.3), v("h", 0.25)], parts)
+    return O.Add(f"t{k}", [v("n", 40.0), v("b", 60.0)], parts[:2])
+
+
+@pytest.mark.parametrize("kinds", ["SPSP", "PSPS", "EPEP", "PEPE", "SSSS", "EEEE", "PPPP", "SEP", "PS", "E"])
+def test_every_level_of_sums_and_products(ctx, kinds):
+    """Sums of both kinds and products on each of the four levels, by event, summed and on a grid,
+    with norms other than 1: a value is some 20 products and sums of positive terms, each within a
+    unit in the last place or two."""
+    rng = np.random.default_rng(len(kinds))
+    x, y = O.Obs("x", -2.0, 3.0, 40), O.Obs("y", -3.0, 3.0, 50)
+    f, p, c, o, n = arrays(_nested(kinds, x, y))[1]
+    n = n * rng.uniform(0.5, 2.0, n.size)
+    n[0::2] = 1.0
+    prog = O.RawProg(f, p, c, o, n)
+    aos = np.stack([rng.uniform(-2.0, 3.0, 777), rng.uniform(-3.0, 3.0, 777)], 1)
+    ncols = int(o[0])
+    aos = np.ascontiguousarray(aos[:, :ncols])
+    ctx.set_program(f, p, c, o, n)
+    ctx.upload_columns([np.ascontiguousarray(aos[:, k]) for k in range(ncols)])
+    np.testing.assert_allclose(ctx.eval_metric("PROB"), prog.eval_metric(aos, "PROB"), rtol=2e-14)
+    ctx.set_tuning(capi.TUNE_FLAT, 0)
+    try:
+        assert math.isclose(ctx.reduce_metric("NLL")[0], prog.reduce_metric(aos, "NLL"), rel_tol=NLL_RTOL)
+    finally:
+        ctx.set_tuning(capi.TUNE_FLAT, 1)
+    if ncols == 2:
+        ranges = [-2.0, 3.0, 40, -3.0, 3.0, 50]
+        assert math.isclose(ctx.reduce_bins(0, ranges), prog.reduce_bins(0, ranges), rel_tol=1e-12)
