@@ -313,7 +313,10 @@ __device__ __forceinline__ void node_step(int kind, const GfIns &in, const GfPro
             atomicOr(A.err, 2);
         }
         break;
-    default: sum_step<EPT>(kind, in, P, Nm, a, T); break;
+    default:
+        if constexpr(FEAT == 2)
+            sum_step<EPT>(kind, in, P, Nm, a, T);
+        break;
     }
 }
 
@@ -455,12 +458,11 @@ __device__ __forceinline__ void run(const GfProgArgs &A, const double *__restric
             GF_SUM_CASE(GK_POP)
 #undef GF_SUM_CASE
         default:
-            if(in.op >= GI_LVL) {
-                const int kind = (in.op - GI_LVL) >> 2, lvl = (in.op - GI_LVL) & 3;
+            if(in.op >= (FEAT == 2 ? GI_LVL : GF_LVL_OP(GK_DALITZ, 0))) {
                 double a[EPT];
-                acc.take(lvl, a);
-                node_step<EPT, FEAT>(kind, in, A, P, Nm, src, row, valid, a, T);
-                acc.put(lvl, a);
+                acc.take((in.op - GI_LVL) & 3, a);
+                node_step<EPT, FEAT>((in.op - GI_LVL) >> 2, in, A, P, Nm, src, row, valid, a, T);
+                acc.put((in.op - GI_LVL) & 3, a);
                 break;
             }
             return;
