@@ -103,8 +103,9 @@ GF_MATH_HD inline void nll_add(double &m, int &e, double v) {
 GF_MATH_HD inline double nll_total(double m, double e) { return -fma(e, ln2_hi, fma(e, ln2_lo, log_d(m))); }
 
 // Powers x^n, x^(n+1), ... of the polynomials, each within half a unit in the last place and
-// some 2^-100 (the power kept as an unevaluated sum h + l): five operations a power, where
-// the library's pow, which knows nothing of whole exponents, takes some 200 each time.
+// some 2^-100 (the power kept as an unevaluated sum h + l): six operations a power, a sum and a
+// select for its value, where the library's pow, which knows nothing of whole exponents, takes
+// some 200 each time.
 // Where l is no number (overflow, infinite x) h alone is the power, as pow gives it.
 struct Powers {
     double h = 1.0, l = 0.0;
@@ -117,7 +118,10 @@ struct Powers {
     // from x^0 to x^n by squarings: any exponent in at most 32 steps
     GF_MATH_HD void start(double x, unsigned n) {
         Powers b;
-        b.next(x);
+        b.h = x;
+        start(b, n);
+    }
+    GF_MATH_HD void start(Powers b, unsigned n) {
         while(n) {
             if(n & 1) {
                 times(b.h, b.l);
@@ -149,15 +153,17 @@ GF_MATH_HD inline double power(double x, int n) {
         p.next(x);
     return p.value();
 }
-// x^n of any whole n, uniform over the wave; a negative one as the reciprocal of h + l.
+// x^n of any whole n, uniform over the wave; a negative one from the reciprocal, kept as h + l
+// too (the reciprocal of x^-n is 0 once that overflows, where x^n may be subnormal yet).
 GF_MATH_HD inline double powi(double x, int n) {
-    Powers p;
-    p.start(x, n < 0 ? 0u - (unsigned)n : (unsigned)n);
-    if(n >= 0)
-        return p.value();
-    const double r = 1.0 / p.h;
-    const double t = fma(r, fma(-p.h, r, 1.0) - p.l * r, r);
-    return t == t ? t : r;
+    Powers p, b;
+    b.h = x;
+    if(n < 0) {
+        b.h = 1.0 / x;
+        b.l = fma(-x, b.h, 1.0) * b.h;
+    }
+    p.start(b, n < 0 ? 0u - (unsigned)n : (unsigned)n);
+    return p.value();
 }
 
 // exp(x), N arguments side by side so that each constant is read once: x = k ln 2 + r with

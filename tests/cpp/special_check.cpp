@@ -49,6 +49,15 @@ struct Worst {
             at  = x;
         }
     }
+    // in units of the least subnormal, 2^-1074
+    void add_tiny(double x, double got, long double ref) {
+        const double e = (double)(fabsl((long double)got - ref) * 0x1p1000L * 0x1p74L);
+        ++n;
+        if(!(e <= err)) {
+            err = e;
+            at  = x;
+        }
+    }
     void print(const char *name) const { std::printf("%s n=%lld err=%.4f at=%.17g\n", name, n, err, at); }
 };
 
@@ -56,7 +65,7 @@ int main(int argc, char **argv) {
     const long long N = argc > 1 ? std::atoll(argv[1]) : 1000000;
     std::mt19937_64 rng(argc > 2 ? std::strtoull(argv[2], nullptr, 10) : 1);
     std::uniform_real_distribution<double> u(0.0, 1.0);
-    Worst e_all, e_small, x_low, x_mid, x_high, pw, pn, pl;
+    Worst e_all, e_small, x_low, x_mid, x_high, pw, pn, pl, pt, nt;
     for(long long i = 0; i < N; ++i) {
         double x = -707.0 + 1416.0 * u(rng);
         e_all.add(x, exp_1(x), expl((long double)x));
@@ -80,6 +89,22 @@ int main(int argc, char **argv) {
         const int big = (int)std::pow(2.0, 31 * u(rng) - 1e-9);
         x             = 1 + (2 * u(rng) - 1) * std::fmin(0.4, 500.0 / big);
         pl.add(x, gfmath::powi(x, big), powl(x, big));
+        // powers in the subnormal range, of small and of huge x
+        const int m = 1 + (int)(i % 6);
+        x           = std::pow(10.0, (-323.0 + 15.0 * u(rng)) / m);
+        if(m > 1) {
+            p = 1;
+            for(int k = 0; k < m; ++k)
+                p *= x;
+            pt.add_tiny(x, gfmath::powi(x, m), p);
+        }
+        x = 1 / x;
+        if(m > 1) {
+            p = 1;
+            for(int k = 0; k < m; ++k)
+                p *= x;
+            nt.add_tiny(x, gfmath::powi(x, -m), 1 / p);
+        }
     }
     e_all.print("exp_range");
     e_small.print("exp_small");
@@ -89,6 +114,8 @@ int main(int argc, char **argv) {
     pw.print("powi");
     pn.print("powi_negative");
     pl.print("powi_large");
+    pt.print("powi_tiny");
+    nt.print("powi_negative_tiny");
     for(double x : {0.0, -0.0, 1.0, 710.0, -746.0, -745.0, 1e300, -1e300, (double)HUGE_VAL, -(double)HUGE_VAL, (double)NAN})
         std::printf("special exp x=%.17g y=%.17g library=%.17g\n", x, exp_1(x), std::exp(x));
     for(double x : {0.0, 1e200, (double)HUGE_VAL, (double)NAN})
