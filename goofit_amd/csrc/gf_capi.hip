@@ -1619,29 +1619,37 @@ gf_status gf_program_set(gf_ctx *ctx, const int32_t *funcs, int nfunc, const dou
         return GF_ERR_INVALID;
     if(nfunc < 1 || !funcs || np < 1 || !params || nc < 1 || !consts || no < 1 || !obs || nn < 2 || !norms)
         return fail(GF_ERR_INVALID, "empty flattened arrays");
+    // until all of it is in place there is no program
+    auto drop = [ctx]() {
+        ctx->funcs.clear();
+        ctx->dalitz.clear();
+        ctx->ins.clear();
+        ctx->sub_pc.clear();
+        ctx->fast_dalitz = ctx->lone_td = ctx->flat = false;
+        ctx->flat_prod   = 0;
+    };
+    drop();
     ctx->funcs.assign(funcs, funcs + nfunc);
     ctx->params.assign(params, params + np);
     ctx->consts.assign(consts, consts + nc);
     ctx->obs.assign(obs, obs + no);
     ctx->norms.assign(norms, norms + nn);
-    ctx->ins.clear();
-    ctx->sub_pc.clear();
     ctx->max_col = -1;
     gf_status st = scan_dalitz(ctx);
     if(st) {
-        ctx->funcs.clear();
+        drop();
         return st;
     }
     Compiler C{ctx, {}, {}, -1};
     Cur q;
     if(!C.emit(q, 0)) {
-        ctx->funcs.clear();
+        drop();
         return fail(GF_ERR_INVALID, "%s", C.err.c_str());
     }
     if(q.f != nfunc) {
         std::string e = "the tree at function 0 covers " + std::to_string(q.f) + " of " + std::to_string(nfunc)
                         + " functions";
-        ctx->funcs.clear();
+        drop();
         return fail(GF_ERR_INVALID, "%s", e.c_str());
     }
     C.push(GI_END, 0, 0, 0, 0, 0, 0, 0);
@@ -1654,7 +1662,6 @@ gf_status gf_program_set(gf_ctx *ctx, const int32_t *funcs, int nfunc, const dou
     ctx->lone_td = ctx->ins.size() >= 4 && ctx->ins[0].op == GF_LVL_OP(GK_TDDP, 0) && ctx->ins[1].op == GI_MULTI_POLY
                    && ctx->ins[2].op == GF_LVL_OP(GK_TDDP_END, 0) && ctx->ins[3].op == GI_END;
     ctx->flat      = flat_program(ctx);
-    ctx->flat_prod = 0;
     if(ctx->flat && (ctx->ins[0].op < GI_LVL || ctx->ins[0].op == GF_LVL_OP(GK_PUSH1, 0))) {
         int leaves = 0, nins = 0;
         for(; ctx->ins[nins].op != GI_END; nins++)

@@ -514,3 +514,25 @@ def test_multi_point_sums_on_the_matrix_cores_equal_single_sweeps(ctx, nres, n):
     finally:
         ctx.set_tuning(capi.TUNE_COH_MFMA, 1)
         ctx.update_params(p0)
+
+
+def test_a_program_that_is_refused_leaves_none(ctx):
+    """After a refused program every call that needs one says so: nothing of the program before it,
+    nor of the refused one (a Dalitz node whose resonances are in order and whose efficiency is no
+    function), is left."""
+    good, _ = prod3d()
+    ctx.set_program(*arrays(good)[1])
+    ctx.upload_columns([np.linspace(0.0, 1.0, 100) for _ in range(3)])
+    top, _ = dalitz(resonances=W.DALITZ_RESONANCES[:4])
+    f, p, c, o, n = arrays(top)[1]
+    f = f.copy()
+    f[-1] = 999
+    with pytest.raises(capi.GooFitError):
+        ctx.set_program(f, p, c, o, n)
+    for call in (lambda: ctx.reduce_metric("NLL"), lambda: ctx.update_params(p),
+                 lambda: ctx.dalitz_set_data_size(0, 100), lambda: ctx.dalitz_cache(0),
+                 lambda: ctx.dalitz_generate(0, 1, 1, [0.0, 3.0, 0.0, 3.0])):
+        with pytest.raises(capi.GooFitError):
+            call()
+    ctx.set_program(*arrays(good)[1])
+    assert math.isfinite(ctx.reduce_metric("NLL")[0])
