@@ -114,6 +114,24 @@ def test_waves_and_integrals(ctx, shapes, decay):
         np.testing.assert_allclose(got, ref, rtol=1e-11, atol=1e-12 * max(np.abs(ref).max(), 1e-300))
 
 
+@pytest.mark.parametrize("shapes", ["gs", "symmetrised"])
+@pytest.mark.parametrize("nb", [362, 363, 401])
+def test_integrals_over_more_cells_than_a_pass(ctx, shapes, nb):
+    """A pass of the integral's grid takes 512 workgroups x 256 cells = 131072: one pass and all but
+    28 cells of it (362^2), 697 cells of a second (363^2), and a fifth of one more, so that waves take
+    their LDS rows again, some of them for a tile with no cell inside the plot."""
+    top, res = _model(SHAPES[shapes], UNEQUAL)
+    M = O.Model(top, np.zeros((1, 3)), decay=UNEQUAL)
+    M.op.sync_params()
+    ctx.set_program(*M.op.prog.arrays())
+    ctx.set_decay(UNEQUAL)
+    funcs, eff = M.op.dalitz_layout(0)
+    grid6 = [0.0, 3.5, nb, 0.0, 3.5, nb]
+    ref = M.op.dalitz_integrals(0, grid6, eff)
+    np.testing.assert_allclose(ctx.dalitz_gram(0, grid6, eff, len(funcs)), ref, rtol=1e-11,
+                               atol=1e-12 * np.abs(ref).max())
+
+
 @pytest.mark.parametrize("shapes", ["spins", "gs", "symmetrised"])
 def test_time_dependent_waves(ctx, shapes):
     """The B waves: every lineshape at the reversed point (a pair below its threshold there).  Alone,
@@ -156,15 +174,10 @@ def _unif(key, counter):
     return (_mix64(key ^ _mix64(counter)) >> np.uint64(11)) * 2.0 ** -53
 
 
-def test_generated_events_are_the_stream(ctx):
-    """The accepted candidates of the documented stream, in its order, over one pass of 2^22
-    and into the second; a few events, a whole pass, one more than a pass; a box that cuts
-    the plot and one that misses it."""
-    decay, passes, fmax, seed = EQUAL, 2, 4000.0, 23
-    shapes = [("RBW", 0.7758, 0.15, 1, 0, True), ("NONRES", 0, 0, 0, 0, True), ("GS", 0.7758, 0.15, 1, 2, True),
-              ("SYM", 0.98, 0.06, 0, 1, True)]
+def _stream(ctx, shapes, box, seed, passes, decay=EQUAL):
+    """The documented stream's candidates over the given passes of 2^22: their points, their
+    uniform numbers, and the values (0 outside the plot), and a program that generates from it."""
     top, res = _model(shapes, decay)
-    box = [0.2, 2.6, 0.1, 3.0]
     with np.errstate(over="ignore"):
         key = _mix64(np.array([seed], np.uint64) ^ np.uint64(0x6A09E667F3BCC909))[0]
         i = np.arange(passes << 22, dtype=np.uint64)
@@ -180,7 +193,22 @@ def test_generated_events_are_the_stream(ctx):
     ctx.set_identity_column(2)
     ctx.dalitz_set_data_size(0, inside.size)
     ctx.dalitz_cache(0)
-    value = ctx.eval_metric("EVAL")
+    return m12, m13, u, inside, ctx.eval_metric("EVAL")
+
+
+SHORT = [("RBW", 0.7758, 0.15, 1, 0, True), ("NONRES", 0, 0, 0, 0, True), ("GS", 0.7758, 0.15, 1, 2, True),
+         ("SYM", 0.98, 0.06, 0, 1, True)]
+LONG = SHORT + [("SYM", 0.8 + 0.05 * k, 0.1, k % 3, k % 3, True) for k in range(7)]  # 19 terms: the plan on the device
+
+
+@pytest.mark.parametrize("shapes,fmax", [(SHORT, 4000.0), (LONG, None)], ids=["short", "long"])
+def test_generated_events_are_the_stream(ctx, shapes, fmax):
+    """The accepted candidates of the documented stream, in its order, over one pass of 2^22
+    and into the second; a few events, a whole pass, one more than a pass; a box that cuts
+    the plot and one that misses it."""
+    seed, box = 23, [0.2, 2.6, 0.1, 3.0]
+    m12, m13, u, inside, value = _stream(ctx, shapes, box, seed, 2)
+    fmax = fmax or 1.01 * value.max()
     assert value.max() < fmax
     keep = inside[u[inside] * fmax < value]
     first = int(np.sum(keep < 1 << 22))
@@ -204,6 +232,27 @@ def test_generated_events_are_the_stream(ctx):
         ctx.dalitz_generate(0, 10, seed, [2.95, 3.0, 2.95, 3.0])
     a2, b2, _, _ = ctx.dalitz_generate(0, 777, seed, box, fmax)
     assert np.array_equal(a2, m12[keep[:777]]) and np.array_equal(b2, m13[keep[:777]])
+
+
+def test_generated_events_of_queued_passes(ctx):
+    """A low acceptance, which needs six passes: one alone, then the others queued together, as
+    many as the first one's acceptance asks for.  Counts just below and just above a pass's
+    end, where one pass too many is queued, which finds the rows complete and must leave them."""
+    seed, box, passes = 31, [0.0, 3.0, 0.0, 3.0], 6
+    m12, m13, u, inside, value = _stream(ctx, SHORT, box, seed, passes)
+    fmax = 40.0 * value.max()
+    keep = inside[u[inside] * fmax < value]
+    ends = np.searchsorted(keep, np.arange(1, passes + 1) << 22)
+    assert ends[0] > 1000 and np.all(np.diff(ends) > 1000)
+    ahead = 0
+    for end in ends[1:5]:
+        for n in (end - 1, end, end + 1):
+            a, b, tried, top_value = ctx.dalitz_generate(0, int(n), seed, box, fmax)
+            assert np.array_equal(a, m12[keep[:n]]) and np.array_equal(b, m13[keep[:n]])
+            need = int(np.searchsorted(ends, n)) + 1
+            assert tried == need << 22 and top_value == fmax
+            ahead += 1 + int(np.ceil((n - ends[0]) / ends[0])) > need
+    assert ahead  # at least one of the calls queued a pass that it did not need
 
 
 def test_refresh_of_one_resonance_is_not_slow(ctx):
