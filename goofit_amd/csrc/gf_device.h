@@ -1,13 +1,14 @@
 // gf_device.h -- per-event FP64 arithmetic of the likelihood path, for gfx950.
 //
-// Each function states, in the same operation order, what the reference's
-// device function computes (file:line given per function), so that results
-// round the same way on both sides; the library is built with
-// -ffp-contract=off so no multiply-add is fused behind our back.  The log of
-// the likelihood metrics is this library's own (gf_math.h: within one unit in
-// the last place of the correctly rounded value, half the device library's
-// FP64 instructions); exp, erfc, pow, sqrt and the trigonometric functions are
-// the device library's.
+// The leaf PDFs, metrics, kinematics and truth resolution state, in the same operation order,
+// what the reference's device function computes (file:line given per function), so that
+// results round the same way on both sides; the library is built with -ffp-contract=off so no
+// multiply-add is fused behind our back.  The lineshapes (factorised over classes of
+// resonances), the three-Gaussian decay-time terms (by erfcx) and the polynomials' powers compute
+// the same functions in other forms, each with its own rounding, given where it stands, as do
+// the products in logarithms (k_reduce_prod).  The log, the whole powers, and exp and erfcx of
+// the latter two are this library's own (gf_math.h); exp and erfc of the leaf PDFs, sqrt and the
+// trigonometric functions are the device library's.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -170,11 +171,13 @@ __device__ __forceinline__ double metric(int m, double rawPdf, double evt0, doub
     }
 }
 
-// The NLL metric over a lane's events as one logarithm (gfmath::nll_add /
-// nll_total): every kernel that reduces the NLL metric accumulates it this way, in
-// its own event order per lane, in the registers of its (sum, residual) pair
-// starting from (1, 0), so kernels that assign events to lanes alike give the same
-// bits (the per-event values of evaluate_with_metric still use metric()).
+// The NLL metric over a lane's events as one logarithm (gfmath::nll_add / nll_total): the
+// kernels that reduce the NLL metric accumulate it this way, in their own event order per
+// lane, in the registers of the (sum, residual) pair starting from (1, 0), so kernels that
+// assign events to lanes alike give the same bits (the per-event values of
+// evaluate_with_metric still use metric()).  k_reduce_prod alone does not: it adds the events'
+// exponents apart and multiplies four events' other factors before each nll_add, and agrees with
+// the others to the rounding of the exponents' sum.
 __device__ __forceinline__ void nll_add(double &m, double &e, double rawPdf, double norm) {
     gfmath::nll_add(m, e, rawPdf * norm);
 }

@@ -889,9 +889,8 @@ int launch_reduce_metric(const GfProgArgs &a, const GfInline *inl, int metric, P
     hipStream_t s = (hipStream_t)stream;
     if(a.fuse_slots)  // the interpreter has no in-kernel finish
         return -1;
-    // time-dependent nodes: the kernels compiled with the TD ops (two events per lane
-    // measured 1.5 % faster than one on the 16-resonance three-Gaussian workload);
-    // programs without Dalitz nodes: the kernels compiled without them
+    // a lone time-dependent node: its own kernel; other trees that hold one: the kernels compiled
+    // with the TD ops; programs without Dalitz nodes: the kernels compiled without them
     const dim3 g(nblocks), b(GF_BLOCK);
     const GfInline none{};
     if(a.lone_td && metric < GF_METRIC_BINAVG_CODE) {

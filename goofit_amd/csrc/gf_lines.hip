@@ -22,9 +22,9 @@ __global__ __launch_bounds__(GF_MAX_TERMS) void k_line_plan(GfLinePlan *plan, co
     gfd::line_plan_term(*plan, threadIdx.x, P, d);
 }
 
-// The wave cache (ALL: every resonance).  16 shapes over 1e6 events: 58 us, 1045 vector
-// instructions per wave of 64 events (29 us of issue) beside 256 MB of stores (40 us at the
-// fill rate); 290 us with each shape evaluated by itself.
+// The wave cache (ALL: every resonance of the plan).  16 shapes over 1e6 events: 59 us on
+// average, 1045 vector instructions per wave of 64 events (29 us of issue) beside 256 MB of
+// stores (40 us at the fill rate); 290 us with each shape evaluated by itself.
 template <bool ALL, class Plan>
 __global__ __launch_bounds__(256) void k_dalitz_cache(GfProgArgs A, int slot, int64_t offset, int64_t n, uint32_t mask,
                                                       const Plan plan) {
@@ -70,7 +70,7 @@ __device__ __forceinline__ void gen_point(const GfGenBox &B, uint64_t key, uint6
 // only those are evaluated, on full waves -- the lineshapes are nine tenths of the work.
 // Out: the accepted candidates as bits, their number and the largest value (to check the
 // envelope).  Nothing is done once st->have has reached limit.  A pass of 2^22 candidates
-// with 16 shapes: 126 us; 208 us with every candidate evaluated in its own lane.
+// with 16 shapes: 130 us; 208 us with every candidate evaluated in its own lane.
 template <bool GEN_EFF, class Plan>
 __global__ __launch_bounds__(256) void k_dalitz_candidates(GfProgArgs A, const Plan plan,
                                                            int p_coup, int eff_pc, double eff_const, int id12,
@@ -311,7 +311,7 @@ __global__ __launch_bounds__(256) void k_dalitz_cells(GramSrc S, double *m12, do
 // each of three 16x16 output tiles: RR = R^T E R, II = I^T E I, RI = R^T E I, with
 // E = diag(eff * weight).  No barrier until the four waves' tiles are added at the end.
 // A point outside the Dalitz plot adds nothing, so a wave with none inside moves on (two
-// fifths of the waves over a box around the plot).  16 shapes on 1414 x 1414 cells: 115 us
+// fifths of the waves over a box around the plot).  16 shapes on 1414 x 1414 cells: 116 us
 // (40 us of vector and 24 us of matrix-core issue; the 16.5 KB of LDS per wave leave two
 // waves per SIMD, so latency shows), 450-520 us with each shape evaluated by itself over
 // every cell.  Partials: 3 tiles x 64 lanes x 4 values per block.

@@ -103,7 +103,9 @@ enum gf_tune {
     GF_TUNE_INLINE_ARGS        = 0, /* 1: parameter and normalisation values travel in the kernel
                                        arguments (no upload copy); 0: device buffers (default 1) */
     GF_TUNE_FAST_DALITZ        = 1, /* 1: dedicated kernels for a lone Amp3Body or Amp3Body_TD (default 1) */
-    GF_TUNE_BLOCKS_PER_CU      = 2, /* interpreter reduction grid cap, workgroups per CU (1..64, default 4) */
+    GF_TUNE_BLOCKS_PER_CU      = 2, /* interpreter and flat reduction grid cap, workgroups per CU (1..64,
+                                       default 4; the kernel of a lone Amp3Body_TD takes at most 3,
+                                       which is what its registers let onto a CU) */
     GF_TUNE_FAST_BLOCKS_PER_CU = 3, /* coherent-sum kernel grid cap, workgroups per CU (1..64, default 3) */
     GF_TUNE_SPIN_US            = 4, /* a reduction's caller polls the result for up to this many
                                        microseconds before blocking on the stream (0..1e6, default 2000) */
@@ -115,8 +117,9 @@ enum gf_tune {
                                        (Gaussian, Exp, ExpGaus) over at most 4 columns, runs a dedicated
                                        kernel that loads every column of a tile before evaluating it, with
                                        2 or 4 events per lane (the value; at 4 the NLL of a leaf or
-                                       product adds exponents and not values), or 1: 4 from 2^20
-                                       events on, 2 below; 0: the general interpreter (default 1) */
+                                       product adds exponents and not values, unless its norms are
+                                       outside 2^+-60), or 1: 4 from 2^20 events on, 2 below; 0: the
+                                       general interpreter (default 1) */
     GF_TUNE_FUSED_FINISH       = 7, /* 1: the coherent-sum and flat reductions add their workgroups'
                                        partials inside the sweep (the last workgroup to finish does it,
                                        in k_finish's order: the same bits) instead of in a second launch;
