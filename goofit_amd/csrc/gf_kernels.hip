@@ -423,7 +423,7 @@ __global__ __launch_bounds__(GF_BLOCK) void k_reduce_flat(GfProgArgs A, GfInline
 // issue in k_reduce_flat's form (257 operations an event for a Gaussian, an exponential and
 // an ExpGaus, which are 24 bytes: 112 us for 1e7 events); here the leaves' exponents are
 // added and not exponentiated, an ExpGaus leaves its erfcx, and a tile's exponents and factors
-// meet in one compensated sum and one product: 70 us (3.4 TB/s).  121 registers, four waves on
+// meet in one compensated sum and one product: 70 us (3.4 TB/s).  125 registers, four waves on
 // a SIMD; loading the next tile ahead takes a wave's place (155 registers: 81 us), two
 // events a lane with the next two ahead also 81.  Taken from 2^20 events on, where k_reduce_flat
 // goes to four events per lane: 16 us against 19 there, with the first tile's columns requested
